@@ -1654,13 +1654,17 @@ __global__ void __launch_bounds__(256) k_plane_sums(Grid g, int axis, int lo_pos
 }
 
 // NTFF: face currents.  Faces 0..5 = x-low, x-high, y-low, y-high, z-low,
-// z-high; per face two magnetic (M) and two electric (J) components with
-// their previous-step values (f90:7512-7641).
+// z-high; per face two magnetic (M) and two electric (J) components, and
+// their differences to the previous step, rounded as the reference's binning
+// rounds them (f90:7512-7641, 7671).  Every binning uses the differences
+// only, and a cell's two components with the same weight, so they are formed
+// once here and stored side by side: one 8-byte load per face cell and
+// weight where a binning pass had loaded four values.
 struct NtffFaces {
     float* M[6][2];
-    float* Mo[6][2];
+    float2* dM[6];
     float* J[6][2];
-    float* Jo[6][2];
+    float2* dJ[6];
     int fd0[6];            // row length of each face array
     int lo[3], hi[3];
     int pbc[3];
@@ -1704,13 +1708,11 @@ __device__ __forceinline__ void ntff_currents_body(const Grid& g, const NtffFace
         j0 = s * (Hy[o] + Hy[o + g.PX]) / 2.0f * wl;
         j1 = (-1.0f * s) * (Hx[o] + Hx[o + 1]) / 2.0f * wl;
     }
-    f.Mo[face][0][fo] = f.M[face][0][fo];
+    f.dM[face][fo] = make_float2(m0 - f.M[face][0][fo], m1 - f.M[face][1][fo]);
+    f.dJ[face][fo] = make_float2(j0 - f.J[face][0][fo], j1 - f.J[face][1][fo]);
     f.M[face][0][fo] = m0;
-    f.Mo[face][1][fo] = f.M[face][1][fo];
     f.M[face][1][fo] = m1;
-    f.Jo[face][0][fo] = f.J[face][0][fo];
     f.J[face][0][fo] = j0;
-    f.Jo[face][1][fo] = f.J[face][1][fo];
     f.J[face][1][fo] = j1;
 }
 
@@ -1760,10 +1762,10 @@ __global__ void k_ntff_bins(NtffFaces f, NtffBins bn, const int* step) {
     // slots: (Ua,Ub) receive (M slot 0, slot 1) except on z faces where the
     // reference orders y before x -- irrelevant for FP64 accumulation.
     const int ua = a == 0 ? 1 : 0, ub = a == 2 ? 1 : 2;
-    const float dM0 = f.M[face][0][fo] - f.Mo[face][0][fo];
-    const float dM1 = f.M[face][1][fo] - f.Mo[face][1][fo];
-    const float dJ0 = f.J[face][0][fo] - f.Jo[face][0][fo];
-    const float dJ1 = f.J[face][1][fo] - f.Jo[face][1][fo];
+    const float dM0 = f.dM[face][fo].x;
+    const float dM1 = f.dM[face][fo].y;
+    const float dJ0 = f.dJ[face][fo].x;
+    const float dJ1 = f.dJ[face][fo].y;
     float t = (float)n + 0.5f + tfv - 1.0f;
     int ii = (int)t;
     float w = t - (float)ii;
@@ -1899,7 +1901,8 @@ __global__ void __launch_bounds__(256) k_ntff_exact(NtffFaces f, NtffBins bn, Nt
                 const long long fo = (long long)u + (long long)f.fd0[face] * v;
                 sii[q] = ii;
                 sw[q] = t - (float)ii;
-                sd[q] = isW ? (f.J[face][slot][fo] - f.Jo[face][slot][fo]) : (f.M[face][slot][fo] - f.Mo[face][slot][fo]);
+                const float2 dd = isW ? f.dJ[face][fo] : f.dM[face][fo];
+                sd[q] = slot ? dd.y : dd.x;
             }
             __syncthreads();
             // this thread's rows in the chunk: the union of the two sides'
@@ -1973,133 +1976,350 @@ __global__ void __launch_bounds__(256) k_ntff_exact(NtffFaces f, NtffBins bn, Nt
 // ntff_lists).  A face cell's retarded time tfv does not change from step
 // to step, so the bins it can reach are fixed relative to n: offset o =
 // int(n + 0.5 + tfv - 1) - n (W: without the 0.5), up to the FP32 rounding
-// of that sum near a bin edge.  For every (angle, accumulator) the host
-// lists, per bin offset k, the cells whose o can be k or k - 1, in the
-// reference's loop order (face pairs x, y, z; rows v outer, u inner; low
-// then high face).  The bin's sum then walks its list, forming t, ii and
-// the weight with the reference's FP32 expressions and adding the
-// contribution when ii or ii + 1 is the bin, so every FP32 sum is the serial
-// reference's bit for bit.
-//  - Short lists: a wave owns 64 consecutive bins, one per lane, and reads
-//    the lists interleaved ([entry][lane]), padded to the wave's longest.
+// of that sum near a bin edge.  A cell of the faces normal to one axis adds
+// its two currents with the same weight to the accumulators of the other two
+// axes, so one list serves the three accumulators of U, and one those of W:
+// for every (angle, U or W) the builder (k_ntff_build) lists, per bin offset
+// k, the cells whose o can be k or k - 1, in the reference's loop order (face
+// pairs x, y, z; rows v outer, u inner; low then high face).  The bin's sums
+// then walk its list, forming t, ii and the weight with the reference's FP32
+// expressions and adding the contributions when ii or ii + 1 is the bin, so
+// every FP32 sum is the serial reference's bit for bit.
+//
+// Each sum is a chain of dependent additions in list order; everything else
+// (entry, weight, the difference it names) can be formed ahead.  A work-group
+// therefore splits: all waves but one form contributions into LDS, a chunk
+// ahead of that one, which only reads and adds them.
+//  - Groups: 64 consecutive bins, one per lane of the adding wave, the lists
+//    interleaved ([entry][lane]) and padded to the longest, face pair by face
+//    pair.
 //  - Long lists (a face whose cells share one retarded time, as when the
-//    direction is along an axis): a wave owns one bin; its lanes compute 64
-//    consecutive contributions at once and the sum takes them in lane
-//    order, so the serial chain waits on arithmetic, not on memory.
+//    direction is along an axis): one bin per work-group; the adding wave's
+//    two halves carry the two sums of the face pair at hand.
+// An entry that does not count (padding, or a cell whose FP32 time falls in
+// the neighbouring bin) reads element 0 of the differences, which no face
+// cell owns and which stays 0, so it adds +-0 and needs no test: a sum that
+// starts at +0 never becomes -0, and x + (+-0) = x.
+// Measured kernel time per step, in brackets that of one list per accumulator
+// walked by one wave (64 bins, or one list longer than 192), which exposed two
+// memory latencies per batch: 100^3 with 37 angles 48 us (140), 200^3 with 3
+// angles 128 us (425; its longest chain, 31,683 additions at 2 ns, takes 63),
+// eight antennas of 80^3-160^3 with 19 angles in one launch 209 us (639).
 // ---------------------------------------------------------------------------
-struct NtffList {
-    const uint2* ent;       // x: element index of the face cell (0xffffffff: padding), y: tfv bits
-    const int4* waves;      // x: accumulator row (arr * n_angles + angle), y: first bin offset,
-                            // z: first entry, w: entries per lane (>= 0) or -(entries of one long list)
-    const unsigned long long* skip;   // per wave of short lists: lanes whose bin a long-list wave owns
-    int n_waves;
-    const float* Mbase;     // M of every (face, slot) at (2 face + slot) * stride; Mo at + off_old
-    const float* Jbase;     // J, likewise; Jo at + off_old
-    unsigned off_old;
-    int face_shift;         // face of an element index: idx >> face_shift
-    float* acc;             // FP32 accumulators [6][n_angles][LL]: Ux,Uy,Uz,Wx,Wy,Wz
+struct ListDesc {           // a group of 64 bins or one long list
+    int row;                // (U: 0, W: 1) * n_angles + angle
+    int bin;                // first bin offset
+    int first;              // first entry
+    int seg[6];             // ends of the face pairs x, y, z (then the images' x, y, z) in entries of a list
+    int pad;
+    unsigned long long skip;   // group: lanes whose bin is a long list's
 };
 
-// Contribution of entry q to bin `bin` at step n (the reference's FP32
-// expressions), without branches: the data
-// loads are unconditional (a padding or non-contributing entry reads element
-// 0), so the loads of a batch of entries are all in flight together; `hit`
-// says whether the value counts.
-__device__ __forceinline__ float list_term_nb(const NtffList& L, const NtffBins& bn, uint2 q, bool isW, float nf,
-                                              int bin, bool& hit) {
-    const float tfv = __uint_as_float(q.y);
-    const float t = isW ? (nf + tfv - 1.0f) : (nf + 0.5f + tfv - 1.0f);
+struct NtffList {
+    const uint2* ent;       // x: element index of the face cell (0: padding) and sign bits, y: tfv bits
+    const ListDesc* groups;
+    const ListDesc* longs;
+    int n_groups, n_long;
+    const float2* dM;       // current differences (both components) of every face at face * stride
+    const float2* dJ;
+    float* acc;             // FP32 accumulators [6][n_angles][LL]: Ux,Uy,Uz,Wx,Wy,Wz
+    __host__ __device__ int blocks() const { return n_long + n_groups; }
+};
+
+// Waves per work-group, the adding one included: 16 while every list has a
+// compute unit of its own (a walk then takes chunks / latency, and 15 waves
+// form twice the chunk), else 8 (two work-groups per unit hide each other's
+// latencies, and more lists fit at once).  200^3 with 3 angles, 50 lists:
+// TUNE2
+constexpr int kListWavesFew = 16, kListWavesMany = 8;
+constexpr int kListUnits = 256;                        // compute units
+constexpr int kListRows = 8;                           // group rows per forming wave and chunk
+constexpr int kLongPer = 4;                            // entries per forming thread and chunk of a long list
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// Reads issued before this point stay there: the compiler otherwise moves a
+// read that serves the next turn of a loop down to that turn, and the
+// additions wait for it.
+__device__ __forceinline__ void stay_above() { __builtin_amdgcn_sched_barrier(0); }
+
+// Element and weight (times the face pair's constant K) of one entry for bin
+// `bin`, by the reference's FP32 expressions (nh = n + 0.5 for U, n for W):
+// the contributions are weight * difference.
+__device__ __forceinline__ void list_entry(uint2 q, float nh, int bin, float K, unsigned& e, float& k) {
+    const float t = nh + __uint_as_float(q.y) - 1.0f;
     const int ii = (int)t;
-    hit = q.x != 0xffffffffu && (ii == bin || ii + 1 == bin);
-    // the top bit marks an image current of sign -1 (infinite ground plane)
-    const unsigned e = hit ? (q.x & 0x7fffffffu) : 0u;
-    const float sg = (hit && (q.x >> 31)) ? -1.0f : 1.0f;
+    e = (ii == bin || ii + 1 == bin) ? (q.x & 0x3fffffffu) : 0u;
     const float wt = t - (float)ii;
-    const float* B = isW ? L.Jbase : L.Mbase;
-    const float dd = B[e] - B[e + L.off_old];
-    const int ax = (int)(e >> L.face_shift) >> 1;
-    const float K = ax == 0 ? bn.K[0] : (ax == 1 ? bn.K[1] : bn.K[2]);
-    return (ii == bin ? (1.0f - wt) * K * dd : wt * K * dd) * sg;
+    k = (ii == bin ? 1.0f - wt : wt) * K;
 }
 
-// Entries per batch: their loads are issued together, then their terms are
-// added in list order (the list walk is bound by load latency otherwise, with
-// about one wave per SIMD in flight).
-constexpr int kListBatch = 8;
-constexpr int kLongBatch = 4;   // 64-entry chunks of a long list formed together
+// The two contributions.  The top two bits of an entry mark image currents of
+// sign -1 (infinite ground plane).
+__device__ __forceinline__ float2 list_terms(uint32_t sign, float k, float2 x) {
+    return make_float2(__uint_as_float(__float_as_uint(k) ^ (sign & 0x80000000u)) * x.x,
+                       __uint_as_float(__float_as_uint(k) ^ ((sign << 1) & 0x80000000u)) * x.y);
+}
 
+template <int W>
 __device__ __forceinline__ void ntff_list_body(const NtffList& L, const NtffBins& bn, const int* step, int blk) {
-    const int w = blk * 4 + (int)(threadIdx.x >> 6);
-    if (w >= L.n_waves) return;
+    constexpr int kListChunk = (W - 1) * kListRows;          // group rows per chunk
+    constexpr int kLongChunk = (W - 1) * 64 * kLongPer;      // entries per chunk of a long list
+    __shared__ __attribute__((aligned(16))) float2 buf[2][kListChunk * 64];
+    const int n = __builtin_amdgcn_readfirstlane(*step);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = (int)(threadIdx.x & 63);
-    const int4 d = L.waves[w];
-    const int arr = d.x / bn.n_angles;
-    const bool isW = arr >= 3;
-    const int n = *step;
-    const float nf = (float)n;
-    float* A = L.acc + (long long)d.x * bn.LL;
-    if (d.w >= 0) {                                   // 64 bins, one per lane
-        const int bin = n + d.y + lane;
-        const bool own = bin >= 0 && bin < bn.LL && !((L.skip[w] >> lane) & 1ull);
-        float acc = own ? A[bin] : 0.0f;
-        const uint2* e = L.ent + d.z + lane;
-        int p = 0;
-        for (; p + kListBatch <= d.w; p += kListBatch) {
-            uint2 q[kListBatch];
+    const bool is_long = blk < L.n_long;
+    const ListDesc* __restrict__ dp = is_long ? L.longs + blk : L.groups + (blk - L.n_long);
+    ListDesc d;                                    // one per work-group: into scalar registers
+    d.row = __builtin_amdgcn_readfirstlane(dp->row);
+    d.bin = __builtin_amdgcn_readfirstlane(dp->bin);
+    d.first = __builtin_amdgcn_readfirstlane(dp->first);
 #pragma unroll
-            for (int u = 0; u < kListBatch; ++u) q[u] = e[(long long)(p + u) * 64];
-            float c[kListBatch];
-            bool hit[kListBatch];
+    for (int q = 0; q < 6; ++q) d.seg[q] = __builtin_amdgcn_readfirstlane(dp->seg[q]);
+    d.skip = dp->skip;
+    const bool isW = d.row >= bn.n_angles;
+    const float nh = isW ? (float)n : (float)n + 0.5f;
+    const float2* __restrict__ D = isW ? L.dJ : L.dM;
+    const uint2* __restrict__ ent = L.ent + d.first;
+    const long long arow = (long long)bn.n_angles * bn.LL;
+    float* A = L.acc + (isW ? 3 * arow : 0) + (long long)(isW ? d.row - bn.n_angles : d.row) * bn.LL;
+    // face pair (0, 1, 2 = x, y, z) of list position p
+    auto pair_of = [&](int p) {
+        int s = 0;
 #pragma unroll
-            for (int u = 0; u < kListBatch; ++u) c[u] = list_term_nb(L, bn, q[u], isW, nf, bin, hit[u]);
+        for (int q = 0; q < 5; ++q) s += p >= d.seg[q] ? 1 : 0;
+        return s >= 3 ? s - 3 : s;
+    };
+    auto seg = [&](int s) {      // d.seg[s] by selects: an index would put d in scratch
+        int r = d.seg[0];
 #pragma unroll
-            for (int u = 0; u < kListBatch; ++u)
-                if (hit[u]) acc = acc + c[u];
+        for (int q = 1; q < 6; ++q) r = s >= q ? d.seg[q] : r;
+        return r;
+    };
+    auto K_of = [&](int a) { return a == 0 ? bn.K[0] : (a == 1 ? bn.K[1] : bn.K[2]); };
+
+    if (is_long) {
+        const int bin = n + d.bin;
+        if (bin < 0 || bin >= bn.LL) return;       // the same for the whole work-group
+        A += bin;
+        float ax = 0.f, ay = 0.f, az = 0.f;
+        if (wave == 0) { ax = A[0]; ay = A[arow]; az = A[2 * arow]; }
+        const int t = (int)threadIdx.x - 64;       // forming thread
+        uint2 q[kLongPer];
+        auto load = [&](int s0, int s1) {
+#pragma unroll
+            for (int u = 0; u < kLongPer; ++u) {
+                const int p = s0 + u * (W - 1) * 64 + t;
+                q[u] = p < s1 ? ent[p] : make_uint2(0u, 0u);
+            }
+        };
+        // chunks never cross a face pair; (s, s0) is the chunk to form,
+        // (sp, sp0) the one before it, to add
+        int s = 0, s0 = 0, par = 0;
+        while (s < 6 && s0 >= seg(s)) ++s;
+        if (wave > 0 && s < 6) load(s0, seg(s));
+        int sp = -1, sp0 = 0;
+        for (;;) {
+            s = __builtin_amdgcn_readfirstlane(s);
+            s0 = __builtin_amdgcn_readfirstlane(s0);
+            sp = __builtin_amdgcn_readfirstlane(sp);
+            sp0 = __builtin_amdgcn_readfirstlane(sp0);
+            // the chunk after this one
+            int ns = s, ns0 = s0 + kLongChunk;
+            if (s < 6 && ns0 >= seg(s)) {
+                ns0 = seg(s);
+                while (ns < 6 && ns0 >= seg(ns)) ++ns;
+            }
+            if (wave > 0) {
+                if (s < 6) {
+                    float* bx = reinterpret_cast<float*>(buf[par]);
+                    const float K = K_of(s >= 3 ? s - 3 : s);
+                    unsigned e[kLongPer];
+                    float k[kLongPer];
+                    uint32_t sg[kLongPer];
+                    float2 x[kLongPer];
+#pragma unroll
+                    for (int u = 0; u < kLongPer; ++u) {
+                        sg[u] = q[u].x;
+                        list_entry(q[u], nh, bin, K, e[u], k[u]);
+                    }
+#pragma unroll
+                    for (int u = 0; u < kLongPer; ++u) x[u] = ldo(D, e[u] * 8u);
+                    if (ns < 6) load(ns0, seg(ns));
+#pragma unroll
+                    for (int u = 0; u < kLongPer; ++u) {
+                        const float2 c = list_terms(sg[u], k[u], x[u]);
+                        bx[u * (W - 1) * 64 + t] = c.x;
+                        bx[kLongChunk + u * (W - 1) * 64 + t] = c.y;
+                    }
+                }
+            } else if (sp >= 0) {
+                const int a = sp >= 3 ? sp - 3 : sp;
+                float acc = lane < 32 ? (a == 0 ? ay : ax) : (a == 2 ? ay : az);
+                const f32x4* b4 = reinterpret_cast<const f32x4*>(buf[par ^ 1]) + (lane < 32 ? 0 : kLongChunk / 4);
+                const int left = min(kLongChunk, seg(sp) - sp0);
+                // 32 additions at a time, the next 32 values read before them
+                const int n4 = (left + 31) / 32 * 8;   // the last additions are of padding
+                f32x4 v[8], w[8];
+                auto read = [&](f32x4* r, int p) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) r[u] = b4[min(p, kLongChunk / 4 - 8) + u];
+                    stay_above();
+                };
+                auto add = [&](const f32x4* r) {
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) {
+                        acc = acc + r[u].x;
+                        acc = acc + r[u].y;
+                        acc = acc + r[u].z;
+                        acc = acc + r[u].w;
+                    }
+                };
+                read(v, 0);
+                for (int p = 0; p < n4; p += 16) {
+                    read(w, p + 8);
+                    add(v);
+                    if (p + 8 >= n4) break;
+                    read(v, p + 16);
+                    add(w);
+                }
+                const float c0 = __shfl(acc, 0), c1 = __shfl(acc, 32);
+                if (a == 0) { ay = c0; az = c1; }
+                else if (a == 1) { ax = c0; az = c1; }
+                else { ax = c0; ay = c1; }
+            }
+            if (s >= 6) break;                     // the last chunk has been added
+            __syncthreads();
+            sp = s;
+            sp0 = s0;
+            s = ns;
+            s0 = ns0;
+            par ^= 1;
         }
-        for (; p < d.w; ++p) {
-            bool hit;
-            const float c = list_term_nb(L, bn, e[(long long)p * 64], isW, nf, bin, hit);
-            if (hit) acc = acc + c;
-        }
-        if (own) A[bin] = acc;
+        if (wave == 0 && lane == 0) { A[0] = ax; A[arow] = ay; A[2 * arow] = az; }
         return;
     }
-    // one long list: lanes form 64 contributions at a time (kLongBatch
-    // chunks together), the sum takes them in order
-    const int bin = n + d.y;
-    if (bin < 0 || bin >= bn.LL) return;
-    float acc = A[bin];
-    const int cnt = -d.w;
-    for (int p0 = 0; p0 < cnt; p0 += 64 * kLongBatch) {
-        float c[kLongBatch];
-        bool hit[kLongBatch];
+
+    const int bin = n + d.bin + lane;
+    const int M = d.seg[5], nc = (M + kListChunk - 1) / kListChunk;
+    if (wave == 0) {
+        const bool own = bin >= 0 && bin < bn.LL && !((d.skip >> lane) & 1ull);
+        A += bin;
+        float acc[3] = {0.f, 0.f, 0.f};
+        if (own) {
 #pragma unroll
-        for (int u = 0; u < kLongBatch; ++u) {
-            const int p = p0 + u * 64 + lane;
-            const uint2 q = p < cnt ? L.ent[d.z + p] : make_uint2(0xffffffffu, 0u);
-            c[u] = list_term_nb(L, bn, q, isW, nf, bin, hit[u]);
+            for (int q = 0; q < 3; ++q) acc[q] = A[q * arow];
         }
+        for (int c = 0; c < nc; ++c) {
+            __syncthreads();
+            const f32x2* b = reinterpret_cast<const f32x2*>(buf[c & 1]) + lane;
+            const int p0 = c * kListChunk, p1 = min(p0 + kListChunk, M);
+            auto add = [&](float& x, float& y, int lo, int hi) {
+                // eight rows at a time, the next eight read before their
+                // additions (rows past hi are read, not added)
+                f32x2 v[8], w[8];
+                auto read = [&](f32x2* r, int p) {
 #pragma unroll
-        for (int u = 0; u < kLongBatch; ++u) {
-            const unsigned long long m = __ballot(hit[u]);
-            if (m == ~0ull) {   // every entry counts (the usual case): no per-entry test
+                    for (int u = 0; u < 8; ++u) r[u] = b[min(p - p0 + u, kListChunk - 1) * 64];
+                    stay_above();
+                };
+                auto sum = [&](const f32x2* r) {
 #pragma unroll
-                for (int l = 0; l < 64; ++l) acc = acc + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c[u]), l));
-            } else {
-                for (int l = 0; l < 64; ++l)
-                    if ((m >> l) & 1ull) acc = acc + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c[u]), l));
+                    for (int u = 0; u < 8; ++u) {
+                        x = x + r[u].x;
+                        y = y + r[u].y;
+                    }
+                };
+                int p = lo;
+                read(v, p);
+                for (; p + 16 <= hi; p += 16) {
+                    read(w, p + 8);
+                    sum(v);
+                    read(v, p + 16);
+                    sum(w);
+                }
+                if (p + 8 <= hi) {
+                    read(w, p + 8);
+                    sum(v);
+                    p += 8;
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = w[u];
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (p + u < hi) {
+                        x = x + v[u].x;
+                        y = y + v[u].y;
+                    }
+            };
+            int from = 0;
+#pragma unroll
+            for (int s = 0; s < 6; ++s) {
+                const int lo = max(from, p0), hi = min(d.seg[s], p1);
+                from = d.seg[s];
+                if (lo >= hi) continue;
+                if (s % 3 == 0) add(acc[1], acc[2], lo, hi);
+                else if (s % 3 == 1) add(acc[0], acc[2], lo, hi);
+                else add(acc[0], acc[1], lo, hi);
             }
         }
+        if (own) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) A[q * arow] = acc[q];
+        }
+        return;
     }
-    if (lane == 0) A[bin] = acc;
+    // forming waves: entries two chunks ahead of the additions' chunk,
+    // differences one ahead
+    constexpr int R = kListRows;
+    uint2 q[R];
+    unsigned e[R];
+    float k[R];
+    uint32_t sg[R];
+    float2 x[R];
+    const int r0 = (wave - 1) * R;
+    auto load = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int p = c * kListChunk + r0 + u;
+            q[u] = p < M ? ent[(long long)p * 64 + lane] : make_uint2(0u, 0u);
+        }
+    };
+    auto form = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int p = c * kListChunk + r0 + u;
+            sg[u] = q[u].x;
+            list_entry(q[u], nh, bin, K_of(pair_of(p)), e[u], k[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u) x[u] = ldo(D, e[u] * 8u);
+    };
+    load(0);
+    form(0);
+    load(1);
+    for (int c = 0; c < nc; ++c) {
+        float2 y[R];
+#pragma unroll
+        for (int u = 0; u < R; ++u) y[u] = list_terms(sg[u], k[u], x[u]);
+#pragma unroll
+        for (int u = 0; u < R; ++u) buf[c & 1][(r0 + u) * 64 + lane] = y[u];
+        if (c + 1 < nc) {
+            form(c + 1);
+            load(c + 2);
+        }
+        __syncthreads();
+    }
 }
 
-__global__ void __launch_bounds__(256) k_ntff_list(NtffList L, NtffBins bn, const int* step) {
-    ntff_list_body(L, bn, step, (int)blockIdx.x);
+template <int W>
+__global__ void __launch_bounds__(64 * W) k_ntff_list(NtffList L, NtffBins bn, const int* step) {
+    ntff_list_body<W>(L, bn, step, (int)blockIdx.x);
 }
 
 // Per-member arguments of the batched list binning: grid (blocks of the
-// member with the most waves, members); a member's surplus blocks exit.
+// member with the most lists, members); a member's surplus blocks exit.
 // Each member's bins take the same sums in the same order as its solo run.
 struct NtffListArgs {
     NtffList L;
@@ -2107,9 +2327,120 @@ struct NtffListArgs {
     const int* step;
 };
 
-__global__ void __launch_bounds__(256) k_ntff_list_batch(const NtffListArgs* __restrict__ args) {
+__global__ void __launch_bounds__(64 * kListWavesMany) k_ntff_list_batch(const NtffListArgs* __restrict__ args) {
     const NtffListArgs& a = args[blockIdx.y];
-    ntff_list_body(a.L, a.bn, a.step, (int)blockIdx.x);
+    if ((int)blockIdx.x >= a.L.blocks()) return;
+    ntff_list_body<kListWavesMany>(a.L, a.bn, a.step, (int)blockIdx.x);
+}
+
+// Builds the contributor lists: one thread per (list row, bin offset) walks
+// the face cells in the reference's loop order and emits those that can reach
+// its bin, counting them per face pair first (FILL false), then writing them.
+// An FP64 linear model of the retarded time, widened by a margin that covers
+// the FP32 evaluation error (as in k_ntff_exact), gives the candidate cells;
+// the FP32 time of each candidate decides.  A cell whose exact offset x lies
+// within eps of a bin edge (eps: the FP32 rounding of n + x, doubled) is
+// listed for every bin it can reach.  On the device because a host loop over
+// the cells, angles and bins took longer than the run's far field itself
+// (100^3 with 37 angles: 117 ms on the host, 5.3 ms here).
+struct NtffBuild {
+    const float* ang;       // [n_angles][6]
+    const int* win;         // per angle: lowest bin offset, offsets
+    int n_angles, win_max, passes;   // passes 2: an infinite ground plane's image cells after the box's
+    int lo[3], hi[3], pbc[3], c[3], fd0[6];
+    float d[3], r_relay, c_dt;
+    int use_m[3], off_m[3]; // image position off_m - i on the plane's axis
+    float sgn_M[3], sgn_J[3];
+    unsigned stride;
+    double eps;
+    int* count;             // [2 n_angles][win_max][6]: entries per face pair, the images' after them
+    const int* dst;         // [2 n_angles][win_max][8]: first entry, step between entries, start of each face pair
+    uint2* ent;
+};
+
+template <bool FILL>
+__global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    const int row = blockIdx.y;
+    const int kk = row % P.n_angles;
+    if (q >= P.win[2 * kk + 1]) return;
+    const int Q = P.win[2 * kk] + q;
+    const bool isW = row >= P.n_angles;
+    const double shift = isW ? -1.0 : -0.5;
+    const float* an = P.ang + 6 * kk;
+    const float s1 = an[2], c1 = an[3], s2 = an[4], c2 = an[5];
+    const double g[3] = {(double)P.d[0] * s1 * c2, (double)P.d[1] * s1 * s2, (double)P.d[2] * c1};
+    const double cdt = (double)P.c_dt;
+    const size_t at = (size_t)row * P.win_max + q;
+    const int step = FILL ? P.dst[8 * at + 1] : 0;
+    for (int m = 0; m < 2; ++m)
+        for (int a = 0; a < 3; ++a) {                     // face pairs in the reference's order
+            int cnt = 0;
+            if (m < P.passes && !P.pbc[a]) {
+                uint2* out = FILL ? P.ent + P.dst[8 * at] + (long long)P.dst[8 * at + 2 + 3 * m + a] * step : nullptr;
+                const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+                // sign bits of the two components of an image current
+                uint32_t sg = 0u;
+                if (m && (isW ? P.sgn_J[b] : P.sgn_M[b]) < 0.0f) sg |= 0x80000000u;
+                if (m && (isW ? P.sgn_J[c] : P.sgn_M[c]) < 0.0f) sg |= 0x40000000u;
+                // position along an axis, the image's on the ground plane's
+                auto pos_of = [&](int ax, int i) { return m && P.use_m[ax] ? P.off_m[ax] - i : i; };
+                const double sb = m && P.use_m[b] ? -1.0 : 1.0, sc = m && P.use_m[c] ? -1.0 : 1.0;
+                const double mu = -sb * g[b] / cdt, mv = -sc * g[c] / cdt;
+                double base[2];
+                for (int side = 0; side < 2; ++side) {
+                    const double S0 = (double)(pos_of(a, side ? P.hi[a] : P.lo[a]) - P.c[a]) * g[a] +
+                                      (double)(pos_of(b, 0) - P.c[b]) * g[b] + (double)(pos_of(c, 0) - P.c[c]) * g[c];
+                    base[side] = ((double)P.r_relay - S0) / cdt + shift;
+                }
+                const double marg = P.eps + 4e-3 + 4e-7 * fabs(base[0] + mu * P.lo[b] + mv * P.lo[c]);
+                const double lo_t = (double)Q - 1.0 - marg, hi_t = (double)Q + 1.0 + marg;
+                const double inv_mu = fabs(mu) < 1e-12 ? 0.0 : 1.0 / mu;
+                for (int v = P.lo[c]; v <= P.hi[c]; ++v) {
+                    int ulo[2], uhi[2];
+                    for (int side = 0; side < 2; ++side) {
+                        const double bv = base[side] + mv * v;
+                        if (inv_mu == 0.0) {
+                            const bool in = bv >= lo_t && bv <= hi_t;
+                            ulo[side] = in ? P.lo[b] : P.hi[b] + 1;
+                            uhi[side] = in ? P.hi[b] : P.lo[b] - 1;
+                        } else {
+                            const double u1 = (lo_t - bv) * inv_mu, u2 = (hi_t - bv) * inv_mu;
+                            ulo[side] = max(P.lo[b], (int)ceil(fmin(fmax(fmin(u1, u2), -1e9), 1e9)));
+                            uhi[side] = min(P.hi[b], (int)floor(fmax(fmin(fmax(u1, u2), 1e9), -1e9)));
+                        }
+                    }
+                    const bool e0 = ulo[0] <= uhi[0], e1 = ulo[1] <= uhi[1];
+                    if (!e0 && !e1) continue;
+                    const int ua = e0 ? (e1 ? min(ulo[0], ulo[1]) : ulo[0]) : ulo[1];
+                    const int ub = e0 ? (e1 ? max(uhi[0], uhi[1]) : uhi[0]) : uhi[1];
+                    for (int u = ua; u <= ub; ++u)
+                        for (int side = 0; side < 2; ++side) {
+                            if (u < ulo[side] || u > uhi[side]) continue;
+                            const int pos = side ? P.hi[a] : P.lo[a];
+                            int i, j, k;
+                            if (a == 0) { i = pos; j = u; k = v; }
+                            else if (a == 1) { i = u; j = pos; k = v; }
+                            else { i = u; j = v; k = pos; }
+                            i = pos_of(0, i);
+                            j = pos_of(1, j);
+                            k = pos_of(2, k);
+                            const float tfv = (P.r_relay - ((float)(i - P.c[0]) * P.d[0] * s1 * c2 +
+                                                            (float)(j - P.c[1]) * P.d[1] * s1 * s2 +
+                                                            (float)(k - P.c[2]) * P.d[2] * c1)) / P.c_dt;
+                            const double x = (double)tfv + shift;
+                            if (Q < (int)floor(x - P.eps) || Q > (int)floor(x + P.eps) + 1) continue;
+                            if (FILL) {
+                                const int face = 2 * a + side;
+                                const unsigned idx = (unsigned)face * P.stride + (unsigned)(u + P.fd0[face] * v);
+                                out[(long long)cnt * step] = make_uint2(idx | sg, __float_as_uint(tfv));
+                            }
+                            ++cnt;
+                        }
+                }
+            }
+            if (!FILL) P.count[6 * at + 3 * m + a] = cnt;
+        }
 }
 
 // NTFF retarded-time binning through an LDS histogram (f90:7643-7927 with
@@ -2161,8 +2492,8 @@ __device__ __forceinline__ void ntff_hist_body(const NtffFaces& f, const NtffBin
             const float tfv = (bn.r_relay - ((float)(i - bn.ic) * bn.dx * s1 * c2 + (float)(j - bn.jc) * bn.dy * s1 * s2 +
                                              (float)(k - bn.kc) * bn.dz * c1)) / bn.c_dt;
             const long long fo = (long long)u + (long long)f.fd0[face] * v;
-            const float d = isW ? (f.J[face][slot][fo] - f.Jo[face][slot][fo])
-                                : (f.M[face][slot][fo] - f.Mo[face][slot][fo]);
+            const float2 dd = isW ? f.dJ[face][fo] : f.dM[face][fo];
+            const float d = slot ? dd.y : dd.x;
             const float t = isW ? ((float)n + tfv - 1.0f) : ((float)n + 0.5f + tfv - 1.0f);
             const int ii = (int)t;
             const float w = t - (float)ii;

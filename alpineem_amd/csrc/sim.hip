@@ -288,7 +288,7 @@ struct aem_sim {
     NtffBins nb{};
     NtffExact nx_acc{};
     int win_max = 0;
-    NtffList nl{};                 // ordered binning by contributor lists (nl.n_waves > 0)
+    NtffList nl{};                 // ordered binning by contributor lists (nl.blocks() > 0)
     bool ntff_lists = true;        // ordered binning from contributor lists (else the row scan)
     void build_ntff_lists(const std::vector<int>& win, unsigned stride);
     double *d_refl = nullptr, *d_trans = nullptr;
@@ -601,35 +601,31 @@ void aem_sim::create(const aem_sim_options* opt) {
     if (v.n_angles > 0) {
         for (int a = 0; a < 3; ++a) { nf.lo[a] = v.ff_lo[a]; nf.hi[a] = v.ff_hi[a]; nf.pbc[a] = v.pbc[a]; }
         for (int f = 0; f < 6; ++f) nf.wall[f] = v.wall[f];
-        // the face arrays of every (face, slot) in one allocation, each at a
-        // power-of-two stride, in blocks M, Mo, J, Jo (the list kernel reaches
-        // any of them from one base and an element index)
+        // the face arrays of every (face, slot) in one allocation, and the
+        // two components' differences side by side per face (the list kernel
+        // reaches any difference from one base and an element index)
         unsigned stride = 1;
         for (int f = 0; f < 6; ++f) {
             const int a = f / 2, b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
             const size_t n = (size_t)(v.ff_hi[b] + 2) * (v.ff_hi[c] + 2);
             while (stride < n) stride <<= 1;
         }
-        float* fb = zeros<float>((size_t)48 * stride);
+        float* fb = zeros<float>((size_t)24 * stride);
+        float2* dM = zeros<float2>((size_t)6 * stride);
+        float2* dJ = zeros<float2>((size_t)6 * stride);
         for (int f = 0; f < 6; ++f) {
             const int a = f / 2, b = a == 0 ? 1 : 0;
             nf.fd0[f] = v.ff_hi[b] + 2;
+            nf.dM[f] = dM + (size_t)f * stride;
+            nf.dJ[f] = dJ + (size_t)f * stride;
             for (int s = 0; s < 2; ++s) {
                 const size_t o = (size_t)(2 * f + s) * stride;
                 nf.M[f][s] = fb + o;
-                nf.Mo[f][s] = fb + (size_t)12 * stride + o;
-                nf.J[f][s] = fb + (size_t)24 * stride + o;
-                nf.Jo[f][s] = fb + (size_t)36 * stride + o;
+                nf.J[f][s] = fb + (size_t)12 * stride + o;
             }
         }
-        nl.Mbase = fb;
-        nl.Jbase = fb + (size_t)24 * stride;
-        nl.off_old = 12u * stride;
-        {
-            int sh = 1;
-            while ((1u << (sh - 1)) < stride) ++sh;
-            nl.face_shift = sh;           // (2 face + slot) * stride >> (log2 stride + 1) = face
-        }
+        nl.dM = dM;
+        nl.dJ = dJ;
         nb.ang = up<float>(v.ang, (size_t)v.n_angles * 6);
         nb.n_angles = v.n_angles;
         nb.ic = v.ic; nb.jc = v.jc; nb.kc = v.kc;
@@ -639,35 +635,29 @@ void aem_sim::create(const aem_sim_options* opt) {
         nb.LL = (long long)v.len_ff + 2;
         nb.exact = ntff_mode == AEM_NTFF_ORDERED ? 1 : 0;
         {
-            // retarded-time offsets of every face cell, per angle, bound the
-            // window of bins one step can touch
+            // retarded-time offsets of the face cells, per angle, bound the
+            // window of bins one step can touch.  The FP32 expression rounds
+            // monotonically in i, j and k, so its extremes over the faces are
+            // those of the box's corners (with a ground plane, of the image
+            // box's too)
             std::vector<int> win(2 * (size_t)v.n_angles);
             win_max = 0;
             for (int kk = 0; kk < v.n_angles; ++kk) {
                 const float* an = v.ang + 6 * kk;
                 const float s1 = an[2], c1 = an[3], s2 = an[4], c2 = an[5];
                 float tmin = 1e30f, tmax = -1e30f;
-                for (int m = 0; m < (v.mirror_type > 0 ? 2 : 1); ++m)   // with a ground plane, the image cells too
-                for (int a = 0; a < 3; ++a) {
-                    if (v.pbc[a]) continue;
-                    const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
-                    for (int side = 0; side < 2; ++side) {
-                        const int pos = side ? v.ff_hi[a] : v.ff_lo[a];
-                        for (int vv = v.ff_lo[c]; vv <= v.ff_hi[c]; ++vv)
-                            for (int uu = v.ff_lo[b]; uu <= v.ff_hi[b]; ++uu) {
-                                int i, j, k;
-                                if (a == 0) { i = pos; j = uu; k = vv; }
-                                else if (a == 1) { i = uu; j = pos; k = vv; }
-                                else { i = uu; j = vv; k = pos; }
-                                if (m) { i = mirror_pos(v, 0, i); j = mirror_pos(v, 1, j); k = mirror_pos(v, 2, k); }
-                                const float tfv = (v.r_relay - ((float)(i - v.ic) * v.dx * s1 * c2 +
-                                                                (float)(j - v.jc) * v.dy * s1 * s2 +
-                                                                (float)(k - v.kc) * v.dz * c1)) / (aem::kC * v.dt);
-                                tmin = std::min(tmin, tfv);
-                                tmax = std::max(tmax, tfv);
-                            }
+                for (int m = 0; m < (v.mirror_type > 0 ? 2 : 1); ++m)
+                    for (int q = 0; q < 8; ++q) {
+                        if (v.pbc[0] && v.pbc[1] && v.pbc[2]) break;   // no faces
+                        int i = q & 1 ? v.ff_hi[0] : v.ff_lo[0], j = q & 2 ? v.ff_hi[1] : v.ff_lo[1],
+                            k = q & 4 ? v.ff_hi[2] : v.ff_lo[2];
+                        if (m) { i = mirror_pos(v, 0, i); j = mirror_pos(v, 1, j); k = mirror_pos(v, 2, k); }
+                        const float tfv = (v.r_relay - ((float)(i - v.ic) * v.dx * s1 * c2 +
+                                                        (float)(j - v.jc) * v.dy * s1 * s2 +
+                                                        (float)(k - v.kc) * v.dz * c1)) / (aem::kC * v.dt);
+                        tmin = std::min(tmin, tfv);
+                        tmax = std::max(tmax, tfv);
                     }
-                }
                 const int lo = (int)std::floor(tmin) - 3, hi = (int)std::floor(tmax) + 3;
                 win[2 * kk] = lo;
                 win[2 * kk + 1] = std::max(hi - lo + 1, 0);
@@ -697,11 +687,11 @@ void aem_sim::create(const aem_sim_options* opt) {
         if (ntff_mode == AEM_NTFF_HISTOGRAM && win_max > kHistMax) ntff_mode = AEM_NTFF_ATOMIC;
         // an infinite ground plane's image currents are binned by the
         // contributor lists only
-        if (v.mirror_type > 0 && (ntff_mode != AEM_NTFF_ORDERED || nl.n_waves == 0))
+        if (v.mirror_type > 0 && (ntff_mode != AEM_NTFF_ORDERED || nl.blocks() == 0))
             throw aem::Error(AEM_ERR_UNSUPPORTED,
                              "the far field of an infinite ground plane deck needs the ordered binning from "
                              "contributor lists (AEM_NTFF_ORDERED, ntff_row_scan 0)");
-        if (ntff_mode == AEM_NTFF_ORDERED && nl.n_waves == 0)   // the row-scan kernel's limit
+        if (ntff_mode == AEM_NTFF_ORDERED && nl.blocks() == 0)   // the row-scan kernel's limit
             for (int a = 0; a < 2; ++a)
                 if (!v.pbc[a] && 2 * (v.ff_hi[a] - v.ff_lo[a] + 1) > kExactCells)
                     throw aem::Error(AEM_ERR_UNSUPPORTED,
@@ -1353,8 +1343,10 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
         const dim3 gf(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6);
         k_ntff_currents<<<gf, bb, 0, s>>>(g, nf, Ex, Ey, Ez, Hx, Hy, Hz);
         if (ntff_mode == AEM_NTFF_ORDERED) {
-            if (nl.n_waves > 0)
-                k_ntff_list<<<cdiv(nl.n_waves, 4), 256, 0, s>>>(nl, nb, d_step);
+            if (nl.blocks() > kListUnits)
+                k_ntff_list<kListWavesMany><<<nl.blocks(), 64 * kListWavesMany, 0, s>>>(nl, nb, d_step);
+            else if (nl.blocks() > 0)
+                k_ntff_list<kListWavesFew><<<nl.blocks(), 64 * kListWavesFew, 0, s>>>(nl, nb, d_step);
             else if (win_max > 0)
                 k_ntff_exact<<<dim3(cdiv(win_max, 256), 6, v.n_angles), 256, 0, s>>>(nf, nb, nx_acc, d_step);
         } else if (ntff_mode == AEM_NTFF_HISTOGRAM) {
@@ -1416,108 +1408,140 @@ void aem_sim::export_step() {
             throw aem::Error(AEM_ERR_IO, "writing a full-field record failed");
 }
 
-// Contributor lists of the ordered far-field binning (k_ntff_list).  For
-// angle kk and accumulator arr (Ux,Uy,Uz,Wx,Wy,Wz) a face cell with retarded
-// time tfv lands at t = n + tfv - 0.5 (W: n + tfv - 1), evaluated in FP32 as
-// the reference does.  Its bin offset ii - n is floor of the exact value,
-// except that the FP32 rounding of t (at most one ulp of the largest t, here
-// doubled) can move it across a bin edge; the cell goes into the list of
-// every offset it can reach with either weight.  Lists keep the reference's
-// loop order (the order k_ntff_exact walks).  Larger than kListBytes in
-// total, the builder gives up and the row-scan kernel stays in use.  A
-// wave's descriptor: row, first bin offset, first entry, and the entries per
-// lane (64 short lists) or minus the length of one long list.
+// Contributor lists of the ordered far-field binning (k_ntff_list), built by
+// k_ntff_build: counted, laid out here, then written.  For an angle and U or W
+// a face cell with retarded time tfv lands at t = n + tfv - 0.5 (W: n + tfv -
+// 1), evaluated in FP32 as the reference does.  Its bin offset ii - n is floor
+// of the exact value, except that the FP32 rounding of t (at most one ulp of
+// the largest t, here doubled) can move it across a bin edge; the cell goes
+// into the list of every offset it can reach with either weight.  Larger than
+// kListBytes in total, the builder gives up and the row-scan kernel stays in
+// use.
 void aem_sim::build_ntff_lists(const std::vector<int>& win, unsigned stride) {
     constexpr size_t kListBytes = size_t(4) << 30;
-    constexpr size_t kLong = 192;     // entries from which a bin's list gets a wave of its own
     const aem_plan_view& v = plan->v;
-    const float cdt = aem::kC * v.dt;
+    // (a difference's byte offset has 32 bits, an element index 30)
+    if (win_max == 0 || 2 * v.n_angles > 65535 || 6ull * stride * sizeof(float2) >= (1ull << 32)) return;
     const double tmax = (double)v.time_steps + (double)v.len_ff + 8.0;
-    const double eps = 2.0 * std::ldexp(1.0, (int)std::ceil(std::log2(tmax)) - 23);
-    std::vector<int4> waves;
-    std::vector<unsigned long long> skip;
-    std::vector<uint2> ent;
-    std::vector<std::vector<uint2>> lists;
-    for (int kk = 0; kk < v.n_angles; ++kk) {
-        const float* an = v.ang + 6 * kk;
-        const float s1 = an[2], c1 = an[3], s2 = an[4], c2 = an[5];
+    NtffBuild B{};
+    B.ang = nb.ang;
+    B.win = nx_acc.win;
+    B.n_angles = v.n_angles;
+    B.win_max = win_max;
+    // with a ground plane the image currents follow every face of the box, in
+    // the same order, their entries flagged where the components' image signs
+    // are -1 (f90:7928-8240)
+    B.passes = v.mirror_type > 0 && v.pbc[0] + v.pbc[1] + v.pbc[2] < 2 ? 2 : 1;
+    const int pc[3] = {v.ic, v.jc, v.kc};
+    const float dd[3] = {v.dx, v.dy, v.dz};
+    for (int a = 0; a < 3; ++a) {
+        B.lo[a] = v.ff_lo[a]; B.hi[a] = v.ff_hi[a]; B.pbc[a] = v.pbc[a]; B.c[a] = pc[a]; B.d[a] = dd[a];
+        B.use_m[a] = v.use_m[a] != 0.0f ? 1 : 0;
+        B.off_m[a] = (int)v.off_m[a];
+        B.sgn_M[a] = v.sgn_M[a];
+        B.sgn_J[a] = v.sgn_J[a];
+    }
+    for (int f = 0; f < 6; ++f) B.fd0[f] = nf.fd0[f];
+    B.r_relay = v.r_relay;
+    B.c_dt = aem::kC * v.dt;
+    B.stride = stride;
+    B.eps = 2.0 * std::ldexp(1.0, (int)std::ceil(std::log2(tmax)) - 23);
+    const int rows = 2 * v.n_angles;
+    const size_t nlist = (size_t)rows * win_max;
+    std::vector<int> cnt(6 * nlist, 0), dst(8 * nlist, 0);
+    std::vector<void*> tmp;           // freed below
+    struct Free {
+        std::vector<void*>& p;
+        ~Free() { for (void* q : p) (void)hipFree(q); }
+    } freer{tmp};
+    B.count = dalloc<int>(cnt.size(), tmp);
+    int* d_dst = dalloc<int>(dst.size(), tmp);
+    B.dst = d_dst;
+    const dim3 grid(cdiv(win_max, 256), rows);
+    k_ntff_build<false><<<grid, 256, 0, st>>>(B);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(cnt.data(), B.count, cnt.size() * sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    // layout: a group per 64 bins of a row; a list much longer than its
+    // group's others (a face in one bin) on its own, since the group's padding
+    // and its chain of additions are those of its longest list
+    constexpr int kLong = 1024;
+    std::vector<ListDesc> groups, longs;
+    size_t n_ent = 0;
+    for (int row = 0; row < rows; ++row) {
+        const int kk = row % v.n_angles;
         const int wlo = win[2 * kk], wlen = win[2 * kk + 1];
-        for (int arr = 0; arr < 6; ++arr) {
-            const int comp = arr % 3;
-            const double shift = arr >= 3 ? -1.0 : -0.5;
-            lists.assign((size_t)wlen, {});
-            // with a ground plane the image currents follow every face of the
-            // box, in the same order, their entries flagged with the top bit
-            // where the component's image sign is -1 (f90:7928-8240)
-            const int passes = v.mirror_type > 0 && v.pbc[0] + v.pbc[1] + v.pbc[2] < 2 ? 2 : 1;
-            for (int m = 0; m < passes; ++m)
-            for (int a = 0; a < 3; ++a) {                     // face pairs in the reference's order
-                if (a == comp || v.pbc[a]) continue;
-                const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
-                const int slot = comp == b ? 0 : 1;
-                for (int vv = v.ff_lo[c]; vv <= v.ff_hi[c]; ++vv)
-                    for (int uu = v.ff_lo[b]; uu <= v.ff_hi[b]; ++uu)
-                        for (int side = 0; side < 2; ++side) {
-                            const int pos = side ? v.ff_hi[a] : v.ff_lo[a];
-                            int i, j, k;
-                            if (a == 0) { i = pos; j = uu; k = vv; }
-                            else if (a == 1) { i = uu; j = pos; k = vv; }
-                            else { i = uu; j = vv; k = pos; }
-                            if (m) { i = mirror_pos(v, 0, i); j = mirror_pos(v, 1, j); k = mirror_pos(v, 2, k); }
-                            const float tfv = (v.r_relay - ((float)(i - v.ic) * v.dx * s1 * c2 +
-                                                            (float)(j - v.jc) * v.dy * s1 * s2 +
-                                                            (float)(k - v.kc) * v.dz * c1)) / cdt;
-                            const double x = (double)tfv + shift;
-                            const int olo = (int)std::floor(x - eps), ohi = (int)std::floor(x + eps);
-                            const int face = 2 * a + side;
-                            const float sg = m ? (arr >= 3 ? v.sgn_J[comp] : v.sgn_M[comp]) : 1.0f;
-                            const unsigned idx = ((unsigned)(2 * face + slot) * stride +
-                                                  (unsigned)(uu + nf.fd0[face] * vv)) |
-                                                 (sg < 0.0f ? 0x80000000u : 0u);
-                            uint32_t tb;
-                            std::memcpy(&tb, &tfv, 4);
-                            for (int o = olo; o <= ohi + 1; ++o) {
-                                const int q = o - wlo;
-                                if (q < 0 || q >= wlen)
-                                    throw aem::Error(AEM_ERR_STATE, "far-field list outside its bin window");
-                                lists[q].push_back(make_uint2(idx, tb));
-                            }
-                        }
+        for (int w0 = 0; w0 < wlen; w0 += 64) {
+            const int nbin = std::min(64, wlen - w0);
+            const size_t o0 = (size_t)row * win_max + w0;
+            int total[64], sorted[64];
+            for (int l = 0; l < nbin; ++l) {
+                total[l] = 0;
+                for (int s = 0; s < 6; ++s) total[l] += cnt[6 * (o0 + l) + s];
+                sorted[l] = total[l];
             }
-            const int row = arr * v.n_angles + kk;
-            for (int w0 = 0; w0 < wlen; w0 += 64) {
-                // lists longer than kLong get a wave of their own; the rest
-                // of the 64 bins share one wave, one lane per bin
-                size_t m = 0;
-                unsigned long long sk = 0;
-                for (int l = 0; l < 64 && w0 + l < wlen; ++l) {
-                    const std::vector<uint2>& li = lists[w0 + l];
-                    if (li.size() > kLong) {
-                        sk |= 1ull << l;
-                        waves.push_back(make_int4(row, wlo + w0 + l, (int)ent.size(), -(int)li.size()));
-                        skip.push_back(0ull);
-                        ent.insert(ent.end(), li.begin(), li.end());
-                    } else {
-                        m = std::max(m, li.size());
-                    }
+            std::nth_element(sorted, sorted + nbin / 2, sorted + nbin);
+            const int lim = std::max(kLong, 4 * sorted[nbin / 2]);
+            ListDesc gd{};
+            gd.row = row;
+            gd.bin = wlo + w0;
+            int m[6] = {0, 0, 0, 0, 0, 0};
+            for (int l = 0; l < nbin; ++l) {
+                const int* c = &cnt[6 * (o0 + l)];
+                if (total[l] <= lim) {
+                    for (int s = 0; s < 6; ++s) m[s] = std::max(m[s], c[s]);
+                    continue;
                 }
-                if ((ent.size() + 64 * m) * sizeof(uint2) > kListBytes) return;
-                waves.push_back(make_int4(row, wlo + w0, (int)ent.size(), (int)m));
-                skip.push_back(sk);
-                for (size_t p = 0; p < m; ++p)
-                    for (int l = 0; l < 64; ++l) {
-                        const int q = w0 + l;
-                        const bool in = q < wlen && !((sk >> l) & 1ull) && p < lists[q].size();
-                        ent.push_back(in ? lists[q][p] : make_uint2(0xffffffffu, 0u));
-                    }
+                gd.skip |= 1ull << l;
+                ListDesc ld{};
+                ld.row = row;
+                ld.bin = wlo + w0 + l;
+                ld.first = (int)n_ent;
+                int* t = &dst[8 * (o0 + l)];
+                t[0] = (int)n_ent;
+                t[1] = 1;
+                for (int s = 0, p = 0; s < 6; ++s) {
+                    t[2 + s] = p;
+                    p += c[s];
+                    ld.seg[s] = p;
+                }
+                longs.push_back(ld);
+                n_ent += (size_t)total[l];
+                if (n_ent * sizeof(uint2) > kListBytes) return;
             }
+            gd.first = (int)n_ent;
+            for (int s = 0, p = 0; s < 6; ++s) {
+                p += m[s];
+                gd.seg[s] = p;
+            }
+            if (gd.seg[5] == 0) continue;
+            n_ent += (size_t)64 * gd.seg[5];
+            if (n_ent * sizeof(uint2) > kListBytes) return;
+            for (int l = 0; l < nbin; ++l)
+                if (!((gd.skip >> l) & 1ull)) {
+                    int* t = &dst[8 * (o0 + l)];
+                    t[0] = gd.first + l;
+                    t[1] = 64;
+                    for (int s = 0; s < 6; ++s) t[2 + s] = s ? gd.seg[s - 1] : 0;
+                }
+            groups.push_back(gd);
         }
     }
-    if (ent.size() > 0x7fffffffull) return;
-    nl.ent = up<uint2>(ent.data(), ent.size());
-    nl.waves = up<int4>(waves.data(), waves.size());
-    nl.skip = up<unsigned long long>(skip.data(), skip.size());
-    nl.n_waves = (int)waves.size();
+    if (groups.empty() && longs.empty()) return;
+    // the longest chains of additions start first
+    auto longer = [](const ListDesc& x, const ListDesc& y) { return x.seg[5] > y.seg[5]; };
+    std::stable_sort(longs.begin(), longs.end(), longer);
+    std::stable_sort(groups.begin(), groups.end(), longer);
+    HIPCHK(hipMemcpyAsync(d_dst, dst.data(), dst.size() * sizeof(int), hipMemcpyHostToDevice, st));
+    B.ent = zeros<uint2>(n_ent);      // padding entries are zero
+    nl.ent = B.ent;
+    k_ntff_build<true><<<grid, 256, 0, st>>>(B);
+    HIPCHK(hipGetLastError());
+    nl.groups = up<ListDesc>(groups.data(), groups.size());
+    nl.longs = up<ListDesc>(longs.data(), longs.size());
+    HIPCHK(hipStreamSynchronize(st));
+    nl.n_groups = (int)groups.size();
+    nl.n_long = (int)longs.size();
 }
 
 void aem_sim::enqueue_watch(hipStream_t s) {
@@ -2174,7 +2198,7 @@ struct aem_batch {
             if (v.n_ports > 0) pa.push_back(s->pa);
             if (v.n_angles > 0 && s->ntff_mode != AEM_NTFF_OFF) {
                 const bool hist = s->ntff_mode == AEM_NTFF_HISTOGRAM;
-                const bool list = s->ntff_mode == AEM_NTFF_ORDERED && s->nl.n_waves > 0;
+                const bool list = s->ntff_mode == AEM_NTFF_ORDERED && s->nl.blocks() > 0;
                 if (hist || list) {
                     na.push_back(s->na);
                     ntff_mu = std::max(ntff_mu, s->ntff_mu);
@@ -2185,7 +2209,7 @@ struct aem_batch {
                     max_angles = std::max(max_angles, v.n_angles);
                 } else if (list) {
                     nla.push_back(NtffListArgs{s->nl, s->nb, s->d_step});
-                    max_list_blocks = std::max(max_list_blocks, (int)cdiv(s->nl.n_waves, 4));
+                    max_list_blocks = std::max(max_list_blocks, s->nl.blocks());
                 } else {
                     ntff_alone.push_back(q);
                 }
@@ -2252,7 +2276,7 @@ struct aem_batch {
         if (n_ntff)
             k_ntff_currents_batch<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * n_ntff), bb, 0, s>>>(d_nargs);
         if (n_hist) k_ntff_hist_batch<<<dim3(max_angles, 6, n_hist), 256, 0, s>>>(d_hist_args);
-        if (n_list) k_ntff_list_batch<<<dim3(max_list_blocks, n_list), 256, 0, s>>>(d_list_args);
+        if (n_list) k_ntff_list_batch<<<dim3(max_list_blocks, n_list), 64 * kListWavesMany, 0, s>>>(d_list_args);
         for (int q : ntff_alone) m[q]->enqueue_parts(nullptr, s, kPartNtff);
         each(kPartObjective | kPartOutPost);
         k_step_inc_batch<<<cdiv(n, 256), 256, 0, s>>>(d_steps, n);
