@@ -2029,8 +2029,8 @@ struct NtffList {
 // Waves per work-group, the adding one included: 16 while every list has a
 // compute unit of its own (a walk then takes chunks / latency, and 15 waves
 // form twice the chunk), else 8 (two work-groups per unit hide each other's
-// latencies, and more lists fit at once).  200^3 with 3 angles, 50 lists:
-// TUNE2
+// latencies, and more lists fit at once).  100^3 with 37 angles: 48 us with
+// 16, 69 us with 8.
 constexpr int kListWavesFew = 16, kListWavesMany = 8;
 constexpr int kListUnits = 256;                        // compute units
 constexpr int kListRows = 8;                           // group rows per forming wave and chunk
