@@ -47,12 +47,22 @@ T* dalloc(size_t n, std::vector<void*>& owned) {
 
 inline unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) / b); }
 
+// A captured graph holds kGraphSteps steps (an even number, so that a graph
+// of single-pass steps ends on the buffer set it began with).  Launching a
+// graph costs about 9 us on the device's queue whatever it holds and 1.8 us
+// per kernel node (measured with empty kernels), so at one step per graph the
+// launch was a quarter of a 40^3 step: 60 -> 52 us.  Steps left over, and runs
+// shorter than kGraphMin steps, which would not earn the capture back, are
+// enqueued one by one (2.5 us per kernel, hidden by the kernels).
+constexpr int kGraphSteps = 16;
+constexpr int kGraphMin = 48;
+
 // Replay loops keep at most two chunks of steps queued ahead of the device:
-// after every kRunAheadChunk launches the host records an event and waits
+// after every kRunAheadChunk steps the host records an event and waits
 // for the one it recorded a chunk earlier.  The device always has a chunk
 // of work queued, while the runtime is never handed a whole run at once (a
 // 3000-step, 64-member population is about 10^6 kernel dispatches).
-constexpr int kRunAheadChunk = 32;
+constexpr int kRunAheadChunk = 64;
 
 // A run checks every field for NaN or infinity after every kWatchSteps
 // steps and after its last step (one read of the six fields: about 0.3 ms
@@ -69,10 +79,10 @@ struct RunAhead {
             if (e) (void)hipEventDestroy(e);
         ev[0] = ev[1] = nullptr;
     }
-    // after launch q (0-based) of a replay loop on stream s
-    void pace(hipStream_t s, int64_t q) {
-        if ((q + 1) % kRunAheadChunk) return;
-        const int slot = (int)(((q + 1) / kRunAheadChunk) & 1);
+    // after the steps up to q (from q0) of a replay loop on stream s
+    void pace(hipStream_t s, int64_t q0, int64_t q) {
+        if (q0 / kRunAheadChunk == q / kRunAheadChunk) return;
+        const int slot = (int)((q / kRunAheadChunk) & 1);
         HIPCHK(hipEventRecord(ev[slot], s));
         live[slot] = true;
         if (live[slot ^ 1]) HIPCHK(hipEventSynchronize(ev[slot ^ 1]));
@@ -380,10 +390,7 @@ struct aem_sim {
                             double* dga, double* dgb);
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
-    hipGraph_t graph2 = nullptr;   // single-pass steps: the step from the other buffer set
-    hipGraphExec_t gexec2 = nullptr;
-    int gpar = 0;                  // buffer set the first graph starts from
-    bool gsp = false;              // the graphs are single-pass steps
+    int gpar = 0;                  // buffer set the graph starts from and ends on
     void drop_graphs();
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     RunAhead ra;                   // bounds the steps a replay loop queues
@@ -1125,10 +1132,8 @@ void aem_sim::enqueue_kmax_step(hipStream_t s) {
 void aem_sim::drop_graphs() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
     if (graph) (void)hipGraphDestroy(graph);
-    if (gexec2) (void)hipGraphExecDestroy(gexec2);
-    if (graph2) (void)hipGraphDestroy(graph2);
-    gexec = gexec2 = nullptr;
-    graph = graph2 = nullptr;
+    gexec = nullptr;
+    graph = nullptr;
 }
 
 // Enqueue the selected parts of one step on stream s, in the reference's
@@ -1634,34 +1639,29 @@ aem_status aem_run(aem_sim* s, int64_t n_steps, int32_t use_graph) {
     }
     return aem::guard([&]() {
         if (n_steps == 0) return;
-        if (use_graph && !s->gexec) {
-            // a single-pass step alternates buffer sets: one graph per set
-            const int p0 = s->par;
+        // checkpoints and the full-field export act between steps
+        const bool whole = use_graph && s->ck_K == 0 && !s->full_on && (s->gexec || n_steps >= kGraphMin);
+        if (whole && !s->gexec) {
+            s->gpar = s->par;
             HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-            s->enqueue_step();
+            for (int q = 0; q < kGraphSteps; ++q) s->enqueue_step();
             HIPCHK(hipStreamEndCapture(s->st, &s->graph));
             HIPCHK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
-            s->gsp = s->par != p0;
-            s->gpar = p0;
-            if (s->gsp) {
-                HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-                s->enqueue_step();
-                HIPCHK(hipStreamEndCapture(s->st, &s->graph2));
-                HIPCHK(hipGraphInstantiate(&s->gexec2, s->graph2, nullptr, nullptr, 0));
-            }
         }
         HIPCHK(hipEventRecord(s->ev0, s->st));
-        for (int64_t q = 0; q < n_steps; ++q) {
+        for (int64_t q = 0, q0 = 0; q < n_steps; q0 = q) {
             if (s->ck_K > 0 && (s->steps_done + q) % s->ck_K == 0) s->snapshot((int)((s->steps_done + q) / s->ck_K));
-            if (use_graph) {
-                HIPCHK(hipGraphLaunch(s->par == s->gpar ? s->gexec : s->gexec2, s->st));
-                if (s->gsp) s->flip();
+            // (a single step first where the fields are in the other buffer set)
+            if (whole && s->par == s->gpar && n_steps - q >= kGraphSteps) {
+                HIPCHK(hipGraphLaunch(s->gexec, s->st));
+                q += kGraphSteps;
             } else {
                 s->enqueue_step();
+                ++q;
             }
             if (s->full_on) s->export_step();
-            if ((q + 1) % kWatchSteps == 0 && q + 1 < n_steps) s->enqueue_watch(s->st);
-            s->ra.pace(s->st, q);
+            if (q0 / kWatchSteps != q / kWatchSteps && q < n_steps) s->enqueue_watch(s->st);
+            s->ra.pace(s->st, q0, q);
         }
         s->enqueue_watch(s->st);
         HIPCHK(hipGetLastError());
@@ -2358,19 +2358,25 @@ aem_status aem_batch_run(aem_batch* b, int64_t n_steps, int32_t use_graph) {
     return aem::guard([&]() {
         if (n_steps == 0) return;
         for (aem_sim* s : b->m) HIPCHK(hipStreamSynchronize(s->st));
-        if (use_graph && !b->gexec) {
+        const bool whole = use_graph && (b->gexec || n_steps >= kGraphMin);
+        if (whole && !b->gexec) {
             HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-            b->enqueue(b->st);
+            for (int q = 0; q < kGraphSteps; ++q) b->enqueue(b->st);
             HIPCHK(hipStreamEndCapture(b->st, &b->graph));
             HIPCHK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
         }
         HIPCHK(hipEventRecord(b->ev0, b->st));
-        for (int64_t q = 0; q < n_steps; ++q) {
-            if (use_graph) HIPCHK(hipGraphLaunch(b->gexec, b->st));
-            else b->enqueue(b->st);
-            if ((q + 1) % kWatchSteps == 0 && q + 1 < n_steps)
+        for (int64_t q = 0, q0 = 0; q < n_steps; q0 = q) {
+            if (whole && n_steps - q >= kGraphSteps) {
+                HIPCHK(hipGraphLaunch(b->gexec, b->st));
+                q += kGraphSteps;
+            } else {
+                b->enqueue(b->st);
+                ++q;
+            }
+            if (q0 / kWatchSteps != q / kWatchSteps && q < n_steps)
                 for (aem_sim* s : b->m) s->enqueue_watch(b->st);
-            b->ra.pace(b->st, q);
+            b->ra.pace(b->st, q0, q);
         }
         for (aem_sim* s : b->m) s->enqueue_watch(b->st);
         HIPCHK(hipGetLastError());
@@ -2966,8 +2972,8 @@ aem_status aem_set_design_eps(aem_sim* s, const float* eps, int64_t n) {
 namespace {
 
 // The full backward sweep of J = |F|^2: dJ/dGa and dJ/dGb of every record
-// edge ([3][edges] each).  Clears the adjoint state, captures one backward
-// step as a graph and replays it time_steps times.
+// edge ([3][edges] each).  Clears the adjoint state and runs the backward step
+// time_steps times, in graphs of kGraphSteps.
 // The adjoint source weights a step's terms by 2 Re(conj(F) w), the
 // derivative of J = |F|^2.  A general real J(F) with dJ/dF = dJ/dRe F +
 // i dJ/dIm F (dj, two doubles) has dJ = Re(conj(dj) dF): the same source
@@ -3019,13 +3025,35 @@ void backward_sweep(aem_sim* s, std::vector<double>& ha, std::vector<double>& hb
     }
     const int T = v.time_steps;
     HIPCHK(hipMemcpyAsync(s->d_bstep, &T, sizeof(int), hipMemcpyHostToDevice, s->st));
+    auto one = [&]() {
+        if (v.idx_bytes == 1) s->enqueue_backward_t<uint8_t>(s->st, ff_src, F[0], F[1], d_wV, d_wI, dga, dgb);
+        else s->enqueue_backward_t<uint16_t>(s->st, ff_src, F[0], F[1], d_wV, d_wI, dga, dgb);
+    };
     hipGraph_t gr = nullptr;
     hipGraphExec_t gx = nullptr;
-    HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-    if (v.idx_bytes == 1) s->enqueue_backward_t<uint8_t>(s->st, ff_src, F[0], F[1], d_wV, d_wI, dga, dgb);
-    else s->enqueue_backward_t<uint16_t>(s->st, ff_src, F[0], F[1], d_wV, d_wI, dga, dgb);
-    HIPCHK(hipStreamEndCapture(s->st, &gr));
-    HIPCHK(hipGraphInstantiate(&gx, gr, nullptr, nullptr, 0));
+    const int per = s->ck_K > 0 ? std::min(s->ck_K, T) : T;   // steps transposed without a break
+    if (per >= kGraphMin) {
+        HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
+        for (int q = 0; q < kGraphSteps; ++q) one();
+        HIPCHK(hipStreamEndCapture(s->st, &gr));
+        HIPCHK(hipGraphInstantiate(&gx, gr, nullptr, nullptr, 0));
+    }
+    int64_t launched = 0;
+    auto back = [&](int n) {
+        while (n > 0) {
+            const int64_t l0 = launched;
+            if (gx && n >= kGraphSteps) {
+                HIPCHK(hipGraphLaunch(gx, s->st));
+                n -= kGraphSteps;
+                launched += kGraphSteps;
+            } else {
+                one();
+                --n;
+                ++launched;
+            }
+            s->ra.pace(s->st, l0, launched);
+        }
+    };
     HIPCHK(hipEventRecord(s->ev0, s->st));
     if (s->ck_K > 0) {
         // intervals from the last: the record of the last one is still in
@@ -3036,36 +3064,30 @@ void backward_sweep(aem_sim* s, std::vector<double>& ha, std::vector<double>& hb
         const int K = s->ck_K, S = (T + K - 1) / K;
         constexpr unsigned kRecompute = kPartAll & ~(kPartOutPre | kPartNtff | kPartOutPost | kPartObjective);
         s->snapshot(S);
-        int launched = 0;
         for (int seg = S - 1; seg >= 0; --seg) {
             const int n0 = seg * K, n1 = std::min(T, n0 + K);
             if (seg < S - 1 || !s->ck_last_ok) {
                 s->restore(seg);
                 for (int n = n0; n < n1; ++n) {
                     s->enqueue_parts(nullptr, s->st, kRecompute);
-                    s->ra.pace(s->st, launched++);
+                    s->ra.pace(s->st, launched, launched + 1);
+                    ++launched;
                 }
             }
-            for (int n = n1; n > n0; --n) {
-                HIPCHK(hipGraphLaunch(gx, s->st));
-                s->ra.pace(s->st, launched++);
-            }
+            back(n1 - n0);
         }
         s->restore(S);
         s->ck_last_ok = false;   // the record now holds the first interval
     } else {
-        for (int n = 0; n < T; ++n) {
-            HIPCHK(hipGraphLaunch(gx, s->st));
-            s->ra.pace(s->st, n);
-        }
+        back(T);
     }
     HIPCHK(hipEventRecord(s->ev1, s->st));
     HIPCHK(hipEventSynchronize(s->ev1));
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, s->ev0, s->ev1));
     s->last_ms = ms / (float)T;
-    (void)hipGraphExecDestroy(gx);
-    (void)hipGraphDestroy(gr);
+    if (gx) (void)hipGraphExecDestroy(gx);
+    if (gr) (void)hipGraphDestroy(gr);
     ha.resize(3 * ne);
     hb.resize(3 * ne);
     HIPCHK(hipMemcpy(ha.data(), dga, ha.size() * sizeof(double), hipMemcpyDeviceToHost));

@@ -169,7 +169,8 @@ void aem_destroy(aem_sim* sim);
 
 /* Advance n_steps leapfrog steps (H phase, E phase, per-step outputs).  The
  * total may not exceed the deck's time_steps (output arrays are sized by
- * it).  use_graph!=0 replays a captured HIP graph of one step.
+ * it).  use_graph!=0 replays a captured HIP graph of several steps where the
+ * run is long enough for one.
  * A deck that exports the full field ("yes" after the video flag,
  * f90:913) appends one record per step to <name>_full_{E,H}{x,y,z}.bin in
  * the current directory (f90:4348-4355, 6992-7003).
@@ -386,8 +387,8 @@ typedef struct aem_batch aem_batch;
 aem_status aem_batch_create(aem_sim* const* sims, int32_t n, aem_batch** out);
 
 /* Advance every member n_steps (each member's total may not exceed its
- * time_steps).  use_graph!=0 replays a captured HIP graph of one batched
- * step.  Returns after the device has finished. */
+ * time_steps).  use_graph!=0 replays a captured HIP graph of several
+ * batched steps where the run is long enough for one.  Returns after the device has finished. */
 aem_status aem_batch_run(aem_batch* batch, int64_t n_steps, int32_t use_graph);
 
 /* Device time per batched step of the last aem_batch_run (ms). */
