@@ -1716,8 +1716,11 @@ __device__ __forceinline__ void ntff_currents_body(const Grid& g, const NtffFace
     f.J[face][1][fo] = j1;
 }
 
+// (fstep: the step these currents belong to, read by the binning, which may
+// run beside the following step)
 __global__ void k_ntff_currents(Grid g, NtffFaces f, const float* Ex, const float* Ey, const float* Ez,
-                                const float* Hx, const float* Hy, const float* Hz) {
+                                const float* Hx, const float* Hy, const float* Hz, const int* step, int* fstep) {
+    if (blockIdx.x + blockIdx.y + blockIdx.z + threadIdx.x + threadIdx.y == 0) *fstep = *step;
     ntff_currents_body(g, f, blockIdx.z, Ex, Ey, Ez, Hx, Hy, Hz);
 }
 
@@ -2542,11 +2545,13 @@ struct NtffArgs {
     const int* win;
     const float *Ex, *Ey, *Ez, *Hx, *Hy, *Hz;
     const int* step;
+    int* fstep;
 };
 
 // grid (x-blocks, y-blocks, 6 * members); blocks beyond a member's faces exit
 __global__ void k_ntff_currents_batch(const NtffArgs* __restrict__ args) {
     const NtffArgs& a = args[blockIdx.z / 6];
+    if (blockIdx.x + blockIdx.y + blockIdx.z % 6 + threadIdx.x + threadIdx.y == 0) *a.fstep = *a.step;
     ntff_currents_body(a.g, a.f, blockIdx.z % 6, a.Ex, a.Ey, a.Ez, a.Hx, a.Hy, a.Hz);
 }
 
@@ -2554,7 +2559,7 @@ __global__ void k_ntff_currents_batch(const NtffArgs* __restrict__ args) {
 __global__ void __launch_bounds__(256) k_ntff_hist_batch(const NtffArgs* __restrict__ args) {
     const NtffArgs& a = args[blockIdx.z];
     if ((int)blockIdx.x >= a.bn.n_angles) return;
-    ntff_hist_body(a.f, a.bn, a.win, blockIdx.x, blockIdx.y, a.step);
+    ntff_hist_body(a.f, a.bn, a.win, blockIdx.x, blockIdx.y, a.fstep);
 }
 
 __global__ void k_step_inc_batch(int* const* __restrict__ steps, int n) {

@@ -50,10 +50,12 @@ inline unsigned cdiv(long long a, long long b) { return (unsigned)((a + b - 1) /
 // A captured graph holds kGraphSteps steps (an even number, so that a graph
 // of single-pass steps ends on the buffer set it began with).  Launching a
 // graph costs about 9 us on the device's queue whatever it holds and 1.8 us
-// per kernel node (measured with empty kernels), so at one step per graph the
-// launch was a quarter of a 40^3 step: 60 -> 52 us.  Steps left over, and runs
-// shorter than kGraphMin steps, which would not earn the capture back, are
-// enqueued one by one (2.5 us per kernel, hidden by the kernels).
+// per kernel node (measured with empty kernels; part of it hides behind the
+// step before).  Per step, one step per graph against sixteen: 40^3 dipole
+// 60.0 -> 56.5 us, 75 x 30 x 30 periodic slab 47.6 -> 43.4 us.  Steps left
+// over, and runs shorter than kGraphMin steps, which would not earn the
+// capture back, are enqueued one by one (2.5 us per kernel, hidden by the
+// kernels).
 constexpr int kGraphSteps = 16;
 constexpr int kGraphMin = 48;
 
@@ -63,6 +65,58 @@ constexpr int kGraphMin = 48;
 // of work queued, while the runtime is never handed a whole run at once (a
 // 3000-step, 64-member population is about 10^6 kernel dispatches).
 constexpr int kRunAheadChunk = 64;
+
+// Beside the next step: the far-field binning of a step reads that step's
+// current differences only, so inside a captured graph it runs on a second
+// stream while the following step's fields are updated.  The differences have
+// two slots, one per parity of the step within the graph: the currents of step
+// q wait for the binning of step q - 2, and the graph ends with the last
+// binning.  The two waits between the streams cost about 11 us per step, so a
+// far-field box of less than kBesideCells face cells keeps one stream.
+// Measured per step, beside / in turn: 40^3 with 3 angles (2,000 face cells)
+// 64 / 57 us, 64^3 (10,600) 70 / 68, 76^3 (17,500) 80 / 82, 100^3 91 / 100;
+// LDS histogram at 64^3 70 / 74, 76^3 82 / 100, 100^3 107 / 151; 200^3 with 3
+// angles 295 / 387.
+constexpr long long kBesideCells = 16000;
+struct Beside {
+    hipStream_t s2 = nullptr;
+    hipEvent_t cur[2] = {nullptr, nullptr}, bin[2] = {nullptr, nullptr};
+    int q = 0;                     // step within the graph
+    bool used = false;             // a binning has been enqueued
+    Beside() {
+        HIPCHK(hipStreamCreateWithFlags(&s2, hipStreamNonBlocking));
+        for (int k = 0; k < 2; ++k) {
+            HIPCHK(hipEventCreateWithFlags(&cur[k], hipEventDisableTiming));
+            HIPCHK(hipEventCreateWithFlags(&bin[k], hipEventDisableTiming));
+        }
+    }
+    ~Beside() {
+        for (int k = 0; k < 2; ++k) {
+            if (cur[k]) (void)hipEventDestroy(cur[k]);
+            if (bin[k]) (void)hipEventDestroy(bin[k]);
+        }
+        if (s2) (void)hipStreamDestroy(s2);
+    }
+    Beside(const Beside&) = delete;
+    int slot() const { return q & 1; }
+    void before_currents(hipStream_t s) {
+        if (q >= 2) HIPCHK(hipStreamWaitEvent(s, bin[slot()], 0));
+    }
+    // the stream of the binning, after the currents enqueued on s
+    hipStream_t after_currents(hipStream_t s) {
+        HIPCHK(hipEventRecord(cur[slot()], s));
+        HIPCHK(hipStreamWaitEvent(s2, cur[slot()], 0));
+        return s2;
+    }
+    void after_binning() {
+        HIPCHK(hipEventRecord(bin[slot()], s2));
+        used = true;
+    }
+    void next() { ++q; }
+    void join(hipStream_t s) {
+        if (used) HIPCHK(hipStreamWaitEvent(s, bin[(q - 1) & 1], 0));
+    }
+};
 
 // A run checks every field for NaN or infinity after every kWatchSteps
 // steps and after its last step (one read of the six fields: about 0.3 ms
@@ -294,11 +348,30 @@ struct aem_sim {
     DrudeBox db[3]{};
     PortDev* d_ports = nullptr;
     float *d_V = nullptr, *d_I = nullptr, *d_Vout = nullptr, *d_Iout = nullptr;
-    NtffFaces nf{};
+    NtffFaces nfs[2]{};            // face currents; their differences by slot (Beside)
     NtffBins nb{};
+    int* d_ffstep = nullptr;       // step of the differences in each slot
+    Beside* beside = nullptr;      // set while a graph is captured
     NtffExact nx_acc{};
     int win_max = 0;
     NtffList nl{};                 // ordered binning by contributor lists (nl.blocks() > 0)
+    // face cells of the far-field box whose binning a step enqueues
+    long long face_cells() const {
+        const aem_plan_view& v = plan->v;
+        if (v.n_angles <= 0 || ntff_mode == AEM_NTFF_OFF) return 0;
+        long long n = 0;
+        for (int a = 0; a < 3; ++a) {
+            const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+            if (!v.pbc[a]) n += 2LL * (v.ff_hi[b] - v.ff_lo[b] + 1) * (v.ff_hi[c] - v.ff_lo[c] + 1);
+        }
+        return n;
+    }
+    NtffList list_of(int slot) const {
+        NtffList l = nl;
+        l.dM = nfs[slot].dM[0];    // face 0 begins the slot's allocation
+        l.dJ = nfs[slot].dJ[0];
+        return l;
+    }
     bool ntff_lists = true;        // ordered binning from contributor lists (else the row scan)
     void build_ntff_lists(const std::vector<int>& win, unsigned stride);
     double *d_refl = nullptr, *d_trans = nullptr;
@@ -606,6 +679,7 @@ void aem_sim::create(const aem_sim_options* opt) {
 
     // NTFF
     if (v.n_angles > 0) {
+        NtffFaces& nf = nfs[0];
         for (int a = 0; a < 3; ++a) { nf.lo[a] = v.ff_lo[a]; nf.hi[a] = v.ff_hi[a]; nf.pbc[a] = v.pbc[a]; }
         for (int f = 0; f < 6; ++f) nf.wall[f] = v.wall[f];
         // the face arrays of every (face, slot) in one allocation, and the
@@ -618,21 +692,24 @@ void aem_sim::create(const aem_sim_options* opt) {
             while (stride < n) stride <<= 1;
         }
         float* fb = zeros<float>((size_t)24 * stride);
-        float2* dM = zeros<float2>((size_t)6 * stride);
-        float2* dJ = zeros<float2>((size_t)6 * stride);
+        d_ffstep = zeros<int>(2);
         for (int f = 0; f < 6; ++f) {
             const int a = f / 2, b = a == 0 ? 1 : 0;
             nf.fd0[f] = v.ff_hi[b] + 2;
-            nf.dM[f] = dM + (size_t)f * stride;
-            nf.dJ[f] = dJ + (size_t)f * stride;
             for (int s = 0; s < 2; ++s) {
                 const size_t o = (size_t)(2 * f + s) * stride;
                 nf.M[f][s] = fb + o;
                 nf.J[f][s] = fb + (size_t)12 * stride + o;
             }
         }
-        nl.dM = dM;
-        nl.dJ = dJ;
+        nfs[1] = nf;
+        for (int q = 0; q < 2; ++q) {
+            float2* d = zeros<float2>((size_t)12 * stride);
+            for (int f = 0; f < 6; ++f) {
+                nfs[q].dM[f] = d + (size_t)f * stride;
+                nfs[q].dJ[f] = d + (size_t)(6 + f) * stride;
+            }
+        }
         nb.ang = up<float>(v.ang, (size_t)v.n_angles * 6);
         nb.n_angles = v.n_angles;
         nb.ic = v.ic; nb.jc = v.jc; nb.kc = v.kc;
@@ -841,7 +918,7 @@ void aem_sim::bind() {
                cpE, v.dx, v.dy, v.dz};
     pa = PortArgs{g, d_ports, v.n_ports, v.M, v.time_steps, d_V, d_I, d_Vout, d_Iout, F[0], F[1], F[2], F[3], F[4],
                   F[5], v.dx, v.dy, v.dz, pu, d_step};
-    na = NtffArgs{g, nf, nb, nx_acc.win, F[0], F[1], F[2], F[3], F[4], F[5], d_step};
+    na = NtffArgs{g, nfs[0], nb, nx_acc.win, F[0], F[1], F[2], F[3], F[4], F[5], d_step, d_ffstep};
     spa = SpiceArgs{g, d_spice, v.n_spice, v.n_spice_extra, v.time_steps, d_spI, d_spV, d_spIout, d_spVout,
                     F[0], F[1], F[2], F[3], F[4], F[5], v.dx, v.dy, v.dz, d_step};
 }
@@ -1346,19 +1423,25 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     }
     if ((parts & kPartNtff) && v.n_angles > 0 && ntff_mode != AEM_NTFF_OFF) {
         const dim3 gf(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6);
-        k_ntff_currents<<<gf, bb, 0, s>>>(g, nf, Ex, Ey, Ez, Hx, Hy, Hz);
+        const int slot = beside ? beside->slot() : 0;
+        const NtffFaces& nf = nfs[slot];
+        int* fstep = d_ffstep + slot;
+        if (beside) beside->before_currents(s);
+        k_ntff_currents<<<gf, bb, 0, s>>>(g, nf, Ex, Ey, Ez, Hx, Hy, Hz, d_step, fstep);
+        const hipStream_t sb = beside ? beside->after_currents(s) : s;
         if (ntff_mode == AEM_NTFF_ORDERED) {
             if (nl.blocks() > kListUnits)
-                k_ntff_list<kListWavesMany><<<nl.blocks(), 64 * kListWavesMany, 0, s>>>(nl, nb, d_step);
+                k_ntff_list<kListWavesMany><<<nl.blocks(), 64 * kListWavesMany, 0, sb>>>(list_of(slot), nb, fstep);
             else if (nl.blocks() > 0)
-                k_ntff_list<kListWavesFew><<<nl.blocks(), 64 * kListWavesFew, 0, s>>>(nl, nb, d_step);
+                k_ntff_list<kListWavesFew><<<nl.blocks(), 64 * kListWavesFew, 0, sb>>>(list_of(slot), nb, fstep);
             else if (win_max > 0)
-                k_ntff_exact<<<dim3(cdiv(win_max, 256), 6, v.n_angles), 256, 0, s>>>(nf, nb, nx_acc, d_step);
+                k_ntff_exact<<<dim3(cdiv(win_max, 256), 6, v.n_angles), 256, 0, sb>>>(nf, nb, nx_acc, fstep);
         } else if (ntff_mode == AEM_NTFF_HISTOGRAM) {
-            k_ntff_hist<<<dim3(v.n_angles, 6), 256, 0, s>>>(nf, nb, nx_acc.win, d_step);
+            k_ntff_hist<<<dim3(v.n_angles, 6), 256, 0, sb>>>(nf, nb, nx_acc.win, fstep);
         } else {
-            k_ntff_bins<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * v.n_angles), bb, 0, s>>>(nf, nb, d_step);
+            k_ntff_bins<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * v.n_angles), bb, 0, sb>>>(nf, nb, fstep);
         }
+        if (beside) beside->after_binning();
     }
     if ((parts & kPartObjective) && obj_on) {
         const dim3 go(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6);
@@ -1446,7 +1529,7 @@ void aem_sim::build_ntff_lists(const std::vector<int>& win, unsigned stride) {
         B.sgn_M[a] = v.sgn_M[a];
         B.sgn_J[a] = v.sgn_J[a];
     }
-    for (int f = 0; f < 6; ++f) B.fd0[f] = nf.fd0[f];
+    for (int f = 0; f < 6; ++f) B.fd0[f] = nfs[0].fd0[f];
     B.r_relay = v.r_relay;
     B.c_dt = aem::kC * v.dt;
     B.stride = stride;
@@ -1643,8 +1726,18 @@ aem_status aem_run(aem_sim* s, int64_t n_steps, int32_t use_graph) {
         const bool whole = use_graph && s->ck_K == 0 && !s->full_on && (s->gexec || n_steps >= kGraphMin);
         if (whole && !s->gexec) {
             s->gpar = s->par;
+            Beside bs;
             HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-            for (int q = 0; q < kGraphSteps; ++q) s->enqueue_step();
+            if (s->face_cells() >= kBesideCells) s->beside = &bs;
+            struct Clear {
+                aem_sim* s;
+                ~Clear() { s->beside = nullptr; }
+            } clear{s};
+            for (int q = 0; q < kGraphSteps; ++q) {
+                s->enqueue_step();
+                bs.next();
+            }
+            bs.join(s->st);
             HIPCHK(hipStreamEndCapture(s->st, &s->graph));
             HIPCHK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
         }
@@ -2111,9 +2204,11 @@ struct aem_batch {
     int n_port = 0;
     // batched far fields: the face currents of every member binned by the
     // LDS histogram or by contributor lists, then each binning's own launch
-    NtffArgs* d_nargs = nullptr;
-    NtffArgs* d_hist_args = nullptr;
-    NtffListArgs* d_list_args = nullptr;
+    // (by slot of the differences, see Beside)
+    NtffArgs* d_nargs[2] = {nullptr, nullptr};
+    NtffArgs* d_hist_args[2] = {nullptr, nullptr};
+    NtffListArgs* d_list_args[2] = {nullptr, nullptr};
+    Beside* beside = nullptr;      // set while a graph is captured
     int n_ntff = 0, n_hist = 0, n_list = 0, max_angles = 0, max_list_blocks = 0, ntff_mu = 0, ntff_mv = 0;
     std::vector<int> ntff_alone;   // members whose far field bins outside the batch
     int** d_steps = nullptr;
@@ -2189,8 +2284,8 @@ struct aem_batch {
         build(false, hg);
         build(true, eg);
         std::vector<PortArgs> pa;
-        std::vector<NtffArgs> na, nh;
-        std::vector<NtffListArgs> nla;
+        std::vector<NtffArgs> na[2], nh[2];
+        std::vector<NtffListArgs> nla[2];
         std::vector<int*> steps(n);
         for (int q = 0; q < n; ++q) {
             aem_sim* s = m[q];
@@ -2199,16 +2294,21 @@ struct aem_batch {
             if (v.n_angles > 0 && s->ntff_mode != AEM_NTFF_OFF) {
                 const bool hist = s->ntff_mode == AEM_NTFF_HISTOGRAM;
                 const bool list = s->ntff_mode == AEM_NTFF_ORDERED && s->nl.blocks() > 0;
+                NtffArgs xa[2] = {s->na, s->na};
+                for (int k = 0; k < 2; ++k) {
+                    xa[k].f = s->nfs[k];
+                    xa[k].fstep = s->d_ffstep + k;
+                }
                 if (hist || list) {
-                    na.push_back(s->na);
+                    for (int k = 0; k < 2; ++k) na[k].push_back(xa[k]);
                     ntff_mu = std::max(ntff_mu, s->ntff_mu);
                     ntff_mv = std::max(ntff_mv, s->ntff_mv);
                 }
                 if (hist) {
-                    nh.push_back(s->na);
+                    for (int k = 0; k < 2; ++k) nh[k].push_back(xa[k]);
                     max_angles = std::max(max_angles, v.n_angles);
                 } else if (list) {
-                    nla.push_back(NtffListArgs{s->nl, s->nb, s->d_step});
+                    for (int k = 0; k < 2; ++k) nla[k].push_back(NtffListArgs{s->list_of(k), s->nb, s->d_ffstep + k});
                     max_list_blocks = std::max(max_list_blocks, s->nl.blocks());
                 } else {
                     ntff_alone.push_back(q);
@@ -2217,13 +2317,15 @@ struct aem_batch {
             steps[q] = s->d_step;
         }
         n_port = (int)pa.size();
-        n_ntff = (int)na.size();
-        n_hist = (int)nh.size();
-        n_list = (int)nla.size();
+        n_ntff = (int)na[0].size();
+        n_hist = (int)nh[0].size();
+        n_list = (int)nla[0].size();
         d_pargs = upload(pa);
-        d_nargs = upload(na);
-        d_hist_args = upload(nh);
-        d_list_args = upload(nla);
+        for (int k = 0; k < 2; ++k) {
+            d_nargs[k] = upload(na[k]);
+            d_hist_args[k] = upload(nh[k]);
+            d_list_args[k] = upload(nla[k]);
+        }
         d_steps = upload(steps);
         HIPCHK(hipStreamSynchronize(st));
     }
@@ -2273,10 +2375,16 @@ struct aem_batch {
         if (n_port) k_ports_e_batch<<<n_port, 256, 0, s>>>(d_pargs);
         each(kPartEPost | kPartEOld);
         each(kPartOutPre);
-        if (n_ntff)
-            k_ntff_currents_batch<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * n_ntff), bb, 0, s>>>(d_nargs);
-        if (n_hist) k_ntff_hist_batch<<<dim3(max_angles, 6, n_hist), 256, 0, s>>>(d_hist_args);
-        if (n_list) k_ntff_list_batch<<<dim3(max_list_blocks, n_list), 64 * kListWavesMany, 0, s>>>(d_list_args);
+        if (n_ntff) {
+            const int slot = beside ? beside->slot() : 0;
+            if (beside) beside->before_currents(s);
+            k_ntff_currents_batch<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * n_ntff), bb, 0, s>>>(d_nargs[slot]);
+            const hipStream_t sb = beside ? beside->after_currents(s) : s;
+            if (n_hist) k_ntff_hist_batch<<<dim3(max_angles, 6, n_hist), 256, 0, sb>>>(d_hist_args[slot]);
+            if (n_list)
+                k_ntff_list_batch<<<dim3(max_list_blocks, n_list), 64 * kListWavesMany, 0, sb>>>(d_list_args[slot]);
+            if (beside) beside->after_binning();
+        }
         for (int q : ntff_alone) m[q]->enqueue_parts(nullptr, s, kPartNtff);
         each(kPartObjective | kPartOutPost);
         k_step_inc_batch<<<cdiv(n, 256), 256, 0, s>>>(d_steps, n);
@@ -2360,8 +2468,20 @@ aem_status aem_batch_run(aem_batch* b, int64_t n_steps, int32_t use_graph) {
         for (aem_sim* s : b->m) HIPCHK(hipStreamSynchronize(s->st));
         const bool whole = use_graph && (b->gexec || n_steps >= kGraphMin);
         if (whole && !b->gexec) {
+            Beside bs;
+            long long cells = 0;
+            for (aem_sim* s : b->m) cells += s->face_cells();
+            if (cells >= kBesideCells) b->beside = &bs;
+            struct Clear {
+                aem_batch* b;
+                ~Clear() { b->beside = nullptr; }
+            } clear{b};
             HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-            for (int q = 0; q < kGraphSteps; ++q) b->enqueue(b->st);
+            for (int q = 0; q < kGraphSteps; ++q) {
+                b->enqueue(b->st);
+                bs.next();
+            }
+            bs.join(b->st);
             HIPCHK(hipStreamEndCapture(b->st, &b->graph));
             HIPCHK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
         }
