@@ -238,8 +238,20 @@ struct Launch {
     }
 };
 
-constexpr int kPlanes = 4;     // default z planes marched by one thread of a bulk kernel
-constexpr int kSpPlanes = 10;  // target z planes marched by one column of the single-pass kernel
+// z planes marched by one thread of a bulk kernel, and by one column of the
+// single-pass kernel, on grids that fill the chip.  Each plane of a march
+// waits for its own loads, so where the launch has fewer work-groups than
+// kBulkGroups (kSlabGroups, kSpGroups) the march is cut: more and shorter
+// columns, although each reads its first plane's neighbour again.  Measured
+// (us per launch, planes 1 / 2 / 4 / 8): bulk H core at 40^3 7.1 / 8.6 / 11.3 /
+// 14.0, 80^3 9.9 / 10.7 / 13.4, 150^3 31.5 / 30.3 / 33.5, 200^3 80 / 74 / 74,
+// 256^3 142 / 133 / 130; y/z slabs (H and E) at 120^3 37 / 36 / 43, 150^3 49 /
+// 48 / 51, 200^3 84 / 81 / 84; single pass at 40^3 11.5 / 13.6 / 18.9 / 29.2,
+// 120^3 35 / 35 / 30 / 40, 160^3 78 / 63 / 58 / 56, 200^3 167 / 133 / 117 /
+// 108, 256^3 296 / 230 / 201 / 196.
+constexpr int kPlanes = 4;
+constexpr int kSpPlanes = 8;
+constexpr long long kBulkGroups = 4096, kSlabGroups = 2048, kSpGroups = 800;
 
 // Parts of a step, in the order the reference applies them.
 enum : unsigned {
@@ -288,20 +300,37 @@ Launch make_launch(const std::vector<Box>& boxes, int c) {
 // y and z outside the y/z slabs) with the x-slab test, then one launch over
 // the y-slab and z-slab boxes.  H slab layers are 1..n-1 and N+1-n..N-1, E
 // layers 2..n and N+1-n..N-1, so one split serves both phases.
-std::vector<Launch> bulk_launches(const aem_plan_view& v, bool fuse, int planes) {
+// `alone`: the launch has the chip to itself, so its z chunks follow the
+// groups rule above; `planes` is otherwise taken as it is.
+std::vector<Launch> bulk_launches(const aem_plan_view& v, bool fuse, int planes, bool alone) {
     const int N[3] = {v.NX, v.NY, v.NZ};
+    auto columns = [](const Box& b) { return (long long)cdiv(b.ni, kTX) * cdiv(b.nj, kTY); };
     auto box = [&](int a0, int a1, int b0, int b1, int c0, int c1) {
-        // z chunks of equal length, at most `planes` each; a box of at most
-        // 16 planes (a z slab) in chunks of 2, for more work-groups (at 400^3
-        // 2.5% faster slab launches than 4 planes; 1 plane the same, the whole
-        // box 23% slower)
-        const int nk = c1 - c0 + 1;
-        const int kc = nk > 0 ? (nk <= 16 ? 2 : (int)cdiv(nk, cdiv(nk, planes))) : planes;
-        return Box{a0, b0, c0, a1 - a0 + 1, b1 - b0 + 1, nk, kc};
+        return Box{a0, b0, c0, a1 - a0 + 1, b1 - b0 + 1, c1 - c0 + 1, planes};
+    };
+    // z chunks of equal length, at most `planes` each; a slab launch's box of at
+    // most 16 planes (a z slab) in chunks of 2, for more work-groups (at 400^3
+    // 2.5% faster slab launches than 4 planes; 1 plane the same, the whole
+    // box 23% slower)
+    auto launch = [&](std::vector<Box> boxes, int c, long long groups) {
+        int most = planes;
+        auto length = [&](const Box& b) {
+            if (b.nk <= 0) return most;
+            return b.nk <= 16 ? std::min(most, 2) : (int)cdiv(b.nk, cdiv(b.nk, most));
+        };
+        auto total = [&]() {
+            long long n = 0;
+            for (const Box& b : boxes) n += columns(b) * cdiv(b.nk, length(b));
+            return n;
+        };
+        if (alone)
+            while (most > 1 && total() < groups) most /= 2;
+        for (Box& b : boxes) b.kc = length(b);
+        return make_launch(boxes, c);
     };
     std::vector<Launch> out;
     if (!fuse) {
-        out.push_back(make_launch({box(1, N[0] - 1, 1, N[1] - 1, 1, N[2] - 1)}, 0));
+        out.push_back(launch({box(1, N[0] - 1, 1, N[1] - 1, 1, N[2] - 1)}, 0, kBulkGroups));
         return out;
     }
     int lo[3], hi[3];
@@ -317,12 +346,12 @@ std::vector<Launch> bulk_launches(const aem_plan_view& v, bool fuse, int planes)
         if (hi[a] < N[a] - 1) edge[a].push_back({hi[a] + 1, N[a] - 1});
     }
     const bool cy = lo[1] <= hi[1], cz = lo[2] <= hi[2];
-    if (cy && cz) out.push_back(make_launch({box(1, N[0] - 1, lo[1], hi[1], lo[2], hi[2])}, kCx));
+    if (cy && cz) out.push_back(launch({box(1, N[0] - 1, lo[1], hi[1], lo[2], hi[2])}, kCx, kBulkGroups));
     std::vector<Box> slabs;
     if (cz)
         for (auto e : edge[1]) slabs.push_back(box(1, N[0] - 1, e.first, e.second, lo[2], hi[2]));
     for (auto e : edge[2]) slabs.push_back(box(1, N[0] - 1, 1, N[1] - 1, e.first, e.second));
-    if (!slabs.empty()) out.push_back(make_launch(slabs, kCx | kCy | kCz));
+    if (!slabs.empty()) out.push_back(launch(slabs, kCx | kCy | kCz, kSlabGroups));
     return out;
 }
 
@@ -838,7 +867,7 @@ void aem_sim::create(const aem_sim_options* opt) {
     rdv[0] = make_rdiv(v.dx, v.kmax != 0);
     rdv[1] = make_rdiv(v.dy, v.kmax != 0);
     rdv[2] = make_rdiv(v.dz, v.kmax != 0);
-    bulk = bulk_launches(v, fuse_cpml, planes);
+    bulk = bulk_launches(v, fuse_cpml, planes, !planes_set);
     for (int f = 0; f < 6; ++f)
         for (int q = 0; q < 2; ++q) {
             cpH.pso[f][q] = cpH.psi[f][q];
@@ -854,17 +883,9 @@ void aem_sim::create(const aem_sim_options* opt) {
             bulk[0].bs.n == 1;
     if (sp_ok) {
         sp_box = bulk[0].bs.b[0];
-        sp_box.kc = planes_set ? planes : kSpPlanes;
-        // small grids: fewer planes per column until the launch has enough
-        // work-groups to fill the chip (16 per CU); then chunks of equal
-        // length (at 400^3: 380 planes in 38 chunks of 10, 2% faster than 16)
-        auto groups = [&](int kc) {
-            return (long long)cdiv(sp_box.ni, 64) * cdiv(sp_box.nj, kSY * kSpRows) * cdiv(sp_box.nk, kc);
-        };
-        if (!planes_set) {
-            while (sp_box.kc > 2 && groups(sp_box.kc) < 4096) sp_box.kc /= 2;
-            sp_box.kc = (int)cdiv(sp_box.nk, cdiv(sp_box.nk, sp_box.kc));
-        }
+        const long long groups = (long long)cdiv(sp_box.ni, 64) * cdiv(sp_box.nj, kSY * kSpRows) * sp_box.nk;
+        sp_box.kc = planes_set ? planes : (int)std::max(1LL, std::min<long long>(kSpPlanes, groups / kSpGroups));
+        if (!planes_set) sp_box.kc = (int)cdiv(sp_box.nk, cdiv(sp_box.nk, sp_box.kc));   // chunks of equal length
         // one launch with the x-slab test compiled in: measured at 400^3,
         // separate launches for the slab-free x tiles (no slab test, fewer
         // registers) and the two x-slab tiles of each row took 5-12% longer,
@@ -2261,7 +2282,8 @@ struct aem_batch {
                     long long blocks = 0;
                     for (int q = 0; q < n; ++q) {
                         if (e_phase && m[q]->plan->v.idx_bytes != ib) continue;
-                        for (const Launch& L : m[q]->bulk) {
+                        // the members share the chip: chunks as for a large grid
+                        for (const Launch& L : bulk_launches(m[q]->plan->v, m[q]->fuse_cpml, m[q]->planes, false)) {
                             if (L.c != c) continue;
                             for (int k = 0; k < L.bs.n; ++k) {
                                 const Box& b = L.bs.b[k];
