@@ -114,19 +114,19 @@ struct Box {
     int kc;           // planes marched by one thread
 };
 
-constexpr int kMaxBoxes = 4;
+constexpr int kMaxBoxes = 5;
 
 struct BoxSet {
     Box b[kMaxBoxes];
     int first[kMaxBoxes + 1];   // first work-group of each box; first[n] = total
     int n;
+    int core;                   // 1: box 0 is the core box (x-slab test only), the others slab boxes
 };
 
-// Box of this work-group and its (x, y, z-chunk) block coordinates.  The
+// Box of work-group g and its (x, y, z-chunk) block coordinates.  The
 // selection uses constant indices only, so the box table stays in kernel
 // arguments (scalar registers) instead of a private copy.
-__device__ __forceinline__ Box box_of(const BoxSet& s, int& bx, int& by, int& bz) {
-    const int g = (int)blockIdx.x;
+__device__ __forceinline__ Box box_of(const BoxSet& s, int g, int& bx, int& by, int& bz) {
     Box b = s.b[0];
     int f = s.first[0];
 #pragma unroll
@@ -429,9 +429,23 @@ __device__ __forceinline__ BatchEntry entry_of(const BatchEntry* __restrict__ e,
 template <int C, bool PP = false, typename OffT = uint64_t>
 __global__ void __launch_bounds__(kTX * kTY) k_h_bulk(HArgs a, BoxSet bs) {
     int bx, by, bz;
-    const Box b = box_of(bs, bx, by, bz);
+    const Box b = box_of(bs, (int)blockIdx.x, bx, by, bz);
     h_bulk_body<C, PP, OffT>(a.g, b, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hxo, a.Hyo, a.Hzo, a.Ex, a.Ey, a.Ez, a.dhx, a.dhy,
                        a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
+}
+
+// The core box and the slab boxes in one launch: the same cells and
+// arithmetic, one launch and one tail less per phase.
+template <typename OffT>
+__global__ void __launch_bounds__(kTX * kTY) k_h_bulk_all(HArgs a, BoxSet bs) {
+    int bx, by, bz;
+    const Box b = box_of(bs, (int)blockIdx.x, bx, by, bz);
+    if ((int)blockIdx.x < bs.first[1] && bs.core)
+        h_bulk_body<kCx, false, OffT>(a.g, b, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hxo, a.Hyo, a.Hzo, a.Ex, a.Ey, a.Ez,
+                                      a.dhx, a.dhy, a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
+    else
+        h_bulk_body<kCx | kCy | kCz, false, OffT>(a.g, b, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hxo, a.Hyo, a.Hzo, a.Ex,
+                                                  a.Ey, a.Ez, a.dhx, a.dhy, a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
 }
 
 template <int C, typename OffT = uint64_t>
@@ -447,9 +461,23 @@ __global__ void __launch_bounds__(kTX * kTY) k_h_bulk_batch(const HArgs* __restr
 template <typename IdxT, int C, bool PP = false, typename OffT = uint64_t>
 __global__ void __launch_bounds__(kTX * kTY) k_e_bulk(EArgs a, BoxSet bs) {
     int bx, by, bz;
-    const Box b = box_of(bs, bx, by, bz);
+    const Box b = box_of(bs, (int)blockIdx.x, bx, by, bz);
     e_bulk_body<IdxT, C, PP, OffT>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo, a.Hx, a.Hy, a.Hz,
                              static_cast<const IdxT*>(a.idx), a.tup, a.dex, a.dey, a.dez, a.cp, a.dx, a.dy, a.dz);
+}
+
+template <typename IdxT, typename OffT>
+__global__ void __launch_bounds__(kTX * kTY) k_e_bulk_all(EArgs a, BoxSet bs) {
+    int bx, by, bz;
+    const Box b = box_of(bs, (int)blockIdx.x, bx, by, bz);
+    const IdxT* idx = static_cast<const IdxT*>(a.idx);
+    if ((int)blockIdx.x < bs.first[1] && bs.core)
+        e_bulk_body<IdxT, kCx, false, OffT>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo, a.Hx, a.Hy, a.Hz,
+                                            idx, a.tup, a.dex, a.dey, a.dez, a.cp, a.dx, a.dy, a.dz);
+    else
+        e_bulk_body<IdxT, kCx | kCy | kCz, false, OffT>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo,
+                                                        a.Hx, a.Hy, a.Hz, idx, a.tup, a.dex, a.dey, a.dez, a.cp, a.dx,
+                                                        a.dy, a.dz);
 }
 
 template <typename IdxT, int C, typename OffT = uint64_t>
@@ -537,11 +565,21 @@ __device__ __forceinline__ float from_lane_above(float v, float last) {
 
 constexpr int kSpRows = 2;   // y rows marched together by one wave
 
+// Work-groups from nsp on update H of the y/z slab boxes (k_h_bulk, ping-pong):
+// they read the step-start state as the core does, so the launch is one where
+// there were two.
 template <typename IdxT, int C>
-__global__ void __launch_bounds__(64 * kSY) k_step_sp(SpArgs a, Box b) {
+__global__ void __launch_bounds__(64 * kSY) k_step_sp(SpArgs a, Box b, int nsp, HArgs h, BoxSet slabs) {
     constexpr int R = kSpRows;
     constexpr bool kPacked = sizeof(IdxT) == 1;
     __shared__ float stup[kPacked ? kSpTupMax * 6 : 1];
+    if ((int)blockIdx.x >= nsp) {
+        int bx, by, bz;
+        const Box sb = box_of(slabs, (int)blockIdx.x - nsp, bx, by, bz);
+        h_bulk_body<kCx | kCy | kCz, true, uint32_t>(h.g, sb, bx, by, bz, h.Hx, h.Hy, h.Hz, h.Hxo, h.Hyo, h.Hzo, h.Ex,
+                                                     h.Ey, h.Ez, h.dhx, h.dhy, h.dhz, h.DB, h.cp, h.dx, h.dy, h.dz);
+        return;
+    }
     if (kPacked) {   // before any wave leaves: every wave reaches the barrier
         const int tid = (int)(threadIdx.y * blockDim.x + threadIdx.x);
         for (int q = tid; q < a.n_tup * 6; q += (int)(blockDim.x * blockDim.y)) stup[q] = a.tup[q];

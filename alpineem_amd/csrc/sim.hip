@@ -253,6 +253,15 @@ constexpr int kPlanes = 4;
 constexpr int kSpPlanes = 8;
 constexpr long long kBulkGroups = 4096, kSlabGroups = 2048, kSpGroups = 800;
 
+// Grids up to kOneLaunchCells update the core box and the slab boxes of a
+// phase in one launch (the single pass with the slabs' H), which saves a launch
+// and lets the slabs fill the core's last work-groups; larger ones keep two,
+// since the combined kernel holds the registers of both.  Step, two launches /
+// one: single pass at 40^3 24 / 20 us, 100^3 51 / 49, 160^3 106 / 100, 256^3
+// 306 / 305, 320^3 472 / 477, 400^3 879 / 897; H and E phases at 40^3 25 / 18,
+// 160^3 124 / 118, 256^3 397 / 393, 400^3 1080 / 1092.
+constexpr long long kOneLaunchCells = 20000000;
+
 // Parts of a step, in the order the reference applies them.
 enum : unsigned {
     kPartHBulk = 1u << 0,    // bulk H (+ fused CPML)
@@ -426,6 +435,8 @@ struct aem_sim {
     bool fuse_cpml = false;        // CPML corrections folded into the bulk kernels
     RDiv rdv[3] = {};              // the CPML kernels' divisions by dx, dy, dz
     std::vector<Launch> bulk;      // bulk launches of each phase; [0] is the core when fused
+    Launch all_boxes{};            // core and slabs in one launch
+    bool one_launch = false;
     HArgs ha{};                    // bulk kernel arguments (fields, tables, CPML state)
     EArgs ea{};
     PortArgs pa{};                 // port kernel arguments
@@ -449,7 +460,6 @@ struct aem_sim {
     bool sp_ok = false;            // the deck admits it (set at creation)
     bool batched = false;          // a batch steps this simulation: in-place kernels only
     Box sp_box{};                  // core box of the single-pass kernel
-    std::vector<std::pair<Box, int>> sp_parts;   // its launches (box, slab tests compiled in)
     int par = 0;                   // which buffer set holds the fields now
     // k_adj_record reads E before its update, which the single pass has
     // already written; a design box records inside k_e_design, after it
@@ -868,6 +878,14 @@ void aem_sim::create(const aem_sim_options* opt) {
     rdv[1] = make_rdiv(v.dy, v.kmax != 0);
     rdv[2] = make_rdiv(v.dz, v.kmax != 0);
     bulk = bulk_launches(v, fuse_cpml, planes, !planes_set);
+    if (bulk.size() == 2 && bulk[0].c == kCx && bulk[0].bs.n == 1 && bulk[0].cells() > 0 &&
+        bulk[0].cells() + bulk[1].cells() <= kOneLaunchCells) {
+        std::vector<Box> boxes{bulk[0].bs.b[0]};
+        for (int q = 0; q < bulk[1].bs.n; ++q) boxes.push_back(bulk[1].bs.b[q]);
+        all_boxes = make_launch(boxes, kCx | kCy | kCz);
+        all_boxes.bs.core = 1;
+        one_launch = true;
+    }
     for (int f = 0; f < 6; ++f)
         for (int q = 0; q < 2; ++q) {
             cpH.pso[f][q] = cpH.psi[f][q];
@@ -886,11 +904,9 @@ void aem_sim::create(const aem_sim_options* opt) {
         const long long groups = (long long)cdiv(sp_box.ni, 64) * cdiv(sp_box.nj, kSY * kSpRows) * sp_box.nk;
         sp_box.kc = planes_set ? planes : (int)std::max(1LL, std::min<long long>(kSpPlanes, groups / kSpGroups));
         if (!planes_set) sp_box.kc = (int)cdiv(sp_box.nk, cdiv(sp_box.nk, sp_box.kc));   // chunks of equal length
-        // one launch with the x-slab test compiled in: measured at 400^3,
-        // separate launches for the slab-free x tiles (no slab test, fewer
-        // registers) and the two x-slab tiles of each row took 5-12% longer,
-        // in sequence or on a second stream beside them
-        sp_parts.push_back({sp_box, (int)kCx});
+        // (separate launches for the slab-free x tiles, no slab test and fewer
+        // registers, and the two x-slab tiles of each row took 5-12% longer at
+        // 400^3, in sequence or on a second stream beside them)
         if (v.idx_bytes == 1) {   // word (cell of plane 1, q) = bytes of planes 4q+1 .. 4q+4
             const size_t pl = (size_t)v.plane, nq = (size_t)(v.NZ + 3) / 4;
             std::vector<uint32_t> w(pl * nq, 0u);
@@ -1283,14 +1299,19 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     if (sp) {
         const SpArgs sa{g, Ex, Ey, Ez, Hx, Hy, Hz, F2[0], F2[1], F2[2], F2[3], F2[4], F2[5], d_idx, d_idx4, d_tup,
                         n_tup, d_den[0], d_den[1], d_den[2], d_den[3], d_den[4], d_den[5], v.DB, cpH, cpE, v.dx, v.dy, v.dz};
-        for (const auto& part : sp_parts) {
-            const Box& b = part.first;
-            const unsigned nblk = cdiv(b.ni, 64) * cdiv(b.nj, kSY * kSpRows) * cdiv(b.nk, b.kc);
-            if (part.second == kCx) k_step_sp<IdxT, kCx><<<nblk, dim3(64, kSY), 0, s>>>(sa, b);
-            else k_step_sp<IdxT, 0><<<nblk, dim3(64, kSY), 0, s>>>(sa, b);
-        }
+        const Box& b = sp_box;
+        const unsigned nsp = cdiv(b.ni, 64) * cdiv(b.nj, kSY * kSpRows) * cdiv(b.nk, b.kc);
+        // (timed phases launch the slabs by themselves)
+        const bool with = !mark && one_launch;
+        k_step_sp<IdxT, kCx><<<nsp + (with ? bulk[1].blocks() : 0u), dim3(64, kSY), 0, s>>>(sa, b, (int)nsp, ha,
+                                                                                           with ? bulk[1].bs : BoxSet{});
     } else if (parts & kPartHBulk) {
-        h_bulk(bulk[0]);
+        if (one_launch && !mark) {
+            if (off32) k_h_bulk_all<uint32_t><<<all_boxes.blocks(), bt, 0, s>>>(ha, all_boxes.bs);
+            else k_h_bulk_all<uint64_t><<<all_boxes.blocks(), bt, 0, s>>>(ha, all_boxes.bs);
+        } else {
+            h_bulk(bulk[0]);
+        }
     }
     if (mark) HIPCHK(hipEventRecord(mark[1], st));
     if (sp) {
@@ -1299,13 +1320,14 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
         es.Hy = F2[4];
         es.Hz = F2[5];
         // (single-pass decks always have 32-bit offsets)
-        for (size_t q = 1; q < bulk.size(); ++q)
-            k_h_bulk<kCx | kCy | kCz, true, uint32_t><<<bulk[q].blocks(), bt, 0, s>>>(ha, bulk[q].bs);
+        if (mark || !one_launch)
+            for (size_t q = 1; q < bulk.size(); ++q)
+                k_h_bulk<kCx | kCy | kCz, true, uint32_t><<<bulk[q].blocks(), bt, 0, s>>>(ha, bulk[q].bs);
         for (size_t q = 1; q < bulk.size(); ++q)
             k_e_bulk<IdxT, kCx | kCy | kCz, true, uint32_t><<<bulk[q].blocks(), bt, 0, s>>>(es, bulk[q].bs);
         flip();
         Ex = F[0]; Ey = F[1]; Ez = F[2]; Hx = F[3]; Hy = F[4]; Hz = F[5];
-    } else if (parts & kPartHBulk) {
+    } else if ((parts & kPartHBulk) && (!one_launch || mark)) {
         for (size_t q = 1; q < bulk.size(); ++q) h_bulk(bulk[q]);
     }
     const float dd[3] = {v.dx, v.dy, v.dz};
@@ -1355,9 +1377,16 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
 
     // ---- E phase ----  (marks: [2,3] the core bulk launch, [3,4] the rest of E)
     if (mark) HIPCHK(hipEventRecord(mark[2], st));
-    if ((parts & kPartEBulk) && !sp) e_bulk(bulk[0]);
+    if ((parts & kPartEBulk) && !sp) {
+        if (one_launch && !mark) {
+            if (off32) k_e_bulk_all<IdxT, uint32_t><<<all_boxes.blocks(), bt, 0, s>>>(ea, all_boxes.bs);
+            else k_e_bulk_all<IdxT, uint64_t><<<all_boxes.blocks(), bt, 0, s>>>(ea, all_boxes.bs);
+        } else {
+            e_bulk(bulk[0]);
+        }
+    }
     if (mark) HIPCHK(hipEventRecord(mark[3], st));
-    if ((parts & kPartEBulk) && !sp)
+    if ((parts & kPartEBulk) && !sp && (!one_launch || mark))
         for (size_t q = 1; q < bulk.size(); ++q) e_bulk(bulk[q]);
     if ((parts & kPartEPre) && des_on)
         k_e_design<<<cdiv(des.nedge, 256), 256, 0, s>>>(g, des, Ex, Ey, Ez, Hx, Hy, Hz, d_den[0], d_den[1], d_den[2],
