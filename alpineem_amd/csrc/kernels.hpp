@@ -1319,79 +1319,130 @@ __device__ __forceinline__ float gap_loop_current(const Grid& g, int dir, const 
     return c;
 }
 
-__device__ __forceinline__ void ports_h_body(const Grid& g, const PortDev* ports, int np, int M, float* V, float* I,
-                                             float* Iout, int T, const float* Hx, const float* Hy, const float* Hz,
-                                             float dx, float dy, float dz, const Pulse& pu, const int* step) {
-    const int n = *step;
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < np; ++q) {
-            const PortDev pt = ports[q];
-            float c = gap_loop_current(g, pt.dir, pt.loc, pt.size, Hx, Hy, Hz, dx, dy, dz);
+// The same sum by one wave: the lanes form 64 terms at a time (their loads in
+// flight together), the sum takes them in the loop order.
+__device__ __forceinline__ float gap_loop_current_wave(const Grid& g, int dir, const int* loc, const int* size,
+                                                       const float* Hx, const float* Hy, const float* Hz, float dx,
+                                                       float dy, float dz, int lane) {
+    const int l1 = loc[0], l2 = loc[1], l3 = loc[2];
+    const int d1 = size[0] + l1 - 1, d2 = size[1] + l2 - 1, d3 = size[2] + l3 - 1;
+    // per outer cell (along the gap), the terms along the first and then the
+    // second transverse axis
+    const int nA = dir == 0 ? size[1] : size[0], nB = dir == 2 ? size[1] : size[2];
+    const int per = nA + nB, total = per * (dir == 0 ? size[0] : (dir == 1 ? size[1] : size[2]));
+    float c = 0.0f;
+    for (int base = 0; base < total; base += 64) {
+        const int t = min(base + lane, total - 1);
+        const int o = t / per, r = t % per;
+        float term;
+        if (dir == 0) {
+            const int ii = l1 + o;
+            if (r < nA) term = dy * (Hy[off(g, ii, l2 + r, l3 - 1)] - Hy[off(g, ii, l2 + r, d3)]);
+            else term = dz * (Hz[off(g, ii, l2, l3 + r - nA)] - Hz[off(g, ii, d2 - 1, l3 + r - nA)]);
+        } else if (dir == 1) {
+            const int jj = l2 + o;
+            if (r < nA) term = dx * (Hx[off(g, l1 + r, jj, l3)] - Hx[off(g, l1 + r, jj, d3 - 1)]);
+            else term = dz * (Hz[off(g, l1 - 1, jj, l3 + r - nA)] - Hz[off(g, d1, jj, l3 + r - nA)]);
+        } else {
+            const int kk = l3 + o;
+            if (r < nA) term = dx * (Hx[off(g, l1 + r, l2 - 1, kk)] - Hx[off(g, l1 + r, d2, kk)]);
+            else term = dy * (Hy[off(g, l1, l2 + r - nA, kk)] - Hy[off(g, d1 - 1, l2 + r - nA, kk)]);
+        }
+        const int cnt = min(64, total - base);
+        for (int l = 0; l < cnt; ++l)
+            c = c + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(term), l));
+    }
+    return c;
+}
+
+// The ports' H phase (DoH) and E phase (DoE) by one work-group of 256 threads
+// (tid): a wave per port for the gap current, all threads along the lines.  With both
+// phases, H has been updated and E of the gaps is overwritten as the reference
+// does after the bulk E update.  inc: also advance the step counter.
+template <bool DoH, bool DoE>
+__device__ __forceinline__ void ports_body(const PortArgs& a, int tid, int* inc) {
+    const int n = *a.step;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    if (DoH) {
+        for (int q = wave; q < a.np; q += 4) {
+            const PortDev pt = a.ports[q];
+            float c = gap_loop_current_wave(a.g, pt.dir, pt.loc, pt.size, a.Hx, a.Hy, a.Hz, a.dx, a.dy, a.dz, lane);
             c = rdiv(c * pt.cur_num, pt.cdv);
-            I[(long long)q * M] = c;
-            Iout[(long long)q * T + (n - 1)] = c;
+            if (lane == 0) {
+                a.I[(long long)q * a.M] = c;
+                a.Iout[(long long)q * a.T + (n - 1)] = c;
+            }
         }
-    }
-    // 1-D line current, j = 2..M-1 (0-based j-1); reads V only
-    for (int q = 0; q < np; ++q) {
-        const float kI = ports[q].kI;
-        float* Iq = I + (long long)q * M;
-        const float* Vq = V + (long long)q * M;
-        for (int j = 2 + threadIdx.x; j <= M - 1; j += blockDim.x) Iq[j - 1] = Iq[j - 1] - kI * (Vq[j] - Vq[j - 1]);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < np; ++q)
-            if (ports[q].excited) {
-                float* Iq = I + (long long)q * M;
-                Iq[1] = Iq[1] - ports[q].kI * pu.src[n - 1];
+        // 1-D line current, j = 2..M-1 (0-based j-1); reads V only
+        for (int q = 0; q < a.np; ++q) {
+            const float kI = a.ports[q].kI;
+            float* Iq = a.I + (long long)q * a.M;
+            const float* Vq = a.V + (long long)q * a.M;
+            for (int j = 2 + tid; j <= a.M - 1; j += 256) {
+                float v = Iq[j - 1] - kI * (Vq[j] - Vq[j - 1]);
+                if (j == 2 && a.ports[q].excited) v = v - kI * a.pu.src[n - 1];
+                Iq[j - 1] = v;
             }
+        }
+        if (DoE) __syncthreads();
     }
-}
-
-__device__ __forceinline__ void ports_e_body(const Grid& g, const PortDev* ports, int np, int M, float* V,
-                                             const float* I, float* Vout, int T, float* Ex, float* Ey, float* Ez,
-                                             const Pulse& pu, const int* step) {
-    const int n = *step;
-    for (int q = 0; q < np; ++q) {
-        const float kV = ports[q].kV;
-        float* Vq = V + (long long)q * M;
-        const float* Iq = I + (long long)q * M;
-        for (int j = 2 + threadIdx.x; j <= M - 1; j += blockDim.x) Vq[j - 1] = Vq[j - 1] - kV * (Iq[j - 1] - Iq[j - 2]);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int q = 0; q < np; ++q)
-            if (ports[q].excited) {
-                float* Vq = V + (long long)q * M;
-                Vq[1] = Vq[1] + ports[q].kS * pu.src[pu.T + n - 1];
+    if (DoE) {
+        for (int q = 0; q < a.np; ++q) {
+            const float kV = a.ports[q].kV;
+            float* Vq = a.V + (long long)q * a.M;
+            const float* Iq = a.I + (long long)q * a.M;
+            for (int j = 2 + tid; j <= a.M - 1; j += 256) {
+                float v = Vq[j - 1] - kV * (Iq[j - 1] - Iq[j - 2]);
+                if (j == 2 && a.ports[q].excited) v = v + a.ports[q].kS * a.pu.src[a.pu.T + n - 1];
+                Vq[j - 1] = v;
             }
-        for (int q = 0; q < np; ++q) {
-            const PortDev pt = ports[q];
-            const float v2 = V[(long long)q * M + 1];
-            float* F = pt.dir == 0 ? Ex : (pt.dir == 1 ? Ey : Ez);
+        }
+        __syncthreads();
+        for (int q = 0; q < a.np && wave == 0; ++q) {   // one wave: gaps that share cells keep the ports' order
+            const PortDev pt = a.ports[q];
+            const float v2 = a.V[(long long)q * a.M + 1];
+            float* F = pt.dir == 0 ? a.Ex : (pt.dir == 1 ? a.Ey : a.Ez);
             const float val = rdiv(1.0f * v2, pt.gdv);
-            for (int ii = pt.loc[0]; ii <= pt.loc[0] + pt.size[0] - 1; ++ii)
-                for (int jj = pt.loc[1]; jj <= pt.loc[1] + pt.size[1] - 1; ++jj)
-                    for (int kk = pt.loc[2]; kk <= pt.loc[2] + pt.size[2] - 1; ++kk) F[off(g, ii, jj, kk)] = val;
-            Vout[(long long)q * T + (n - 1)] = v2;
+            const int cells = pt.size[0] * pt.size[1] * pt.size[2];
+            for (int t = lane; t < cells; t += 64) {
+                const int kk = t % pt.size[2], jj = t / pt.size[2] % pt.size[1], ii = t / (pt.size[2] * pt.size[1]);
+                F[off(a.g, pt.loc[0] + ii, pt.loc[1] + jj, pt.loc[2] + kk)] = val;
+            }
+            if (lane == 0) a.Vout[(long long)q * a.T + (n - 1)] = v2;
         }
+        if (inc && tid == 0) *inc = n + 1;   // every thread has read n before the barrier above
     }
 }
 
-__global__ void __launch_bounds__(256) k_ports_h(PortArgs a) {
-    ports_h_body(a.g, a.ports, a.np, a.M, a.V, a.I, a.Iout, a.T, a.Hx, a.Hy, a.Hz, a.dx, a.dy, a.dz, a.pu, a.step);
-}
-__global__ void __launch_bounds__(256) k_ports_e(PortArgs a) {
-    ports_e_body(a.g, a.ports, a.np, a.M, a.V, a.I, a.Vout, a.T, a.Ex, a.Ey, a.Ez, a.pu, a.step);
-}
+__global__ void __launch_bounds__(256) k_ports_h(PortArgs a) { ports_body<true, false>(a, (int)threadIdx.x, nullptr); }
+__global__ void __launch_bounds__(256) k_ports_e(PortArgs a) { ports_body<false, true>(a, (int)threadIdx.x, nullptr); }
 __global__ void __launch_bounds__(256) k_ports_h_batch(const PortArgs* __restrict__ args) {
-    const PortArgs& a = args[blockIdx.x];
-    ports_h_body(a.g, a.ports, a.np, a.M, a.V, a.I, a.Iout, a.T, a.Hx, a.Hy, a.Hz, a.dx, a.dy, a.dz, a.pu, a.step);
+    ports_body<true, false>(args[blockIdx.x], (int)threadIdx.x, nullptr);
 }
 __global__ void __launch_bounds__(256) k_ports_e_batch(const PortArgs* __restrict__ args) {
-    const PortArgs& a = args[blockIdx.x];
-    ports_e_body(a.g, a.ports, a.np, a.M, a.V, a.I, a.Vout, a.T, a.Ex, a.Ey, a.Ez, a.pu, a.step);
+    ports_body<false, true>(args[blockIdx.x], (int)threadIdx.x, nullptr);
+}
+
+// After the single pass: E of the y/z slab boxes (ping-pong) and, in the
+// first work-group when `ports` is set, the ports' H and E phases.  They read
+// the new H and write E of the gaps, which the slabs, a cell clear of every
+// port (cpml_fusable), neither read nor write; so the ports' chain of small
+// loads and the two launches it had hide behind the slabs.
+template <typename IdxT>
+__global__ void __launch_bounds__(kTX * kTY) k_e_slabs(EArgs a, BoxSet bs, PortArgs p, int ports, int* inc) {
+    int g = (int)blockIdx.x;
+    if (ports) {
+        if (g == 0) {
+            ports_body<true, true>(p, (int)(threadIdx.y * kTX + threadIdx.x), inc);
+            return;
+        }
+        --g;
+    }
+    int bx, by, bz;
+    const Box b = box_of(bs, g, bx, by, bz);
+    e_bulk_body<IdxT, kCx | kCy | kCz, true, uint32_t>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo, a.Hx,
+                                                       a.Hy, a.Hz, static_cast<const IdxT*>(a.idx), a.tup, a.dex, a.dey,
+                                                       a.dez, a.cp, a.dx, a.dy, a.dz);
 }
 
 // ---------------------------------------------------------------------------
@@ -1654,7 +1705,7 @@ __global__ void k_sheet_pbc(Sheets s, int mode, int src, int n_other) {
 __global__ void __launch_bounds__(256) k_plane_sums(Grid g, int axis, int lo_pos, int hi_pos, int u0, int u1, int v0,
                                                     int v1, const float* Ea, const float* Eb, float c_a, float c_b1,
                                                     float c_b2, int minus_b, double* refl, double* trans,
-                                                    const int* step) {
+                                                    int* step, int inc) {
     // axis 0: planes x=lo/hi, (u,v)=(j,k), Ea=Ez, Eb=Ey;  axis 1: (u,v)=(i,k), Ea=Ez, Eb=Ex;
     // axis 2: (u,v)=(i,j), Ea=Ey, Eb=Ex
     __shared__ double sr[256], st[256];
@@ -1688,6 +1739,7 @@ __global__ void __launch_bounds__(256) k_plane_sums(Grid g, int axis, int lo_pos
     if (threadIdx.x == 0) {
         refl[n - 1] = sr[0];
         trans[n - 1] = st[0];
+        if (inc) *step = n + 1;   // ends the step: every thread has read n before the barriers above
     }
 }
 
@@ -1754,12 +1806,48 @@ __device__ __forceinline__ void ntff_currents_body(const Grid& g, const NtffFace
     f.J[face][1][fo] = j1;
 }
 
-// (fstep: the step these currents belong to, read by the binning, which may
-// run beside the following step)
-__global__ void k_ntff_currents(Grid g, NtffFaces f, const float* Ex, const float* Ey, const float* Ez,
-                                const float* Hx, const float* Hy, const float* Hz, const int* step, int* fstep) {
-    if (blockIdx.x + blockIdx.y + blockIdx.z + threadIdx.x + threadIdx.y == 0) *fstep = *step;
-    ntff_currents_body(g, f, blockIdx.z, Ex, Ey, Ez, Hx, Hy, Hz);
+// The end of a step: phase-centre samples (f90:8259-8290) when do_pc, and the
+// step counter.  By one thread, of a kernel of its own or of the step's last
+// kernel that reads the counter.
+struct StepEnd {
+    int on;
+    int ic, jc, kc, T, do_pc;
+    float* pc;
+};
+
+__device__ __forceinline__ void step_end_body(const Grid& g, const StepEnd& e, const float* Ex, const float* Ey,
+                                              const float* Ez, const float* Hx, const float* Hy, const float* Hz,
+                                              int* step) {
+    const int n = *step, T = e.T;
+    if (e.do_pc) {
+        const long long o = off(g, e.ic, e.jc, e.kc);
+        float* P0 = e.pc;
+        float* P1 = e.pc + (long long)(T + 1);
+        float* P2 = e.pc + 2 * (long long)(T + 1);
+        float* P3 = e.pc + 3 * (long long)(T + 1);
+        float* P4 = e.pc + 4 * (long long)(T + 1);
+        float* P5 = e.pc + 5 * (long long)(T + 1);
+        P0[n - 1] = (Ex[o] + Ex[o + g.PX] + Ex[o + g.plane] + Ex[o + g.PX + g.plane]) / 4.0f;
+        P1[n - 1] = (Ey[o] + Ey[o + 1] + Ey[o + g.plane] + Ey[o + 1 + g.plane]) / 4.0f;
+        P2[n - 1] = (Ez[o] + Ez[o + 1] + Ez[o + g.PX] + Ez[o + 1 + g.PX]) / 4.0f;
+        const float hx = (Hx[o] + Hx[o + 1]) / 4.0f, hy = (Hy[o] + Hy[o + g.PX]) / 4.0f,
+                    hz = (Hz[o] + Hz[o + g.plane]) / 4.0f;
+        P3[n - 1] = hx; P4[n - 1] = hy; P5[n - 1] = hz;
+        if (n < T) { P3[n] = hx; P4[n] = hy; P5[n] = hz; }
+    }
+    *step = n + 1;
+}
+
+// fstep: the step these currents belong to, read by the binning, which may
+// run beside the following step.  With e.on the grid has a seventh z layer,
+// one thread of which ends the step (the only reader of the counter here).
+__global__ void k_ntff_currents(Grid g, NtffFaces f, StepEnd e, const float* Ex, const float* Ey, const float* Ez,
+                                const float* Hx, const float* Hy, const float* Hz, int* step, int* fstep) {
+    if (blockIdx.z == (e.on ? 6u : 0u) && blockIdx.x + blockIdx.y + threadIdx.x + threadIdx.y == 0) {
+        *fstep = *step;
+        if (e.on) step_end_body(g, e, Ex, Ey, Ez, Hx, Hy, Hz, step);
+    }
+    if (blockIdx.z < 6) ntff_currents_body(g, f, blockIdx.z, Ex, Ey, Ez, Hx, Hy, Hz);
 }
 
 // NTFF retarded-time binning (f90:7643-7927).  Index and weight arithmetic is
@@ -2625,26 +2713,9 @@ __global__ void k_phase_centre(Grid g, int ic, int jc, int kc, int T, const floa
 __global__ void k_step_inc(int* step) { *step = *step + 1; }
 
 // Phase-centre samples (when do_pc) and the step counter in one launch.
-__global__ void k_step_end(Grid g, int ic, int jc, int kc, int T, const float* Ex, const float* Ey, const float* Ez,
-                           const float* Hx, const float* Hy, const float* Hz, float* pc, int* step, int do_pc) {
-    const int n = *step;
-    if (do_pc) {
-        const long long o = off(g, ic, jc, kc);
-        float* P0 = pc;
-        float* P1 = pc + (long long)(T + 1);
-        float* P2 = pc + 2 * (long long)(T + 1);
-        float* P3 = pc + 3 * (long long)(T + 1);
-        float* P4 = pc + 4 * (long long)(T + 1);
-        float* P5 = pc + 5 * (long long)(T + 1);
-        P0[n - 1] = (Ex[o] + Ex[o + g.PX] + Ex[o + g.plane] + Ex[o + g.PX + g.plane]) / 4.0f;
-        P1[n - 1] = (Ey[o] + Ey[o + 1] + Ey[o + g.plane] + Ey[o + 1 + g.plane]) / 4.0f;
-        P2[n - 1] = (Ez[o] + Ez[o + 1] + Ez[o + g.PX] + Ez[o + 1 + g.PX]) / 4.0f;
-        const float hx = (Hx[o] + Hx[o + 1]) / 4.0f, hy = (Hy[o] + Hy[o + g.PX]) / 4.0f,
-                    hz = (Hz[o] + Hz[o + g.plane]) / 4.0f;
-        P3[n - 1] = hx; P4[n - 1] = hy; P5[n - 1] = hz;
-        if (n < T) { P3[n] = hx; P4[n] = hy; P5[n] = hz; }
-    }
-    *step = n + 1;
+__global__ void k_step_end(Grid g, StepEnd e, const float* Ex, const float* Ey, const float* Ez, const float* Hx,
+                           const float* Hy, const float* Hz, int* step) {
+    step_end_body(g, e, Ex, Ey, Ez, Hx, Hy, Hz, step);
 }
 
 // ---------------------------------------------------------------------------

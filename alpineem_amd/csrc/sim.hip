@@ -1292,6 +1292,24 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     // boxes' H and E as ping-pong bulk launches; the rest of the step then
     // runs on the new buffer set
     const bool sp = (parts & kPartHBulk) && (parts & kPartEBulk) && sp_active();
+    // the ports of a single-pass step run beside its slabs' E phase
+    const bool sp_ports = sp && !mark && bulk.size() > 1 && v.n_ports > 0 && (parts & kPartHPort) && (parts & kPartEPort);
+    // the step's last kernel that reads the step counter also advances it
+    // (and takes the phase-centre samples); a kernel of its own does where
+    // others read the counter after that one, or a phase is timed
+    enum { kEndNone, kEndOwn, kEndCurrents, kEndSums, kEndPorts } end = kEndNone;
+    const bool ff_step = (parts & kPartNtff) && v.n_angles > 0 && ntff_mode != AEM_NTFF_OFF;
+    const bool pc_on = (parts & kPartOutPost) && v.n_angles > 0 && v.plane_wave_amp > 0;
+    if (parts & kPartStep) {
+        const bool readers = ((parts & kPartObjective) && (obj_on || ff_on)) || ((parts & kPartOutPost) && vid_on);
+        if (mark || readers || v.kmax) end = kEndOwn;
+        else if (ff_step) end = kEndCurrents;
+        else if (pc_on) end = kEndOwn;
+        else if ((parts & kPartOutPre) && v.plane_sum_axis >= 0) end = kEndSums;
+        else if (sp_ports && !des_on && !rec_on) end = kEndPorts;
+        else end = kEndOwn;
+    }
+    const StepEnd se{end == kEndCurrents ? 1 : 0, v.ic, v.jc, v.kc, v.time_steps, pc_on ? 1 : 0, d_pc};
 
     // ---- H phase ----  (marks: [0,1] the core bulk launch -- the single-pass
     // launch when sp --, [1,2] the rest of H)
@@ -1323,9 +1341,10 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
         if (mark || !one_launch)
             for (size_t q = 1; q < bulk.size(); ++q)
                 k_h_bulk<kCx | kCy | kCz, true, uint32_t><<<bulk[q].blocks(), bt, 0, s>>>(ha, bulk[q].bs);
+        flip();          // the port arguments now name the new fields
         for (size_t q = 1; q < bulk.size(); ++q)
-            k_e_bulk<IdxT, kCx | kCy | kCz, true, uint32_t><<<bulk[q].blocks(), bt, 0, s>>>(es, bulk[q].bs);
-        flip();
+            k_e_slabs<IdxT><<<bulk[q].blocks() + (sp_ports ? 1u : 0u), bt, 0, s>>>(
+                es, bulk[q].bs, pa, sp_ports ? 1 : 0, end == kEndPorts ? d_step : nullptr);
         Ex = F[0]; Ey = F[1]; Ez = F[2]; Hx = F[3]; Hy = F[4]; Hz = F[5];
     } else if ((parts & kPartHBulk) && (!one_launch || mark)) {
         for (size_t q = 1; q < bulk.size(); ++q) h_bulk(bulk[q]);
@@ -1355,7 +1374,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
             }
         }
     }
-    if ((parts & kPartHPort) && v.n_ports > 0) k_ports_h<<<1, 256, 0, s>>>(pa);
+    if ((parts & kPartHPort) && v.n_ports > 0 && !sp_ports) k_ports_h<<<1, 256, 0, s>>>(pa);
     if (parts & kPartHPost) {
         const long long tx = (long long)(std::max(v.npml[0] - 1, 0) + std::max(v.npml[1] - 1, 0)) * (v.NY - 1) * (v.NZ - 1);
         const long long ty = (long long)(v.NX - 1) * (std::max(v.npml[2] - 1, 0) + std::max(v.npml[3] - 1, 0)) * (v.NZ - 1);
@@ -1414,7 +1433,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
             }
         }
     }
-    if ((parts & kPartEPort) && v.n_ports > 0) k_ports_e<<<1, 256, 0, s>>>(pa);
+    if ((parts & kPartEPort) && v.n_ports > 0 && !sp_ports) k_ports_e<<<1, 256, 0, s>>>(pa);
     if ((parts & kPartSpiceE) && v.n_spice > 0) k_spice_e<<<1, 64, 0, s>>>(spa);
     if (parts & kPartEPost) {
         const long long tx = (long long)(std::max(v.npml[0] - 1, 0) + std::max(v.npml[1] - 1, 0)) * (v.NY - 1) * (v.NZ - 1);
@@ -1455,29 +1474,29 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
         // (x normal: Ez, Ey with k_y, k_z; y normal: Ez, Ex with k_x, k_z; z normal: Ex, Ey with k_y, k_x)
         const float k1 = ax == 2 ? v.k_exc[1] : v.k_exc[p], k2 = ax == 2 ? v.k_exc[0] : v.k_exc[q];
         k_plane_sums<<<1, 256, 0, s>>>(g, ax, lo, hi, v.ff_lo[p], v.ff_hi[p], v.ff_lo[q], v.ff_hi[q], Ea, Eb, k1, k2,
-                                        1.0f, 1, d_refl, d_trans, d_step);
+                                        1.0f, 1, d_refl, d_trans, d_step, end == kEndSums ? 1 : 0);
         k_plane_sums<<<1, 256, 0, s>>>(g, ax, lo, hi, v.ff_lo[p], v.ff_hi[p], v.ff_lo[q], v.ff_hi[q], Ea, Eb, k2, k1,
-                                        1.0f, 0, d_refl2, d_trans2, d_step);
+                                        1.0f, 0, d_refl2, d_trans2, d_step, 0);
     } else if ((parts & kPartOutPre) && v.plane_sum_axis >= 0) {
         const int ax = v.plane_sum_axis;
         const int lo = v.tf_lo[ax], hi = v.tf_hi[ax];
         if (ax == 0)
             k_plane_sums<<<1, 256, 0, s>>>(g, 0, lo, hi, v.ff_lo[1], v.ff_hi[1], v.ff_lo[2], v.ff_hi[2], Ez, Ey, v.s_pol,
-                                            v.c_pol, v.c_ph, 1, d_refl, d_trans, d_step);
+                                            v.c_pol, v.c_ph, 1, d_refl, d_trans, d_step, end == kEndSums ? 1 : 0);
         else if (ax == 1)
             k_plane_sums<<<1, 256, 0, s>>>(g, 1, lo, hi, v.ff_lo[0], v.ff_hi[0], v.ff_lo[2], v.ff_hi[2], Ez, Ex, v.s_pol,
-                                            v.c_pol, v.s_ph, 0, d_refl, d_trans, d_step);
+                                            v.c_pol, v.s_ph, 0, d_refl, d_trans, d_step, end == kEndSums ? 1 : 0);
         else
             k_plane_sums<<<1, 256, 0, s>>>(g, 2, lo, hi, v.ff_lo[0], v.ff_hi[0], v.ff_lo[1], v.ff_hi[1], Ey, Ex, v.ps_c1,
-                                            v.ps_c2, 1.0f, 0, d_refl, d_trans, d_step);
+                                            v.ps_c2, 1.0f, 0, d_refl, d_trans, d_step, end == kEndSums ? 1 : 0);
     }
-    if ((parts & kPartNtff) && v.n_angles > 0 && ntff_mode != AEM_NTFF_OFF) {
-        const dim3 gf(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6);
+    if (ff_step) {
+        const dim3 gf(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), se.on ? 7 : 6);
         const int slot = beside ? beside->slot() : 0;
         const NtffFaces& nf = nfs[slot];
         int* fstep = d_ffstep + slot;
         if (beside) beside->before_currents(s);
-        k_ntff_currents<<<gf, bb, 0, s>>>(g, nf, Ex, Ey, Ez, Hx, Hy, Hz, d_step, fstep);
+        k_ntff_currents<<<gf, bb, 0, s>>>(g, nf, se, Ex, Ey, Ez, Hx, Hy, Hz, d_step, fstep);
         const hipStream_t sb = beside ? beside->after_currents(s) : s;
         if (ntff_mode == AEM_NTFF_ORDERED) {
             if (nl.blocks() > kListUnits)
@@ -1504,10 +1523,9 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     }
     if ((parts & kPartOutPost) && vid_on)
         k_video<<<dim3(cdiv(vid.v1, 32), cdiv(vid.v2, 8)), bb, 0, s>>>(g, vid, Ex, Ey, Ez, Hx, Hy, Hz, d_step);
-    const bool pc_on = (parts & kPartOutPost) && v.n_angles > 0 && v.plane_wave_amp > 0;
-    if (parts & kPartStep)
-        k_step_end<<<1, 1, 0, s>>>(g, v.ic, v.jc, v.kc, T, Ex, Ey, Ez, Hx, Hy, Hz, d_pc, d_step, pc_on ? 1 : 0);
-    else if (pc_on)
+    if (end == kEndOwn)
+        k_step_end<<<1, 1, 0, s>>>(g, se, Ex, Ey, Ez, Hx, Hy, Hz, d_step);
+    else if (end == kEndNone && pc_on)
         k_phase_centre<<<1, 1, 0, s>>>(g, v.ic, v.jc, v.kc, T, Ex, Ey, Ez, Hx, Hy, Hz, d_pc, d_step);
     if (mark) HIPCHK(hipEventRecord(mark[5], st));
 }
