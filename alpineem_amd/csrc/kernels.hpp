@@ -1548,29 +1548,31 @@ __global__ void k_h_sheets(Grid g, Sheets s, int axis, float* Hx, float* Hy, flo
     }
 }
 
+// New special E of sheet cell (p, q) of plane pl.
+__device__ __forceinline__ float sheet_es(const Grid& g, const Sheets& s, int axis, int pl, int p, int q, const float* Hx,
+                                          const float* Hy, const float* Hz, const float* dex, const float* dey,
+                                          const float* dez, float dt, float ep0) {
+    const int c = s.pos[pl];
+    const int i = axis == 0 ? c : p, j = axis == 1 ? c : (axis == 0 ? p : q), k = axis == 2 ? c : q;
+    const long long so = sh_off(s, pl, p, q);
+    const float sg = s.sig[so], ep = s.ep[so];
+    const long long o = off(g, i, j, k);
+    float curl;
+    if (axis == 0) curl = (Hz[o] - Hz[o - g.PX]) * dey[j - 1] + (Hy[o - g.plane] - Hy[o]) * dez[k - 1];
+    else if (axis == 1) curl = (Hz[o - 1] - Hz[o]) * dex[i - 1] + (Hx[o] - Hx[o - g.plane]) * dez[k - 1];
+    else curl = (Hy[o] - Hy[o - 1]) * dex[i - 1] + (Hx[o - g.PX] - Hx[o]) * dey[j - 1];
+    return ((1.0f - sg * dt / (2.0f * ep0 * ep)) / (1.0f + sg * dt / (2.0f * ep0 * ep))) * s.es[so] +
+           ((dt / (ep0 * ep)) / (1.0f + sg * dt / (2.0f * ep0 * ep))) * curl;
+}
+
 __global__ void k_e_sheets(Grid g, Sheets s, int axis, const float* Hx, const float* Hy, const float* Hz,
                            const float* dex, const float* dey, const float* dez, float dt, float ep0) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x + 2;
     const int q = blockIdx.y * blockDim.y + threadIdx.y + 2;
-    for (int pl = 0; pl < s.np; ++pl) {
-        const int c = s.pos[pl];
-        int i, j, k;
-        float d1, d2;
-        if (axis == 0) { i = c; j = p; k = q; if (j > g.NY - 1 || k > g.NZ - 1) continue; }
-        else if (axis == 1) { i = p; j = c; k = q; if (i > g.NX - 1 || k > g.NZ - 1) continue; }
-        else { i = p; j = q; k = c; if (i > g.NX - 1 || j > g.NY - 1) continue; }
-        if (!sh_on(s, pl, p, q)) continue;
-        const long long so = sh_off(s, pl, p, q);
-        const float sg = s.sig[so], ep = s.ep[so];
-        const long long o = off(g, i, j, k);
-        float curl;
-        if (axis == 0) curl = (Hz[o] - Hz[o - g.PX]) * dey[j - 1] + (Hy[o - g.plane] - Hy[o]) * dez[k - 1];
-        else if (axis == 1) curl = (Hz[o - 1] - Hz[o]) * dex[i - 1] + (Hx[o] - Hx[o - g.plane]) * dez[k - 1];
-        else curl = (Hy[o] - Hy[o - 1]) * dex[i - 1] + (Hx[o - g.PX] - Hx[o]) * dey[j - 1];
-        (void)d1; (void)d2;
-        s.es[so] = ((1.0f - sg * dt / (2.0f * ep0 * ep)) / (1.0f + sg * dt / (2.0f * ep0 * ep))) * s.es[so] +
-                   ((dt / (ep0 * ep)) / (1.0f + sg * dt / (2.0f * ep0 * ep))) * curl;
-    }
+    if (p > s.P - 1 || q > s.Q - 1) return;
+    for (int pl = 0; pl < s.np; ++pl)
+        if (sh_on(s, pl, p, q))
+            s.es[sh_off(s, pl, p, q)] = sheet_es(g, s, axis, pl, p, q, Hx, Hy, Hz, dex, dey, dez, dt, ep0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1586,10 +1588,10 @@ struct DrudeBox {
     float* Eold;
 };
 
+// Drude update of box cell tid; returns its E.
 template <typename IdxT>
-__global__ void k_drude(Grid g, DrudeBox b, int comp, int P, float* E, const IdxT* idx, const float* tup) {
-    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (tid >= b.nb) return;
+__device__ __forceinline__ float drude_cell(const Grid& g, const DrudeBox& b, int comp, int P, float* E, const IdxT* idx,
+                                            const float* tup, long long tid) {
     const int bx = b.hi[0] - b.lo[0] + 1, by = b.hi[1] - b.lo[1] + 1;
     const int i = b.lo[0] + (int)(tid % bx);
     const int j = b.lo[1] + (int)((tid / bx) % by);
@@ -1601,6 +1603,13 @@ __global__ void k_drude(Grid g, DrudeBox b, int comp, int P, float* E, const Idx
     E[o] = e;
     const float eo = b.Eold[tid];
     for (int q = 0; q < P; ++q) b.J[q * b.nb + tid] = b.Ja[q * b.nb + tid] * b.J[q * b.nb + tid] + b.Jb[q * b.nb + tid] * (e + eo);
+    return e;
+}
+
+template <typename IdxT>
+__global__ void k_drude(Grid g, DrudeBox b, int comp, int P, float* E, const IdxT* idx, const float* tup) {
+    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (tid < b.nb) (void)drude_cell(g, b, comp, P, E, idx, tup, tid);
 }
 
 __global__ void k_save_eold(Grid g, DrudeBox b, const float* E) {
@@ -1694,6 +1703,209 @@ __global__ void k_sheet_pbc(Sheets s, int mode, int src, int n_other) {
     if (u > n_other || pl >= s.np) return;
     if (mode == 0) s.es[sh_off(s, pl, 1, u)] = s.es[sh_off(s, pl, src, u)];
     else s.es[sh_off(s, pl, u, 1)] = s.es[sh_off(s, pl, u, src)];
+}
+
+// ---------------------------------------------------------------------------
+// Periodic slabs (two periodic axes, one axis `ax` with CPML): what follows
+// the bulk update of a phase in one launch, where it had been one launch each
+// for the sheets, the TF/SF planes and the copies of every periodic axis.
+// Each thread owns one cell: it applies the cell's sheet and TF/SF terms in
+// the reference's order and writes the result to the cell and to the cells the
+// periodic copies give it to (H: index 1 -> N-1, f90:5377-5433; E: N-1 -> 1,
+// f90:6672-6741).  A component is copied along the periodic axes normal to
+// it; an element that a copy fills has no thread of its own.  The first
+// blocks cover the whole planes that carry terms, the others the two edge
+// strips of every other plane that only feed copies.  These kernels are bound
+// by launch and memory latency (3-7 us each whatever the size), so their number
+// is what counts: step with k_slab_media, separate launches / this, 75 x 30 x
+// 30 34 / 25 us, 120 x 30 x 30 with 3 poles 50 / 31, 32 x 32 x 1200 with 6 poles
+// and a sheet 104 / 68.
+// ---------------------------------------------------------------------------
+struct SlabFix {
+    int ax, p, q;              // slab axis and the periodic ones (p < q)
+    int n[3];                  // NX, NY, NZ
+    long long st[3];           // strides of i, j, k
+    int n_planes;              // whole planes: TF/SF, then sheets
+    int plane[8];
+    int sheet0;                // index of the first sheet plane in `plane`
+    unsigned plane_blocks;     // blocks of the whole planes
+};
+
+// Cell (s, u, w) along (ax, p, q) of this thread, or false.
+__device__ __forceinline__ bool slab_cell(const SlabFix& f, bool src_low, int& pl, int& s, int& u, int& w) {
+    const int np = f.n[f.p] - 1, nq = f.n[f.q] - 1, ns = f.n[f.ax] - 1;
+    long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    pl = -1;
+    if (blockIdx.x < f.plane_blocks) {
+        const long long per = (long long)np * nq;
+        if (t >= per * f.n_planes) return false;
+        pl = (int)(t / per);
+        t -= pl * per;
+        u = 1 + (int)(t % np);
+        w = 1 + (int)(t / np);
+        s = f.plane[0];
+#pragma unroll
+        for (int k = 1; k < 8; ++k)
+            if (pl == k) s = f.plane[k];
+        return true;
+    }
+    t -= (long long)f.plane_blocks * blockDim.x;
+    const int strip = np + nq - 1;               // the line w = edge, then u = edge without the corner
+    if (t >= (long long)strip * ns) return false;
+    s = 1 + (int)(t / strip);
+    const int r = (int)(t % strip);
+    const int eu = src_low ? 1 : np, ew = src_low ? 1 : nq;
+    if (r < np) {
+        u = 1 + r;
+        w = ew;
+    } else {
+        u = eu;
+        w = 1 + (r - np);
+        if (w >= ew) ++w;                        // skips w = ew
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        if (k < f.n_planes && s == f.plane[k]) return false;   // a whole plane's
+    return true;
+}
+
+__device__ __forceinline__ void slab_store(const SlabFix& f, bool src_low, int c, float* F, long long o, int u, int w,
+                                           float v, bool own) {
+    const int np = f.n[f.p] - 1, nq = f.n[f.q] - 1;
+    const int su = src_low ? 1 : np, sw = src_low ? 1 : nq;
+    const long long du = (src_low ? np - 1 : 1 - np) * f.st[f.p], dw = (src_low ? nq - 1 : 1 - nq) * f.st[f.q];
+    const bool cu = c != f.p && u == su, cw = c != f.q && w == sw;
+    if (own) F[o] = v;
+    if (cu) F[o + du] = v;
+    if (cw) F[o + dw] = v;
+    if (cu && cw) F[o + du + dw] = v;
+}
+
+__global__ void __launch_bounds__(256) k_h_slab_fix(Grid g, SlabFix f, Tfsf t, Sheets sh, float sf, float* Hx, float* Hy,
+                                                    float* Hz, const float* Ex, const float* Ey, const float* Ez,
+                                                    const float* dhx, const float* dhy, const float* dhz,
+                                                    const int* step) {
+    int pl, s, u, w;
+    if (!slab_cell(f, true, pl, s, u, w)) return;
+    const int np = f.n[f.p] - 1, nq = f.n[f.q] - 1;
+    const int i = f.ax == 0 ? s : u, j = f.ax == 1 ? s : (f.ax == 0 ? u : w), k = f.ax == 2 ? s : w;
+    const long long o = off(g, i, j, k);
+    // an element that a copy fills belongs to the copy's source
+    const bool fu = u == np, fw = w == nq;
+    auto filled = [&](int c) { return (c != f.p && fu) || (c != f.q && fw); };
+    float h[3] = {Hx[o], Hy[o], Hz[o]};
+    if (pl >= f.sheet0) {                        // sheets normal to ax (k_h_sheets)
+        const int ps = pl - f.sheet0;
+        if (f.ax == 0 && sh_on(sh, ps, j, k)) {
+            h[1] = h[1] + sf * ((Ex[o + g.plane] - Ex[o] + sh.es[sh_off(sh, ps, j, k)] - sh.es[sh_off(sh, ps, j, k + 1)]) * dhz[k - 1]);
+            h[2] = h[2] + sf * ((Ex[o] - Ex[o + g.PX] + sh.es[sh_off(sh, ps, j + 1, k)] - sh.es[sh_off(sh, ps, j, k)]) * dhy[j - 1]);
+        } else if (f.ax == 1 && sh_on(sh, ps, i, k)) {
+            h[0] = h[0] + sf * (Ey[o] - Ey[o + g.plane] + sh.es[sh_off(sh, ps, i, k + 1)] - sh.es[sh_off(sh, ps, i, k)]) * dhz[k - 1];
+            h[2] = h[2] + sf * ((Ey[o + 1] - Ey[o] - sh.es[sh_off(sh, ps, i + 1, k)] + sh.es[sh_off(sh, ps, i, k)]) * dhx[i - 1]);
+        } else if (f.ax == 2 && sh_on(sh, ps, i, j)) {
+            h[0] = h[0] + sf * (Ez[o + g.PX] - Ez[o] - sh.es[sh_off(sh, ps, i, j + 1)] + sh.es[sh_off(sh, ps, i, j)]) * dhy[j - 1];
+            h[1] = h[1] + sf * ((Ez[o] - Ez[o + 1] + sh.es[sh_off(sh, ps, i + 1, j)] - sh.es[sh_off(sh, ps, i, j)]) * dhx[i - 1]);
+        }
+    } else if (pl >= 0) {                        // TF/SF plane 0 (low) or 1 (high) (h_tfsf_body)
+        const float cf = (float)*step - 1.0f;
+        const float fi = (float)i, fj = (float)j, fk = (float)k;
+        if (f.ax == 0) {
+            const float x = (float)(pl ? t.hi[0] : t.lo[0]);
+            const float a = t.kH[0] * inc_fn(t, t.WE[1], x, fj + 0.5f, fk, cf) * t.wall[pl];
+            const float b = t.kH[0] * inc_fn(t, t.WE[2], x, fj, fk + 0.5f, cf) * t.wall[pl];
+            h[2] = pl ? h[2] - a : h[2] + a;
+            h[1] = pl ? h[1] + b : h[1] - b;
+        } else if (f.ax == 1) {
+            const float y = (float)(pl ? t.hi[1] : t.lo[1]);
+            const float a = t.kH[1] * inc_fn(t, t.WE[0], fi + 0.5f, y, fk, cf) * t.wall[2 + pl];
+            const float b = t.kH[1] * inc_fn(t, t.WE[2], fi, y, fk + 0.5f, cf) * t.wall[2 + pl];
+            h[2] = pl ? h[2] + a : h[2] - a;
+            h[0] = pl ? h[0] - b : h[0] + b;
+        } else {
+            const float z = (float)(pl ? t.hi[2] : t.lo[2]);
+            const float a = t.kH[2] * inc_fn(t, t.WE[0], fi + 0.5f, fj, z, cf) * t.wall[4 + pl];
+            const float b = t.kH[2] * inc_fn(t, t.WE[1], fi, fj + 0.5f, z, cf) * t.wall[4 + pl];
+            h[1] = pl ? h[1] - a : h[1] + a;
+            h[0] = pl ? h[0] + b : h[0] - b;
+        }
+    }
+    if (!filled(0)) slab_store(f, true, 0, Hx, o, u, w, h[0], pl >= 0);
+    if (!filled(1)) slab_store(f, true, 1, Hy, o, u, w, h[1], pl >= 0);
+    if (!filled(2)) slab_store(f, true, 2, Hz, o, u, w, h[2], pl >= 0);
+}
+
+__global__ void __launch_bounds__(256) k_e_slab_fix(Grid g, SlabFix f, Tfsf t, float* Ex, float* Ey, float* Ez,
+                                                    const int* step) {
+    int pl, s, u, w;
+    if (!slab_cell(f, false, pl, s, u, w)) return;
+    const int i = f.ax == 0 ? s : u, j = f.ax == 1 ? s : (f.ax == 0 ? u : w), k = f.ax == 2 ? s : w;
+    const long long o = off(g, i, j, k);
+    const bool fu = u == 1, fw = w == 1;
+    auto filled = [&](int c) { return (c != f.p && fu) || (c != f.q && fw); };
+    float e[3] = {Ex[o], Ey[o], Ez[o]};
+    if (pl >= 0) {                               // TF/SF plane 0 (low) or 1 (high) (k_e_tfsf)
+        const float cf = (float)*step - 0.5f;
+        const float fi = (float)i, fj = (float)j, fk = (float)k;
+        if (f.ax == 0) {
+            const float x = pl ? (float)t.hi[0] + 0.5f : (float)t.lo[0] - 0.5f;
+            const float a = t.kE[0] * inc_fn(t, t.WH[1], x, fj, fk + 0.5f, cf) * t.wall[pl];
+            const float b = t.kE[0] * inc_fn(t, t.WH[2], x, fj + 0.5f, fk, cf) * t.wall[pl];
+            e[2] = pl ? e[2] + a : e[2] - a;
+            e[1] = pl ? e[1] - b : e[1] + b;
+        } else if (f.ax == 1) {
+            const float y = pl ? (float)t.hi[1] + 0.5f : (float)t.lo[1] - 0.5f;
+            const float a = t.kE[1] * inc_fn(t, t.WH[0], fi, y, fk + 0.5f, cf) * t.wall[2 + pl];
+            const float b = t.kE[1] * inc_fn(t, t.WH[2], fi + 0.5f, y, fk, cf) * t.wall[2 + pl];
+            e[2] = pl ? e[2] - a : e[2] + a;
+            e[0] = pl ? e[0] + b : e[0] - b;
+        } else {
+            const float z = pl ? (float)t.hi[2] + 0.5f : (float)t.lo[2] - 0.5f;
+            const float a = t.kE[2] * inc_fn(t, t.WH[0], fi, fj + 0.5f, z, cf) * t.wall[4 + pl];
+            const float b = t.kE[2] * inc_fn(t, t.WH[1], fi + 0.5f, fj, z, cf) * t.wall[4 + pl];
+            e[1] = pl ? e[1] + a : e[1] - a;
+            e[0] = pl ? e[0] - b : e[0] + b;
+        }
+    }
+    if (!filled(0)) slab_store(f, false, 0, Ex, o, u, w, e[0], pl >= 0);
+    if (!filled(1)) slab_store(f, false, 1, Ey, o, u, w, e[1], pl >= 0);
+    if (!filled(2)) slab_store(f, false, 2, Ez, o, u, w, e[2], pl >= 0);
+}
+
+// Between a slab deck's bulk E update and its TF/SF planes: the Drude boxes of
+// the three components (blockIdx.y) with their E_old, which no later term of
+// the step touches there, and (blockIdx.y = 3) the special E of the sheets
+// normal to `ax` with its periodic copies.
+struct DrudeSet {
+    DrudeBox b[3];
+    int P;
+};
+
+template <typename IdxT>
+__global__ void __launch_bounds__(256) k_slab_media(Grid g, SlabFix f, DrudeSet d, Sheets sh, float* Ex, float* Ey,
+                                                    float* Ez, const float* Hx, const float* Hy, const float* Hz,
+                                                    const IdxT* idx, const float* tup, const float* dex,
+                                                    const float* dey, const float* dez, float dt, float ep0) {
+    if (blockIdx.y == 3) {
+        const int per = (sh.P - 2) * (sh.Q - 2);
+        const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+        if (t >= (long long)per * sh.np) return;
+        const int pl = (int)(t / per), r = (int)(t % per);
+        const int p = 2 + r % (sh.P - 2), q = 2 + r / (sh.P - 2);
+        if (!sh_on(sh, pl, p, q)) return;
+        const float v = sheet_es(g, sh, f.ax, pl, p, q, Hx, Hy, Hz, dex, dey, dez, dt, ep0);
+        const int lp = sh.P - 1, lq = sh.Q - 1;
+        sh.es[sh_off(sh, pl, p, q)] = v;
+        if (p == lp) sh.es[sh_off(sh, pl, 1, q)] = v;
+        if (q == lq) sh.es[sh_off(sh, pl, p, 1)] = v;
+        if (p == lp && q == lq) sh.es[sh_off(sh, pl, 1, 1)] = v;
+        return;
+    }
+    const int comp = (int)blockIdx.y;
+    const DrudeBox& b = comp == 0 ? d.b[0] : (comp == 1 ? d.b[1] : d.b[2]);
+    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (tid >= b.nb) return;
+    float* E = comp == 0 ? Ex : (comp == 1 ? Ey : Ez);
+    b.Eold[tid] = drude_cell(g, b, comp, d.P, E, idx, tup, tid);
 }
 
 // ---------------------------------------------------------------------------

@@ -248,10 +248,12 @@ struct Launch {
 // 256^3 142 / 133 / 130; y/z slabs (H and E) at 120^3 37 / 36 / 43, 150^3 49 /
 // 48 / 51, 200^3 84 / 81 / 84; single pass at 40^3 11.5 / 13.6 / 18.9 / 29.2,
 // 120^3 35 / 35 / 30 / 40, 160^3 78 / 63 / 58 / 56, 200^3 167 / 133 / 117 /
-// 108, 256^3 296 / 230 / 201 / 196.
+// 108, 256^3 296 / 230 / 201 / 196; with more than kSpLargeGroups columns left
+// at twelve planes that is the better length (400^3 8 / 10 / 12 planes 625 / 617
+// / 607, 320^3 318 / 321 / 320, 200^3 104 / 112 / 121).
 constexpr int kPlanes = 4;
-constexpr int kSpPlanes = 8;
-constexpr long long kBulkGroups = 4096, kSlabGroups = 2048, kSpGroups = 800;
+constexpr int kSpPlanes = 8, kSpPlanesLarge = 12;
+constexpr long long kBulkGroups = 4096, kSlabGroups = 2048, kSpGroups = 800, kSpLargeGroups = 8192;
 
 // Grids up to kOneLaunchCells update the core box and the slab boxes of a
 // phase in one launch (the single pass with the slabs' H), which saves a launch
@@ -435,6 +437,11 @@ struct aem_sim {
     bool fuse_cpml = false;        // CPML corrections folded into the bulk kernels
     RDiv rdv[3] = {};              // the CPML kernels' divisions by dx, dy, dz
     std::vector<Launch> bulk;      // bulk launches of each phase; [0] is the core when fused
+    // periodic slab decks: terms and copies after the bulk updates in one
+    // launch per phase (k_h_slab_fix, k_e_slab_fix, k_slab_media)
+    bool slab_ok = false;
+    SlabFix sfH{}, sfE{};
+    void slab_setup();
     Launch all_boxes{};            // core and slabs in one launch
     bool one_launch = false;
     HArgs ha{};                    // bulk kernel arguments (fields, tables, CPML state)
@@ -902,7 +909,8 @@ void aem_sim::create(const aem_sim_options* opt) {
     if (sp_ok) {
         sp_box = bulk[0].bs.b[0];
         const long long groups = (long long)cdiv(sp_box.ni, 64) * cdiv(sp_box.nj, kSY * kSpRows) * sp_box.nk;
-        sp_box.kc = planes_set ? planes : (int)std::max(1LL, std::min<long long>(kSpPlanes, groups / kSpGroups));
+        const int most = groups / kSpPlanesLarge >= kSpLargeGroups ? kSpPlanesLarge : kSpPlanes;
+        sp_box.kc = planes_set ? planes : (int)std::max(1LL, std::min<long long>(most, groups / kSpGroups));
         if (!planes_set) sp_box.kc = (int)cdiv(sp_box.nk, cdiv(sp_box.nk, sp_box.kc));   // chunks of equal length
         // (separate launches for the slab-free x tiles, no slab test and fewer
         // registers, and the two x-slab tiles of each row took 5-12% longer at
@@ -927,6 +935,7 @@ void aem_sim::create(const aem_sim_options* opt) {
             }
         }
     }
+    slab_setup();
     for (int a = 0; a < 3; ++a) {
         const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
         ntff_mu = std::max(ntff_mu, v.ff_hi[b] - v.ff_lo[b] + 1);
@@ -941,6 +950,56 @@ void aem_sim::create(const aem_sim_options* opt) {
         kim->create(opt);
         kmax_setup();
     }
+}
+
+// The one-launch form of a periodic slab's terms and copies holds where every
+// cell has one owner: two periodic axes, the CPML folded into the bulk, no
+// ports or ground plane, sheets only across the slab axis and on planes of
+// their own, and Drude boxes clear of the TF/SF planes (their E is then final
+// before those).
+void aem_sim::slab_setup() {
+    const aem_plan_view& v = plan->v;
+    if (!fuse_cpml || v.kmax || v.mirror_type > 0 || v.n_ports > 0 || v.n_spice > 0 ||
+        v.pbc[0] + v.pbc[1] + v.pbc[2] != 2)
+        return;
+    const int ax = !v.pbc[0] ? 0 : (!v.pbc[1] ? 1 : 2);
+    SlabFix f{};
+    f.ax = ax;
+    f.p = ax == 0 ? 1 : 0;
+    f.q = ax == 2 ? 1 : 2;
+    f.n[0] = v.NX; f.n[1] = v.NY; f.n[2] = v.NZ;
+    f.st[0] = 1; f.st[1] = v.PX; f.st[2] = v.plane;
+    const int np = f.n[f.p] - 1, nq = f.n[f.q] - 1, ns = f.n[ax] - 1;
+    if (np < 3 || nq < 3) return;
+    for (int a = 0; a < 3; ++a)
+        if (a != ax && v.n_sheet_planes[a] > 0) return;
+    if (v.n_sheet_planes[ax] > 6) return;
+    SlabFix h = f, e = f;
+    if (v.has_tfsf) {
+        const int lo = v.tf_lo[ax], hi = v.tf_hi[ax];
+        if (lo - 1 < 1 || hi > ns || lo >= hi) return;
+        if (v.tf_lo[f.p] != 1 || v.tf_hi[f.p] != np || v.tf_lo[f.q] != 1 || v.tf_hi[f.q] != nq) return;
+        h.plane[0] = lo - 1; h.plane[1] = hi;
+        e.plane[0] = lo; e.plane[1] = hi;
+        h.n_planes = e.n_planes = 2;
+        if (v.has_drude)
+            for (int c = 0; c < 3; ++c) {
+                const int b0 = v.dbox[c][2 * ax], b1 = v.dbox[c][2 * ax + 1];
+                if (db[c].nb > 0 && ((lo >= b0 && lo <= b1) || (hi >= b0 && hi <= b1))) return;
+            }
+    }
+    h.sheet0 = h.n_planes;
+    for (int q = 0; q < v.n_sheet_planes[ax]; ++q) {
+        const int c = v.sheet_pos[ax][q];
+        for (int k = 0; k < h.n_planes; ++k)
+            if (h.plane[k] == c) return;
+        h.plane[h.n_planes++] = c;
+    }
+    e.sheet0 = e.n_planes;
+    for (SlabFix* x : {&h, &e}) x->plane_blocks = cdiv((long long)np * nq * x->n_planes, 256);
+    sfH = h;
+    sfE = e;
+    slab_ok = true;
 }
 
 // Kernel argument blocks from the current field and psi pointers.  In place,
@@ -1350,8 +1409,17 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
         for (size_t q = 1; q < bulk.size(); ++q) h_bulk(bulk[q]);
     }
     const float dd[3] = {v.dx, v.dy, v.dz};
+    constexpr unsigned kSlabParts = kPartHPre | kPartHPost | kPartEPre | kPartEPost | kPartEOld;
+    const bool slab = slab_ok && !mark && (parts & kSlabParts) == kSlabParts;
+    auto slab_blocks = [](const SlabFix& f) {   // the whole planes, then the strips
+        const long long strip = (long long)(f.n[f.p] - 1) + (f.n[f.q] - 1) - 1;
+        return f.plane_blocks + cdiv(strip * (f.n[f.ax] - 1), 256);
+    };
+    if (slab)
+        k_h_slab_fix<<<slab_blocks(sfH), 256, 0, s>>>(g, sfH, tf, sh[sfH.ax], v.DB * (v.sheet_thickness / dd[sfH.ax]),
+                                                      Hx, Hy, Hz, Ex, Ey, Ez, d_den[3], d_den[4], d_den[5], d_step);
     for (int a = 0; a < 3; ++a)
-        if ((parts & kPartHPre) && sh[a].np > 0) {
+        if ((parts & kPartHPre) && !slab && sh[a].np > 0) {
             const float f = v.DB * (v.sheet_thickness / dd[a]);
             const dim3 gs(cdiv(sh[a].P, 32), cdiv(sh[a].Q, 8));
             k_h_sheets<<<gs, bb, 0, s>>>(g, sh[a], a, Hx, Hy, Hz, Ex, Ey, Ez, d_den[3], d_den[4], d_den[5], f);
@@ -1359,7 +1427,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     // the incident wave's faces, then (infinite ground plane) the mirrored
     // wave's, as the reference orders them (f90:4627-4790, 5950-6111)
     const int ntf = v.mirror_type > 0 ? 2 : 1;
-    if ((parts & kPartHPre) && v.has_tfsf) {
+    if ((parts & kPartHPre) && !slab && v.has_tfsf) {
         const int nx = v.tf_hi[0] - v.tf_lo[0] + 2, ny = v.tf_hi[1] - v.tf_lo[1] + 2, nz = v.tf_hi[2] - v.tf_lo[2] + 2;
         for (int w = 0; w < ntf; ++w) {
             const Tfsf& t = w ? tfm : tf;
@@ -1375,7 +1443,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
         }
     }
     if ((parts & kPartHPort) && v.n_ports > 0 && !sp_ports) k_ports_h<<<1, 256, 0, s>>>(pa);
-    if (parts & kPartHPost) {
+    if ((parts & kPartHPost) && !slab) {
         const long long tx = (long long)(std::max(v.npml[0] - 1, 0) + std::max(v.npml[1] - 1, 0)) * (v.NY - 1) * (v.NZ - 1);
         const long long ty = (long long)(v.NX - 1) * (std::max(v.npml[2] - 1, 0) + std::max(v.npml[3] - 1, 0)) * (v.NZ - 1);
         const long long tz = (long long)(v.NX - 1) * (v.NY - 1) * (std::max(v.npml[4] - 1, 0) + std::max(v.npml[5] - 1, 0));
@@ -1410,15 +1478,30 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     if ((parts & kPartEPre) && des_on)
         k_e_design<<<cdiv(des.nedge, 256), 256, 0, s>>>(g, des, Ex, Ey, Ez, Hx, Hy, Hz, d_den[0], d_den[1], d_den[2],
                                                          rec, rec_on ? 1 : 0, d_step);
+    if (slab) {
+        const Sheets& ss = sh[sfE.ax];
+        const long long nsh = ss.np > 0 ? (long long)(ss.P - 2) * (ss.Q - 2) * ss.np : 0;
+        long long most = nsh;
+        DrudeSet ds{};
+        ds.P = v.n_poles;
+        for (int c = 0; c < 3; ++c) {
+            if (v.has_drude) ds.b[c] = db[c];
+            most = std::max(most, ds.b[c].nb);
+        }
+        if (most > 0)
+            k_slab_media<IdxT><<<dim3(cdiv(most, 256), nsh > 0 ? 4 : 3), 256, 0, s>>>(
+                g, sfE, ds, ss, Ex, Ey, Ez, Hx, Hy, Hz, idx, d_tup, d_den[0], d_den[1], d_den[2], v.dt, aem::kEp0);
+        k_e_slab_fix<<<slab_blocks(sfE), 256, 0, s>>>(g, sfE, tf, Ex, Ey, Ez, d_step);
+    }
     for (int a = 0; a < 3; ++a)
-        if ((parts & kPartEPre) && sh[a].np > 0) {
+        if ((parts & kPartEPre) && !slab && sh[a].np > 0) {
             const dim3 gs(cdiv(sh[a].P, 32), cdiv(sh[a].Q, 8));
             k_e_sheets<<<gs, bb, 0, s>>>(g, sh[a], a, Hx, Hy, Hz, d_den[0], d_den[1], d_den[2], v.dt, aem::kEp0);
         }
-    if ((parts & kPartEPre) && v.has_drude)
+    if ((parts & kPartEPre) && !slab && v.has_drude)
         for (int c = 0; c < 3; ++c)
             if (db[c].nb > 0) k_drude<IdxT><<<cdiv(db[c].nb, 256), 256, 0, s>>>(g, db[c], c, v.n_poles, F[c], idx, d_tup);
-    if ((parts & kPartEPre) && v.has_tfsf) {
+    if ((parts & kPartEPre) && !slab && v.has_tfsf) {
         const int nx = v.tf_hi[0] - v.tf_lo[0] + 2, ny = v.tf_hi[1] - v.tf_lo[1] + 2, nz = v.tf_hi[2] - v.tf_lo[2] + 2;
         for (int w = 0; w < ntf; ++w) {
             const Tfsf& t = w ? tfm : tf;
@@ -1435,7 +1518,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     }
     if ((parts & kPartEPort) && v.n_ports > 0 && !sp_ports) k_ports_e<<<1, 256, 0, s>>>(pa);
     if ((parts & kPartSpiceE) && v.n_spice > 0) k_spice_e<<<1, 64, 0, s>>>(spa);
-    if (parts & kPartEPost) {
+    if ((parts & kPartEPost) && !slab) {
         const long long tx = (long long)(std::max(v.npml[0] - 1, 0) + std::max(v.npml[1] - 1, 0)) * (v.NY - 1) * (v.NZ - 1);
         const long long ty = (long long)(v.NX - 1) * (std::max(v.npml[2] - 1, 0) + std::max(v.npml[3] - 1, 0)) * (v.NZ - 1);
         const long long tz = (long long)(v.NX - 1) * (v.NY - 1) * (std::max(v.npml[4] - 1, 0) + std::max(v.npml[5] - 1, 0));
@@ -1458,7 +1541,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
             if (sh[0].np) k_sheet_pbc<<<dim3(cdiv(v.NY - 1, 256), sh[0].np), 256, 0, s>>>(sh[0], 1, v.NZ - 1, v.NY - 1);
         }
     }
-    if ((parts & kPartEOld) && v.has_drude)
+    if ((parts & kPartEOld) && !slab && v.has_drude)
         for (int c = 0; c < 3; ++c)
             if (db[c].nb > 0) k_save_eold<<<cdiv(db[c].nb, 256), 256, 0, s>>>(g, db[c], F[c]);
 
