@@ -2785,93 +2785,159 @@ __global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
 }
 
 // NTFF retarded-time binning through an LDS histogram (f90:7643-7927 with
-// FP64 accumulation).  One work-group per (angle, accumulator): the step's
-// contributions all fall in a window of bins [n + win[0], n + win[0] +
-// win[1]) fixed by the NTFF box geometry, so the work-group adds them into an
-// FP64 histogram of that window in LDS and then adds the window into its own
-// accumulator row -- one global read-modify-write per bin instead of eight
-// global atomics per face cell.  Index and weight arithmetic per contribution
-// is the reference's FP32, as in k_ntff_bins; only the FP64 summation order
-// differs from the serial reference (agreement at FP32 rounding level).
-constexpr int kHistMax = 4096;   // bins of one window held in LDS (32 KB)
+// FP64 accumulation).  The step's contributions all fall in a window of bins
+// [n + win[0], n + win[0] + win[1]) fixed by the NTFF box geometry.  One
+// work-group per (angle, U or W, face pair): the faces normal to one axis add
+// their two currents, with the same bin and weight, to the accumulators of the
+// other two axes, so it keeps two FP64 histograms of the window in LDS and then
+// adds them to the accumulators (by atomics: two face pairs meet in each).
+// Index and weight arithmetic per contribution is the reference's FP32, as in
+// k_ntff_bins; only the FP64 summation order differs from the serial reference
+// (agreement at FP32 rounding level).
+//
+// Bound by the retarded time's arithmetic and the LDS additions.  So both
+// currents share one bin and weight, the three products of the time come from
+// tables per row and column, indices are 32-bit, and 16 waves with four cells
+// per thread in flight cover the loads.  150^3 with 73 angles: 134 us; one
+// histogram per accumulator with 4 waves had taken 263, 16 waves alone 213,
+// all but the lane orientation and the DPP sums 201.
+constexpr int kHistMax = 4096;   // bins of one window held in LDS (64 KB for two)
+constexpr int kHistThreads = 1024;
+constexpr int kHistCells = 4;    // cells per thread in flight
+constexpr int kHistRow = 1024;   // rows and columns with a table entry
 
-__device__ __forceinline__ void ntff_hist_body(const NtffFaces& f, const NtffBins& bn, const int* win, int kk,
-                                               int arr, const int* step) {
-    __shared__ double h[kHistMax];
-    const int n = *step;
-    const int lo = n + win[2 * kk], len = min(win[2 * kk + 1], kHistMax);
-    for (int t = threadIdx.x; t < len; t += blockDim.x) h[t] = 0.0;
-    __syncthreads();
-    const int comp = arr % 3;
-    const bool isW = arr >= 3;
-    const float* an = bn.ang + 6 * kk;
-    const float s1 = an[2], c1 = an[3], s2 = an[4], c2 = an[5];
-    for (int a = 0; a < 3; ++a) {
-        if (a == comp || f.pbc[a]) continue;
-        const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
-        const int slot = comp == b ? 0 : 1;
-        const int nu = f.hi[b] - f.lo[b] + 1, nv = f.hi[c] - f.lo[c] + 1;
-        // each wave takes 64 consecutive cells of one face side, so at
-        // angles where a row of cells shares one time bin the whole wave
-        // does (below); the loop bound is a multiple of 128 and whole waves
-        // stay converged through it
-        const long long nuv = (long long)nu * nv;
-        const long long ncell = ((nuv + 63) >> 6) << 7;
-        const float K = bn.K[a];
-        for (long long cid = threadIdx.x; cid - (long long)(threadIdx.x & 63) < ncell; cid += blockDim.x) {
-            const int side = (int)((cid >> 6) & 1);
-            const long long uvr = ((cid >> 7) << 6) | (cid & 63);
-            const bool live = uvr < nuv;
-            const long long uv = live ? uvr : 0;
-            const int u = f.lo[b] + (int)(uv % nu), v = f.lo[c] + (int)(uv / nu);
-            const int face = 2 * a + side;
-            const int pos = side ? f.hi[a] : f.lo[a];
-            int i, j, k;
-            if (a == 0) { i = pos; j = u; k = v; }
-            else if (a == 1) { i = u; j = pos; k = v; }
-            else { i = u; j = v; k = pos; }
-            const float tfv = (bn.r_relay - ((float)(i - bn.ic) * bn.dx * s1 * c2 + (float)(j - bn.jc) * bn.dy * s1 * s2 +
-                                             (float)(k - bn.kc) * bn.dz * c1)) / bn.c_dt;
-            const long long fo = (long long)u + (long long)f.fd0[face] * v;
-            const float2 dd = isW ? f.dJ[face][fo] : f.dM[face][fo];
-            const float d = slot ? dd.y : dd.x;
-            const float t = isW ? ((float)n + tfv - 1.0f) : ((float)n + 0.5f + tfv - 1.0f);
-            const int ii = (int)t;
-            const float w = t - (float)ii;
-            int q = ii - lo;
-            if (!live || q < 0 || q + 1 >= len) q = -1;
-            const float clo = (1.0f - w) * K * d, chi = w * K * d;
-            // a wave whose cells all fall in one bin adds its FP64 wave sum
-            // once instead of 64 contending LDS atomics on one address
-            const int q0 = __builtin_amdgcn_readfirstlane(q);
-            if (__all(q == q0)) {
-                if (q0 >= 0) {
-                    double slo = (double)clo, shi = (double)chi;
+// FP64 sum over a wave, in lane 63 (DPP row shifts and broadcasts; no LDS).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {
+    const long long x = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(x & 0xffffffffLL), CTRL, ROWS, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(x >> 32), CTRL, ROWS, 0xf, true);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+__device__ __forceinline__ double wave_sum63(double v) {
+    v += dpp_f64<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v += dpp_f64<0x112, 0xf>(v);
+    v += dpp_f64<0x114, 0xf>(v);
+    v += dpp_f64<0x118, 0xf>(v);
+    v += dpp_f64<0x142, 0xa>(v);   // row_bcast 15 into rows 1 and 3
+    v += dpp_f64<0x143, 0xc>(v);   // row_bcast 31 into rows 2 and 3
+    return v;
+}
+
+// Adds the lanes' contributions to bins q and q + 1 (q < 0: none) of both
+// histograms.  Lanes that share a bin contend for one LDS address: where many
+// do (a row of cells at an angle that gives it one retarded time, or two rows
+// meeting in a wave) their sum is formed across the wave and added once.
+__device__ __forceinline__ void hist_add(double* h, int q, float w0, float w1, float2 d) {
 #pragma unroll
-                    for (int o = 32; o >= 1; o >>= 1) {
-                        slo += __shfl_xor(slo, o);
-                        shi += __shfl_xor(shi, o);
-                    }
-                    if ((threadIdx.x & 63) == 0) {
-                        atomicAdd(&h[q0], slo);
-                        atomicAdd(&h[q0 + 1], shi);
-                    }
-                }
-            } else if (q >= 0) {
-                atomicAdd(&h[q], (double)clo);
-                atomicAdd(&h[q + 1], (double)chi);
-            }
+    for (int round = 0; round < 2; ++round) {
+        const unsigned long long act = __ballot(q >= 0);
+        if (!act) return;
+        const int q0 = __builtin_amdgcn_readlane(q, (int)__builtin_ctzll(act));
+        const bool in = q == q0;
+        if (__popcll(__ballot(in)) < 16) break;
+        const double s0 = wave_sum63(in ? (double)(w0 * d.x) : 0.0), s1 = wave_sum63(in ? (double)(w1 * d.x) : 0.0);
+        const double s2 = wave_sum63(in ? (double)(w0 * d.y) : 0.0), s3 = wave_sum63(in ? (double)(w1 * d.y) : 0.0);
+        if ((threadIdx.x & 63) == 63) {
+            atomicAdd(&h[q0], s0);
+            atomicAdd(&h[q0 + 1], s1);
+            atomicAdd(&h[kHistMax + q0], s2);
+            atomicAdd(&h[kHistMax + q0 + 1], s3);
         }
+        if (in) q = -1;
     }
-    __syncthreads();
-    double* A = (isW ? bn.W[comp] : bn.U[comp]) + (long long)kk * bn.LL;
-    for (int t = threadIdx.x; t < len; t += blockDim.x) {
-        const long long bin = (long long)lo + t;
-        if (bin >= 0 && bin < bn.LL) A[bin] += h[t];
+    if (q >= 0) {
+        atomicAdd(&h[q], (double)(w0 * d.x));
+        atomicAdd(&h[q + 1], (double)(w1 * d.x));
+        atomicAdd(&h[kHistMax + q], (double)(w0 * d.y));
+        atomicAdd(&h[kHistMax + q + 1], (double)(w1 * d.y));
     }
 }
 
-__global__ void __launch_bounds__(256) k_ntff_hist(NtffFaces f, NtffBins bn, const int* win, const int* step) {
+__device__ __forceinline__ void ntff_hist_body(const NtffFaces& f, const NtffBins& bn, const int* win, int kk, int y,
+                                               const int* step) {
+    __shared__ double h[2 * kHistMax];
+    __shared__ float tu[kHistRow], tv[kHistRow];
+    const int a = y % 3;                           // face pair
+    const bool isW = y >= 3;
+    if (f.pbc[a]) return;
+    const int n = *step;
+    const int lo = n + win[2 * kk], len = min(win[2 * kk + 1], kHistMax);
+    const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+    const float* an = bn.ang + 6 * kk;
+    const float s1 = an[2], c1 = an[3], s2 = an[4], c2 = an[5];
+    // product of the retarded time along an axis, in the reference's order
+    auto prod = [&](int ax, int i) {
+        return ax == 0 ? (float)(i - bn.ic) * bn.dx * s1 * c2
+                       : (ax == 1 ? (float)(i - bn.jc) * bn.dy * s1 * s2 : (float)(i - bn.kc) * bn.dz * c1);
+    };
+    const unsigned nu = (unsigned)(f.hi[b] - f.lo[b] + 1), nv = (unsigned)(f.hi[c] - f.lo[c] + 1);
+    for (int t = threadIdx.x; t < len; t += blockDim.x) {
+        h[t] = 0.0;
+        h[kHistMax + t] = 0.0;
+    }
+    for (int t = threadIdx.x; t < min((int)nu, kHistRow); t += blockDim.x) tu[t] = prod(b, f.lo[b] + t);
+    for (int t = threadIdx.x; t < min((int)nv, kHistRow); t += blockDim.x) tv[t] = prod(c, f.lo[c] + t);
+    const bool tables = nu <= (unsigned)kHistRow && nv <= (unsigned)kHistRow;
+    __syncthreads();
+    // Each wave takes 64 consecutive cells of one face side, along the face
+    // axis on which the retarded time changes faster, so that few lanes share
+    // a bin; whole waves stay converged through the loop.
+    auto slope = [&](int ax) { return fabsf(ax == 0 ? bn.dx * s1 * c2 : (ax == 1 ? bn.dy * s1 * s2 : bn.dz * c1)); };
+    const bool along_v = slope(c) > slope(b);
+    const unsigned ni = along_v ? nv : nu;             // cells along the lanes
+    const unsigned nuv = nu * nv, ncell = ((nuv + 63) >> 6) << 7;
+    const bool by_mul = ni > 1 && (unsigned long long)nuv * ni < (1ull << 32);   // uv / ni by a high product
+    const unsigned mul = 0xffffffffu / ni + 1u;
+    const float K = bn.K[a];
+    const float2* D0 = isW ? f.dJ[2 * a] : f.dM[2 * a];
+    const float2* D1 = isW ? f.dJ[2 * a + 1] : f.dM[2 * a + 1];
+    const unsigned fd = (unsigned)f.fd0[2 * a];        // the same for both sides
+    const float p0 = prod(a, f.lo[a]), p1 = prod(a, f.hi[a]);
+    const float nh = isW ? (float)n : (float)n + 0.5f;
+    for (unsigned base = 0; base < ncell; base += kHistCells * blockDim.x) {
+        unsigned u[kHistCells], v[kHistCells];
+        float2 d[kHistCells];
+        bool live[kHistCells];
+#pragma unroll
+        for (int r = 0; r < kHistCells; ++r) {
+            const unsigned cid = base + r * blockDim.x + threadIdx.x;
+            unsigned uv = ((cid >> 7) << 6) | (cid & 63);
+            live[r] = cid < ncell && uv < nuv;
+            uv = live[r] ? uv : 0u;
+            const unsigned qo = by_mul ? __umulhi(uv, mul) : uv / ni, qi = uv - qo * ni;
+            u[r] = along_v ? qo : qi;
+            v[r] = along_v ? qi : qo;
+            const float2* D = ((cid >> 6) & 1) ? D1 : D0;
+            d[r] = D[(size_t)(f.lo[b] + u[r]) + (size_t)fd * (f.lo[c] + v[r])];
+        }
+#pragma unroll
+        for (int r = 0; r < kHistCells; ++r) {
+            const unsigned cid = base + r * blockDim.x + threadIdx.x;
+            const float pa = ((cid >> 6) & 1) ? p1 : p0;
+            const float pu = tables ? tu[u[r]] : prod(b, f.lo[b] + (int)u[r]);
+            const float pv = tables ? tv[v[r]] : prod(c, f.lo[c] + (int)v[r]);
+            const float tfv = (bn.r_relay - (a == 2 ? pu + pv + pa : pa + pu + pv)) / bn.c_dt;
+            const float t = nh + tfv - 1.0f;
+            const int ii = (int)t;
+            const float w = t - (float)ii;
+            int q = ii - lo;
+            if (!live[r] || q < 0 || q + 1 >= len) q = -1;
+            hist_add(h, q, (1.0f - w) * K, w * K, d[r]);
+        }
+    }
+    __syncthreads();
+    double* A = (isW ? bn.W[b] : bn.U[b]) + (long long)kk * bn.LL;
+    double* B = (isW ? bn.W[c] : bn.U[c]) + (long long)kk * bn.LL;
+    for (int t = threadIdx.x; t < len; t += blockDim.x) {
+        const long long bin = (long long)lo + t;
+        if (bin < 0 || bin >= bn.LL) continue;
+        if (h[t] != 0.0) atomicAdd(&A[bin], h[t]);
+        if (h[kHistMax + t] != 0.0) atomicAdd(&B[bin], h[kHistMax + t]);
+    }
+}
+
+__global__ void __launch_bounds__(kHistThreads) k_ntff_hist(NtffFaces f, NtffBins bn, const int* win, const int* step) {
     ntff_hist_body(f, bn, win, blockIdx.x, blockIdx.y, step);
 }
 
@@ -2893,8 +2959,8 @@ __global__ void k_ntff_currents_batch(const NtffArgs* __restrict__ args) {
     ntff_currents_body(a.g, a.f, blockIdx.z % 6, a.Ex, a.Ey, a.Ez, a.Hx, a.Hy, a.Hz);
 }
 
-// grid (max angles, 6, members)
-__global__ void __launch_bounds__(256) k_ntff_hist_batch(const NtffArgs* __restrict__ args) {
+// grid (max angles, 6 = (U, W) x face pairs, members)
+__global__ void __launch_bounds__(kHistThreads) k_ntff_hist_batch(const NtffArgs* __restrict__ args) {
     const NtffArgs& a = args[blockIdx.z];
     if ((int)blockIdx.x >= a.bn.n_angles) return;
     ntff_hist_body(a.f, a.bn, a.win, blockIdx.x, blockIdx.y, a.fstep);

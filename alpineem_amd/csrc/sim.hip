@@ -1589,7 +1589,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
             else if (win_max > 0)
                 k_ntff_exact<<<dim3(cdiv(win_max, 256), 6, v.n_angles), 256, 0, sb>>>(nf, nb, nx_acc, fstep);
         } else if (ntff_mode == AEM_NTFF_HISTOGRAM) {
-            k_ntff_hist<<<dim3(v.n_angles, 6), 256, 0, sb>>>(nf, nb, nx_acc.win, fstep);
+            k_ntff_hist<<<dim3(v.n_angles, 6), kHistThreads, 0, sb>>>(nf, nb, nx_acc.win, fstep);
         } else {
             k_ntff_bins<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * v.n_angles), bb, 0, sb>>>(nf, nb, fstep);
         }
@@ -2532,7 +2532,7 @@ struct aem_batch {
             if (beside) beside->before_currents(s);
             k_ntff_currents_batch<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * n_ntff), bb, 0, s>>>(d_nargs[slot]);
             const hipStream_t sb = beside ? beside->after_currents(s) : s;
-            if (n_hist) k_ntff_hist_batch<<<dim3(max_angles, 6, n_hist), 256, 0, sb>>>(d_hist_args[slot]);
+            if (n_hist) k_ntff_hist_batch<<<dim3(max_angles, 6, n_hist), kHistThreads, 0, sb>>>(d_hist_args[slot]);
             if (n_list)
                 k_ntff_list_batch<<<dim3(max_list_blocks, n_list), 64 * kListWavesMany, 0, sb>>>(d_list_args[slot]);
             if (beside) beside->after_binning();
