@@ -160,6 +160,10 @@ __device__ __forceinline__ float ldo_once(const float* p, OffT ob) {
     return __builtin_nontemporal_load(reinterpret_cast<const float*>(reinterpret_cast<const char*>(p) + ob));
 }
 template <class OffT>
+__device__ __forceinline__ void sto(float v, float* p, OffT ob) {
+    *reinterpret_cast<float*>(reinterpret_cast<char*>(p) + ob) = v;
+}
+template <class OffT>
 __device__ __forceinline__ void sto_once(float v, float* p, OffT ob) {
     __builtin_nontemporal_store(v, reinterpret_cast<float*>(reinterpret_cast<char*>(p) + ob));
 }
@@ -3528,6 +3532,47 @@ __device__ __forceinline__ int term_stencil(int A, int q, int d[4][3]) {
     }
 }
 
+// The increments of face F that reach the cell (x0, x1, x2), in term-then-offset
+// order.  F is a template argument, so the stencils unroll to constants (tables
+// in scratch had the gather take 35 us at 128^3, now 17).
+template <int F>
+__device__ __forceinline__ void gather_face(const Objective& ob, const float* __restrict__ D, int x0, int x1, int x2,
+                                            float acc[6], bool hit[6]) {
+    constexpr int A = F / 2, b = A == 0 ? 1 : 0, c = A == 2 ? 1 : 2;
+    if (ob.pbc[A]) return;
+    const int x[3] = {x0, x1, x2};
+    const int pf = (F & 1) ? ob.hi[A] : ob.lo[A];
+    // a face reaches only the two planes pf, pf+1 and lo..hi+1 across
+    if ((x[A] != pf && x[A] != pf + 1) || x[b] < ob.lo[b] || x[b] > ob.hi[b] + 1 || x[c] < ob.lo[c] ||
+        x[c] > ob.hi[c] + 1)
+        return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        int d[4][3];
+        const int code = term_stencil(A, q, d);
+        const int comp = code / 10, n = code % 10;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            if (r >= n) continue;
+            const int y[3] = {x[0] - d[r][0], x[1] - d[r][1], x[2] - d[r][2]};
+            if (y[A] != pf || y[b] < ob.lo[b] || y[b] > ob.hi[b] || y[c] < ob.lo[c] || y[c] > ob.hi[c]) continue;
+            const float dj = D[(((long long)F * 4 + q) * ob.mv + (y[c] - ob.lo[c])) * ob.mu + (y[b] - ob.lo[b])];
+            acc[comp] = acc[comp] + dj;
+            hit[comp] = true;
+        }
+    }
+}
+
+// Is the cell on shell S ({lo, lo+1} or {hi, hi+1} of axis S / 2)?
+template <int S>
+__device__ __forceinline__ bool on_shell(const Objective& ob, int x0, int x1, int x2) {
+    constexpr int A = S / 2, b = A == 0 ? 1 : 0, c = A == 2 ? 1 : 2;
+    const int x[3] = {x0, x1, x2};
+    const int p = (S & 1) ? ob.hi[A] : ob.lo[A];
+    return !ob.pbc[A] && (x[A] == p || x[A] == p + 1) && x[b] >= ob.lo[b] && x[b] <= ob.hi[b] + 1 && x[c] >= ob.lo[c] &&
+           x[c] <= ob.hi[c] + 1;
+}
+
 // One thread per cell of the shells {lo, lo+1} and {hi, hi+1} of each axis
 // of the far-field box (tangentially lo..hi+1), each cell taken by the first
 // shell holding it; grid z = shell * 2 + layer.
@@ -3538,51 +3583,31 @@ __global__ void __launch_bounds__(256) k_adj_source_gather(Grid g, Objective ob,
                                                            float* mEz, const IdxT* idx, const float* tup) {
     const int sh = (int)blockIdx.z >> 1, layer = (int)blockIdx.z & 1;
     const int A = sh / 2;
-    if (ob.pbc[A]) return;
-    const int b = A == 0 ? 1 : 0, c = A == 2 ? 1 : 2;
     const int uu = blockIdx.x * 32 + (threadIdx.x & 31), vv = blockIdx.y * 8 + (threadIdx.x >> 5);
-    if (uu > ob.hi[b] - ob.lo[b] + 1 || vv > ob.hi[c] - ob.lo[c] + 1) return;
-    int x[3];
-    x[A] = ((sh & 1) ? ob.hi[A] : ob.lo[A]) + layer;
-    x[b] = ob.lo[b] + uu;
-    x[c] = ob.lo[c] + vv;
-    // taken by an earlier shell?
-    for (int s2 = 0; s2 < sh; ++s2) {
-        const int A2 = s2 / 2;
-        if (ob.pbc[A2]) continue;
-        const int p2 = (s2 & 1) ? ob.hi[A2] : ob.lo[A2];
-        bool in = x[A2] == p2 || x[A2] == p2 + 1;
-        for (int a = 0; a < 3; ++a)
-            if (a != A2 && (x[a] < ob.lo[a] || x[a] > ob.hi[a] + 1)) in = false;
-        if (in) return;
+    const int pA = ((sh & 1) ? (A == 0 ? ob.hi[0] : (A == 1 ? ob.hi[1] : ob.hi[2]))
+                             : (A == 0 ? ob.lo[0] : (A == 1 ? ob.lo[1] : ob.lo[2]))) + layer;
+    const int x0 = A == 0 ? pA : ob.lo[0] + uu;
+    const int x1 = A == 1 ? pA : ob.lo[1] + (A == 0 ? uu : vv);
+    const int x2 = A == 2 ? pA : ob.lo[2] + vv;
+    const bool on[6] = {on_shell<0>(ob, x0, x1, x2), on_shell<1>(ob, x0, x1, x2), on_shell<2>(ob, x0, x1, x2),
+                        on_shell<3>(ob, x0, x1, x2), on_shell<4>(ob, x0, x1, x2), on_shell<5>(ob, x0, x1, x2)};
+    // on its own shell and on no earlier one
+    bool mine = false;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+        if (q < sh && on[q]) return;
+        if (q == sh) mine = on[q];
     }
-    const long long o = off(g, x[0], x[1], x[2]);
+    if (!mine) return;
+    const long long o = off(g, x0, x1, x2);
     float acc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     bool hit[6] = {false, false, false, false, false, false};
-    for (int f = 0; f < 6; ++f) {
-        const int Af = f / 2;
-        if (ob.pbc[Af]) continue;
-        const int bf = Af == 0 ? 1 : 0, cf = Af == 2 ? 1 : 2;
-        const int pf = (f & 1) ? ob.hi[Af] : ob.lo[Af];
-        // a face reaches only the two planes pf, pf+1 and lo..hi+1 across
-        if ((x[Af] != pf && x[Af] != pf + 1) || x[bf] < ob.lo[bf] || x[bf] > ob.hi[bf] + 1 || x[cf] < ob.lo[cf] ||
-            x[cf] > ob.hi[cf] + 1)
-            continue;
-        for (int q = 0; q < 4; ++q) {
-            int d[4][3];
-            const int code = term_stencil(Af, q, d);
-            const int comp = code / 10, n = code % 10;
-            for (int r = 0; r < n; ++r) {
-                const int y0 = x[0] - d[r][0], y1 = x[1] - d[r][1], y2 = x[2] - d[r][2];
-                const int y[3] = {y0, y1, y2};
-                if (y[Af] != pf || y[bf] < ob.lo[bf] || y[bf] > ob.hi[bf] || y[cf] < ob.lo[cf] || y[cf] > ob.hi[cf])
-                    continue;
-                const float dj = D[(((long long)f * 4 + q) * ob.mv + (y[cf] - ob.lo[cf])) * ob.mu + (y[bf] - ob.lo[bf])];
-                acc[comp] = acc[comp] + dj;
-                hit[comp] = true;
-            }
-        }
-    }
+    gather_face<0>(ob, D, x0, x1, x2, acc, hit);
+    gather_face<1>(ob, D, x0, x1, x2, acc, hit);
+    gather_face<2>(ob, D, x0, x1, x2, acc, hit);
+    gather_face<3>(ob, D, x0, x1, x2, acc, hit);
+    gather_face<4>(ob, D, x0, x1, x2, acc, hit);
+    gather_face<5>(ob, D, x0, x1, x2, acc, hit);
 #pragma unroll
     for (int comp = 0; comp < 6; ++comp) {
         if (!hit[comp]) continue;
@@ -3671,7 +3696,7 @@ __device__ __forceinline__ bool e_psi(const Grid& g, const Cpml& p, int A, int i
     const int side = slab_e(x[A], N[A], p.n[2 * A], p.n[2 * A + 1], q, t);
     if (side < 0) return false;
     f = 2 * A + side;
-    const long long ntf = p.n[f] - 1;
+    const long long ntf = (side ? p.n[2 * A + 1] : p.n[2 * A]) - 1;
     if (A == 0) po = t + ntf * ((long long)(j - 1) + (long long)g.NY * (k - 1));
     else if (A == 1) po = (long long)(i - 1) + (long long)g.PX * (t + ntf * (k - 1));
     else po = (long long)(i - 1) + (long long)g.PX * ((long long)(j - 1) + (long long)g.NY * t);
@@ -3686,7 +3711,7 @@ __device__ __forceinline__ bool h_psi(const Grid& g, const Cpml& p, int A, int i
     const int side = slab_h(x[A], N[A], p.n[2 * A], p.n[2 * A + 1], q);
     if (side < 0) return false;
     f = 2 * A + side;
-    const long long ntf = p.n[f] - 1;
+    const long long ntf = (side ? p.n[2 * A + 1] : p.n[2 * A]) - 1;
     if (A == 0) po = (q - 1) + ntf * ((long long)(j - 1) + (long long)g.NY * (k - 1));
     else if (A == 1) po = (long long)(i - 1) + (long long)g.PX * ((q - 1) + ntf * (k - 1));
     else po = (long long)(i - 1) + (long long)g.PX * ((long long)(j - 1) + (long long)g.NY * (q - 1));
@@ -3737,17 +3762,19 @@ __device__ __forceinline__ void cnu_e_pair(const Grid& g, const Cpml& p, const C
             cn[0][h] = cn[1][h] = 0.0f;
             continue;
         }
-        const int f = 2 * A + side;
-        const long long ntf = p.n[f] - 1;
+        // (selects, not an index: the face differs between the lanes of an x row)
+        const long long ntf = (side ? p.n[2 * A + 1] : p.n[2 * A]) - 1;
         long long po;
         if (A == 0) po = t + ntf * ((long long)(j - 1) + (long long)g.NY * (k - 1));
         else if (A == 1) po = (long long)(i - 1) + (long long)g.PX * (t + ntf * (k - 1));
         else po = (long long)(i - 1) + (long long)g.PX * ((long long)(j - 1) + (long long)g.NY * t);
-        const float cc = p.c[f][q - 1];
+        const float cc = (side ? p.c[2 * A + 1] : p.c[2 * A])[q - 1];
+        const float nu0 = (side ? lp.psi[2 * A + 1][0] : lp.psi[2 * A][0])[po];
+        const float nu1 = (side ? lp.psi[2 * A + 1][1] : lp.psi[2 * A][1])[po];
         int xx[3] = {i, j, k};
         xx[A] += h;
-        cn[0][h] = e_slot_ok(A, 0, xx[0], xx[1], xx[2]) ? cc * lp.psi[f][0][po] : 0.0f;
-        cn[1][h] = e_slot_ok(A, 1, xx[0], xx[1], xx[2]) ? cc * lp.psi[f][1][po] : 0.0f;
+        cn[0][h] = e_slot_ok(A, 0, xx[0], xx[1], xx[2]) ? cc * nu0 : 0.0f;
+        cn[1][h] = e_slot_ok(A, 1, xx[0], xx[1], xx[2]) ? cc * nu1 : 0.0f;
     }
 }
 
@@ -3767,22 +3794,27 @@ __device__ __forceinline__ void cnu_h_pair(const Grid& g, const Cpml& p, const C
             cn[0][h] = cn[1][h] = 0.0f;
             continue;
         }
-        const int f = 2 * A + side;
-        const long long ntf = p.n[f] - 1;
+        // (selects, not an index: the face differs between the lanes of an x row)
+        const long long ntf = (side ? p.n[2 * A + 1] : p.n[2 * A]) - 1;
         long long po;
         if (A == 0) po = (q - 1) + ntf * ((long long)(j - 1) + (long long)g.NY * (k - 1));
         else if (A == 1) po = (long long)(i - 1) + (long long)g.PX * ((q - 1) + ntf * (k - 1));
         else po = (long long)(i - 1) + (long long)g.PX * ((long long)(j - 1) + (long long)g.NY * (q - 1));
-        const float cc = p.c[f][q - 1];
-        cn[0][h] = cc * lp.psi[f][0][po];
-        cn[1][h] = cc * lp.psi[f][1][po];
+        const float cc = (side ? p.c[2 * A + 1] : p.c[2 * A])[q - 1];
+        cn[0][h] = cc * (side ? lp.psi[2 * A + 1][0] : lp.psi[2 * A][0])[po];
+        cn[1][h] = cc * (side ? lp.psi[2 * A + 1][1] : lp.psi[2 * A][1])[po];
     }
 }
 
-// Within one cell of a CPML slab (either field's layers)?
-__device__ __forceinline__ bool near_slab(const Grid& g, const Cpml& p, int i, int j, int k) {
-    return i <= p.n[0] + 1 || i >= g.NX - p.n[1] - 1 || j <= p.n[2] + 1 || j >= g.NY - p.n[3] - 1 ||
-           k <= p.n[4] + 1 || k >= g.NZ - p.n[5] - 1;
+// Within one cell of a CPML slab (either field's layers) of each axis?  A wave
+// is one row, so y and z are one value per wave and their slab work a scalar
+// branch; only the lanes of the x slabs diverge.
+struct Near {
+    bool x, y, z;
+};
+__device__ __forceinline__ Near near_axes(const Grid& g, const Cpml& p, int i, int j, int k) {
+    return Near{i <= p.n[0] + 1 || i >= g.NX - p.n[1] - 1, j <= p.n[2] + 1 || j >= g.NY - p.n[3] - 1,
+                k <= p.n[4] + 1 || k >= g.NZ - p.n[5] - 1};
 }
 
 // The adjoint state keeps mu_c = gb_c lambda_E_c beside lambda_E (0 on the
@@ -3790,122 +3822,178 @@ __device__ __forceinline__ bool near_slab(const Grid& g, const Cpml& p, int i, i
 // lambda_E, k_adj_source_gather adds gb times its own increments, and k_adj_mu
 // rebuilds it after a host write.  The H gather then needs no tuple lookups.
 
+// Both transposed bulk kernels wait on loads, not on bandwidth (about half the
+// rate of the forward updates); what counts is the length of a thread's chain
+// of dependent loads.  128^3, H / E gather: 47 / 52 us with every axis' slab
+// terms behind one test and face arrays indexed per lane (a pointer load from
+// the argument block before each), 32 / 43 with a test per axis, pointers by
+// select, 32-bit offsets and no tile for the outermost column.
+
 // Transposed E phase, gathered per H cell (one thread per cell of
 // [1, N-1]^3, block 64 x 4):
 //   lambda_H += S^T mu                                 (bulk E update)
 //             + D^T (c nu_E) / d                        (E-phase CPML)
 // then nu_H <- b nu_H + DB lambda_H on the H-phase psi cells.
-__global__ void __launch_bounds__(256) k_adj_h(Grid g, float* lHx, float* lHy, float* lHz, const float* mEx,
-                                               const float* mEy, const float* mEz, const float* dex,
-                                               const float* dey, const float* dez, Cpml pe, Cpml lpe, Cpml ph,
-                                               Cpml lph, float DB, float dx, float dy, float dz) {
+template <typename OffT>
+__global__ void __launch_bounds__(256) k_adj_h(Grid g, float* __restrict__ lHx, float* __restrict__ lHy,
+                                               float* __restrict__ lHz, const float* __restrict__ mEx,
+                                               const float* __restrict__ mEy, const float* __restrict__ mEz,
+                                               const float* __restrict__ dex, const float* __restrict__ dey,
+                                               const float* __restrict__ dez, Cpml pe, Cpml lpe, Cpml ph, Cpml lph,
+                                               float DB, float dx, float dy, float dz) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
+    const int j = __builtin_amdgcn_readfirstlane(blockIdx.y * blockDim.y + threadIdx.y + 1);   // one row per wave
     const int k = blockIdx.z + 1;
     if (i > g.NX - 1 || j > g.NY - 1) return;
-    const long long o = off(g, i, j, k), X = g.PX, P = g.plane;
-    const float mx = mEx[o], mx_j = mEx[o + X], mx_k = mEx[o + P];
-    const float my = mEy[o], my_i = mEy[o + 1], my_k = mEy[o + P];
-    const float mz = mEz[o], mz_i = mEz[o + 1], mz_j = mEz[o + X];
+    const OffT o = (OffT)off(g, i, j, k) * 4u, X = (OffT)g.PX * 4u, P = (OffT)g.plane * 4u;
+    const float mx = ldo(mEx, o), mx_j = ldo(mEx, o + X), mx_k = ldo(mEx, o + P);
+    const float my = ldo(mEy, o), my_i = ldo(mEy, o + 4u), my_k = ldo(mEy, o + P);
+    const float mz = ldo(mEz, o), mz_i = ldo(mEz, o + 4u), mz_j = ldo(mEz, o + X);
     const float dx_i = dex[i - 1], dy_j = dey[j - 1], dz_k = dez[k - 1];
     const float dx_i1 = i + 1 <= g.NX - 1 ? dex[i] : 0.0f, dy_j1 = j + 1 <= g.NY - 1 ? dey[j] : 0.0f,
                 dz_k1 = k + 1 <= g.NZ - 1 ? dez[k] : 0.0f;
-    float hx = lHx[o] + (my * dz_k - my_k * dz_k1 + mz_j * dy_j1 - mz * dy_j);
-    float hy = lHy[o] + (mx_k * dz_k1 - mx * dz_k + mz * dx_i - mz_i * dx_i1);
-    float hz = lHz[o] + (mx * dy_j - mx_j * dy_j1 + my_i * dx_i1 - my * dx_i);
-    if (near_slab(g, pe, i, j, k)) {
-        float cx[2][2], cy[2][2], cz[2][2];   // [slot][cell, +1]: x (Eyx, Ezx), y (Exy, Ezy), z (Exz, Eyz)
-        cnu_e_pair(g, pe, lpe, 0, i, j, k, cx);
-        cnu_e_pair(g, pe, lpe, 1, i, j, k, cy);
-        cnu_e_pair(g, pe, lpe, 2, i, j, k, cz);
-        hx += (cy[1][1] - cy[1][0]) / dy + (cz[1][0] - cz[1][1]) / dz;
-        hy += (cx[1][0] - cx[1][1]) / dx + (cz[0][1] - cz[0][0]) / dz;
-        hz += (cx[0][1] - cx[0][0]) / dx + (cy[0][0] - cy[0][1]) / dy;
+    float hx = ldo(lHx, o) + (my * dz_k - my_k * dz_k1 + mz_j * dy_j1 - mz * dy_j);
+    float hy = ldo(lHy, o) + (mx_k * dz_k1 - mx * dz_k + mz * dx_i - mz_i * dx_i1);
+    float hz = ldo(lHz, o) + (mx * dy_j - mx_j * dy_j1 + my_i * dx_i1 - my * dx_i);
+    const Near nr = near_axes(g, pe, i, j, k);
+    if (nr.x || nr.y || nr.z) {
+        // differences of c nu over d along each axis, 0 away from its slabs
+        float x0 = 0.f, x1 = 0.f, y0 = 0.f, y1 = 0.f, z0 = 0.f, z1 = 0.f;
+        float cn[2][2];   // [slot][cell, +1]: x (Eyx, Ezx), y (Exy, Ezy), z (Exz, Eyz)
+        if (nr.x) {
+            cnu_e_pair(g, pe, lpe, 0, i, j, k, cn);
+            x0 = (cn[0][1] - cn[0][0]) / dx;
+            x1 = (cn[1][0] - cn[1][1]) / dx;
+        }
+        if (nr.y) {
+            cnu_e_pair(g, pe, lpe, 1, i, j, k, cn);
+            y0 = (cn[0][0] - cn[0][1]) / dy;
+            y1 = (cn[1][1] - cn[1][0]) / dy;
+        }
+        if (nr.z) {
+            cnu_e_pair(g, pe, lpe, 2, i, j, k, cn);
+            z0 = (cn[0][1] - cn[0][0]) / dz;
+            z1 = (cn[1][0] - cn[1][1]) / dz;
+        }
+        hx += y1 + z1;
+        hy += x1 + z0;
+        hz += x0 + y0;
 #pragma unroll
         for (int A = 0; A < 3; ++A) {
+            if (!(A == 0 ? nr.x : (A == 1 ? nr.y : nr.z))) continue;
             int f, q;
             long long po;
             if (!h_psi(g, ph, A, i, j, k, f, q, po)) continue;
-            const float b = ph.b[f][q - 1];
+            const float b = (f & 1 ? ph.b[2 * A + 1] : ph.b[2 * A])[q - 1];
 #pragma unroll
             for (int sl = 0; sl < 2; ++sl) {
                 const int c = h_slot_comp(A, sl);
-                float* nu = lph.psi[f][sl];
+                float* nu = f & 1 ? lph.psi[2 * A + 1][sl] : lph.psi[2 * A][sl];
                 nu[po] = b * nu[po] + DB * (c == 0 ? hx : (c == 1 ? hy : hz));
             }
         }
     }
-    lHx[o] = hx;
-    lHy[o] = hy;
-    lHz[o] = hz;
+    sto(hx, lHx, o);
+    sto(hy, lHy, o);
+    sto(hz, lHz, o);
 }
 
 // Transposed H phase, gathered per E cell (one thread per cell of
-// [1, NX] x [1, NY] x [1, NZ], block 64 x 4) on the updated components:
+// [1, NX-1] x [1, NY] x [1, NZ], block 64 x 4) on the updated components:
 //   lambda_E <- ga lambda_E + DB C^T lambda_H + D^T (c nu_H) / d,
 // 0 on the fixed outer tangential components, and mu = gb lambda_E; then
 // nu_E <- b nu_E + mu on the E-phase psi cells.  Every lambda_H an updated
 // component reads lies in [1, N-1]^3; the i-1 / j-1 / k-1 offsets are
 // clamped so the other cells' loads stay in bounds.
-template <typename IdxT>
-__global__ void __launch_bounds__(256) k_adj_e(Grid g, float* lEx, float* lEy, float* lEz, float* mEx, float* mEy,
-                                               float* mEz, const float* lHx, const float* lHy, const float* lHz,
-                                               const IdxT* idx, const float* tup, const float* dhx, const float* dhy,
-                                               const float* dhz, Cpml pe, Cpml lpe, Cpml ph, Cpml lph, float DB,
-                                               float dx, float dy, float dz) {
+template <typename IdxT, typename OffT>
+__global__ void __launch_bounds__(256) k_adj_e(Grid g, float* __restrict__ lEx, float* __restrict__ lEy,
+                                               float* __restrict__ lEz, float* __restrict__ mEx,
+                                               float* __restrict__ mEy, float* __restrict__ mEz,
+                                               const float* __restrict__ lHx, const float* __restrict__ lHy,
+                                               const float* __restrict__ lHz, const IdxT* __restrict__ idx,
+                                               const float* __restrict__ tup, const float* __restrict__ dhx,
+                                               const float* __restrict__ dhy, const float* __restrict__ dhz, Cpml pe,
+                                               Cpml lpe, Cpml ph, Cpml lph, float DB, float dx, float dy, float dz,
+                                               int* step) {
+    // (the last kernel of the backward step; the others that read its counter have run)
+    if (blockIdx.x + blockIdx.y + blockIdx.z + threadIdx.x + threadIdx.y == 0) *step = *step - 1;
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
+    const int j = __builtin_amdgcn_readfirstlane(blockIdx.y * blockDim.y + threadIdx.y + 1);   // one row per wave
     const int k = blockIdx.z + 1;
-    if (i > g.NX || j > g.NY) return;
-    const long long o = off(g, i, j, k);
+    if (i > g.NX - 1 || j > g.NY) return;
+    const OffT o = (OffT)off(g, i, j, k) * 4u;
     const bool in = i <= g.NX - 1 && j <= g.NY - 1 && k <= g.NZ - 1;
     const bool ux = in && j >= 2 && k >= 2, uy = in && i >= 2 && k >= 2, uz = in && i >= 2 && j >= 2;
     float ex = 0.0f, ey = 0.0f, ez = 0.0f, mx = 0.0f, my = 0.0f, mz = 0.0f;
     int t = 0;
     if (ux || uy || uz) {
-        const long long xm = i >= 2 ? 1 : 0, ym = j >= 2 ? g.PX : 0, zm = k >= 2 ? g.plane : 0;
-        const float hx = lHx[o], hy = lHy[o], hz = lHz[o];
-        const float hx_ym = lHx[o - ym], hx_km = lHx[o - zm], hy_xm = lHy[o - xm], hy_km = lHy[o - zm];
-        const float hz_xm = lHz[o - xm], hz_ym = lHz[o - ym];
+        const OffT xm = i >= 2 ? 4u : 0u, ym = j >= 2 ? (OffT)g.PX * 4u : (OffT)0, zm = k >= 2 ? (OffT)g.plane * 4u : (OffT)0;
+        t = (int)ldo(idx, o / 4u * (OffT)sizeof(IdxT)) * 6;
+        const float hx = ldo(lHx, o), hy = ldo(lHy, o), hz = ldo(lHz, o);
+        const float hx_ym = ldo(lHx, o - ym), hx_km = ldo(lHx, o - zm), hy_xm = ldo(lHy, o - xm), hy_km = ldo(lHy, o - zm);
+        const float hz_xm = ldo(lHz, o - xm), hz_ym = ldo(lHz, o - ym);
+        const float ex0 = ldo(lEx, o), ey0 = ldo(lEy, o), ez0 = ldo(lEz, o);
         const float dh_x = in ? dhx[i - 1] : 0.0f, dh_y = in ? dhy[j - 1] : 0.0f, dh_z = in ? dhz[k - 1] : 0.0f;
         const float dh_xm = i >= 2 ? dhx[i - 2] : 0.0f, dh_ym = j >= 2 ? dhy[j - 2] : 0.0f,
                     dh_zm = k >= 2 ? dhz[k - 2] : 0.0f;
-        t = (int)idx[o] * 6;
-        if (ux) ex = tup[t] * lEx[o] + DB * (hy * dh_z - hy_km * dh_zm + hz_ym * dh_ym - hz * dh_y);
-        if (uy) ey = tup[t + 2] * lEy[o] + DB * (hx_km * dh_zm - hx * dh_z + hz * dh_x - hz_xm * dh_xm);
-        if (uz) ez = tup[t + 4] * lEz[o] + DB * (hx * dh_y - hx_ym * dh_ym + hy_xm * dh_xm - hy * dh_x);
+        if (ux) ex = tup[t] * ex0 + DB * (hy * dh_z - hy_km * dh_zm + hz_ym * dh_ym - hz * dh_y);
+        if (uy) ey = tup[t + 2] * ey0 + DB * (hx_km * dh_zm - hx * dh_z + hz * dh_x - hz_xm * dh_xm);
+        if (uz) ez = tup[t + 4] * ez0 + DB * (hx * dh_y - hx_ym * dh_ym + hy_xm * dh_xm - hy * dh_x);
     }
-    const bool ns = near_slab(g, pe, i, j, k);
+    const Near nr = near_axes(g, pe, i, j, k);
+    const bool ns = nr.x || nr.y || nr.z;
     if (ns && (ux || uy || uz)) {
-        float cx[2][2], cy[2][2], cz[2][2];   // [slot][cell, -1]: x (Hyx, Hzx), y (Hxy, Hzy), z (Hxz, Hyz)
-        cnu_h_pair(g, ph, lph, 0, i, j, k, cx);
-        cnu_h_pair(g, ph, lph, 1, i, j, k, cy);
-        cnu_h_pair(g, ph, lph, 2, i, j, k, cz);
-        if (ux) ex += (cz[1][0] - cz[1][1]) / dz + (cy[1][1] - cy[1][0]) / dy;
-        if (uy) ey += (cz[0][1] - cz[0][0]) / dz + (cx[1][0] - cx[1][1]) / dx;
-        if (uz) ez += (cx[0][1] - cx[0][0]) / dx + (cy[0][0] - cy[0][1]) / dy;
+        // differences of c nu over d along each axis, 0 away from its slabs
+        float x0 = 0.f, x1 = 0.f, y0 = 0.f, y1 = 0.f, z0 = 0.f, z1 = 0.f;
+        float cn[2][2];   // [slot][cell, -1]: x (Hyx, Hzx), y (Hxy, Hzy), z (Hxz, Hyz)
+        if (nr.x) {
+            cnu_h_pair(g, ph, lph, 0, i, j, k, cn);
+            x0 = (cn[0][1] - cn[0][0]) / dx;
+            x1 = (cn[1][0] - cn[1][1]) / dx;
+        }
+        if (nr.y) {
+            cnu_h_pair(g, ph, lph, 1, i, j, k, cn);
+            y0 = (cn[0][0] - cn[0][1]) / dy;
+            y1 = (cn[1][1] - cn[1][0]) / dy;
+        }
+        if (nr.z) {
+            cnu_h_pair(g, ph, lph, 2, i, j, k, cn);
+            z0 = (cn[0][1] - cn[0][0]) / dz;
+            z1 = (cn[1][0] - cn[1][1]) / dz;
+        }
+        if (ux) ex += z1 + y1;
+        if (uy) ey += z0 + x1;
+        if (uz) ez += x0 + y0;
     }
     if (ux) mx = tup[t + 1] * ex;
     if (uy) my = tup[t + 3] * ey;
     if (uz) mz = tup[t + 5] * ez;
-    lEx[o] = ex;
-    lEy[o] = ey;
-    lEz[o] = ez;
-    mEx[o] = mx;
-    mEy[o] = my;
-    mEz[o] = mz;
+    sto(ex, lEx, o);
+    sto(ey, lEy, o);
+    sto(ez, lEz, o);
+    sto(mx, mEx, o);
+    sto(my, mEy, o);
+    sto(mz, mEz, o);
+    if (i == g.NX - 1) {   // the cell past the last column of tiles: fixed components
+        sto(0.0f, lEx, o + 4u);
+        sto(0.0f, lEy, o + 4u);
+        sto(0.0f, lEz, o + 4u);
+        sto(0.0f, mEx, o + 4u);
+        sto(0.0f, mEy, o + 4u);
+        sto(0.0f, mEz, o + 4u);
+    }
     if (ns) {
 #pragma unroll
         for (int A = 0; A < 3; ++A) {
             int f, q;
             long long po;
-            if (!e_psi(g, pe, A, i, j, k, f, q, po)) continue;
-            const float b = pe.b[f][q - 1];
+            if (!(A == 0 ? nr.x : (A == 1 ? nr.y : nr.z)) || !e_psi(g, pe, A, i, j, k, f, q, po)) continue;
+            const float b = (f & 1 ? pe.b[2 * A + 1] : pe.b[2 * A])[q - 1];
 #pragma unroll
             for (int sl = 0; sl < 2; ++sl) {
                 if (!e_slot_ok(A, sl, i, j, k)) continue;
                 const int c = e_slot_comp(A, sl);
-                float* nu = lpe.psi[f][sl];
+                float* nu = f & 1 ? lpe.psi[2 * A + 1][sl] : lpe.psi[2 * A][sl];
                 nu[po] = b * nu[po] + (c == 0 ? mx : (c == 1 ? my : mz));
             }
         }
@@ -3933,7 +4021,8 @@ __global__ void k_adj_nu_adjust(Grid g, const float* lE, int comp, float sign, c
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
     if (i > g.NX || j > g.NY) return;
-    if (!near_slab(g, pe, i, j, k)) return;
+    const Near nr = near_axes(g, pe, i, j, k);
+    if (!nr.x && !nr.y && !nr.z) return;
     const long long o = off(g, i, j, k);
     for (int A = 0; A < 3; ++A) {
         int f, q;
@@ -4117,7 +4206,10 @@ __global__ void k_e_design(Grid g, DesignDev d, float* Ex, float* Ey, float* Ez,
 // of every design edge ([3][nedge]) and scales lambda_E by ga;
 // k_adj_design_gather gives every H cell of the box extended by one below
 // to one thread, which adds the terms of the edges that reach it.
-__global__ void k_adj_design_m(Grid g, DesignDev d, float* lEx, float* lEy, float* lEz, float* m) {
+// Before it, where `dga` is given, the edge's terms of the gradient (k_adj_grad;
+// the record box is the design box).
+__global__ void k_adj_design_m(Grid g, DesignDev d, float* lEx, float* lEy, float* lEz, float* m, AdjRec r, double* dga,
+                               double* dgb, const int* step) {
     const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= d.nedge) return;
     const int i = d.lo[0] + (int)(e % d.n[0]);
@@ -4126,6 +4218,15 @@ __global__ void k_adj_design_m(Grid g, DesignDev d, float* lEx, float* lEy, floa
     const long long o = off(g, i, j, k), n = d.nedge;
     const float* c = d.coef;
     const float lx = lEx[o], ly = lEy[o], lz = lEz[o];
+    if (dga) {
+        const float* h = r.hist + (long long)((*step - 1) % r.slots) * 6 * n;
+        const float lam[3] = {lx, ly, lz};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            dga[q * n + e] += (double)lam[q] * (double)h[q * n + e];
+            dgb[q * n + e] += (double)lam[q] * (double)h[(3 + q) * n + e];
+        }
+    }
     m[e] = c[n + e] * lx;
     m[n + e] = c[3 * n + e] * ly;
     m[2 * n + e] = c[5 * n + e] * lz;
@@ -4173,6 +4274,5 @@ __global__ void k_adj_design_gather(Grid g, DesignDev d, const float* __restrict
     if (hz) lHz[o] = lHz[o] + sz;
 }
 
-__global__ void k_step_dec(int* step) { *step = *step - 1; }
 
 }  // namespace aemk

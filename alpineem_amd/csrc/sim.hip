@@ -2748,21 +2748,28 @@ void aem_sim::enqueue_backward_t(hipStream_t s, bool objective, double Fr, doubl
             if (adb[c].nb > 0)
                 k_adj_drude<IdxT><<<cdiv(adb[c].nb, 256), 256, 0, s>>>(g, adb[c], c, v.n_poles, lE[c], mE[c], idx, d_tup);
     }
-    if (dga && rec_on) k_adj_grad<<<cdiv(rec.nedge, 256), 256, 0, s>>>(g, rec, lEx, lEy, lEz, dga, dgb, d_bstep);
+    if (dga && rec_on && !des_on) k_adj_grad<<<cdiv(rec.nedge, 256), 256, 0, s>>>(g, rec, lEx, lEy, lEz, dga, dgb, d_bstep);
     if (des_on) {
-        k_adj_design_m<<<cdiv(des.nedge, 256), 256, 0, s>>>(g, des, lEx, lEy, lEz, d_desm);
+        k_adj_design_m<<<cdiv(des.nedge, 256), 256, 0, s>>>(g, des, lEx, lEy, lEz, d_desm, rec, rec_on ? dga : nullptr,
+                                                            dgb, d_bstep);
         const long long nh = (long long)(des.n[0] + 1) * (des.n[1] + 1) * (des.n[2] + 1);
         k_adj_design_gather<<<cdiv(nh, 256), 256, 0, s>>>(g, des, d_desm, lHx, lHy, lHz, d_den[0], d_den[1],
                                                           d_den[2]);
     }
-    const dim3 bt(64, 4, 1);
-    k_adj_h<<<dim3(cdiv(v.NX - 1, 64), cdiv(v.NY - 1, 4), v.NZ - 1), bt, 0, s>>>(
-        g, lHx, lHy, lHz, mEx, mEy, mEz, d_den[0], d_den[1], d_den[2], cpE, lpE, cpH, lpH, v.DB, v.dx, v.dy, v.dz);
+    const dim3 bt(64, 4, 1), gh(cdiv(v.NX - 1, 64), cdiv(v.NY - 1, 4), v.NZ - 1), ge(cdiv(v.NX - 1, 64), cdiv(v.NY, 4), v.NZ);
+    if (off32)
+        k_adj_h<uint32_t><<<gh, bt, 0, s>>>(g, lHx, lHy, lHz, mEx, mEy, mEz, d_den[0], d_den[1], d_den[2], cpE, lpE, cpH,
+                                            lpH, v.DB, v.dx, v.dy, v.dz);
+    else
+        k_adj_h<uint64_t><<<gh, bt, 0, s>>>(g, lHx, lHy, lHz, mEx, mEy, mEz, d_den[0], d_den[1], d_den[2], cpE, lpE, cpH,
+                                            lpH, v.DB, v.dx, v.dy, v.dz);
     if (v.n_ports > 0) k_adj_ports_h<<<1, 64, 0, s>>>(g, ap, lHx, lHy, lHz, v.dx, v.dy, v.dz, d_bstep);
-    k_adj_e<IdxT><<<dim3(cdiv(v.NX, 64), cdiv(v.NY, 4), v.NZ), bt, 0, s>>>(
-        g, lEx, lEy, lEz, mEx, mEy, mEz, lHx, lHy, lHz, idx, d_tup, d_den[3], d_den[4], d_den[5], cpE, lpE, cpH, lpH,
-        v.DB, v.dx, v.dy, v.dz);
-    k_step_dec<<<1, 1, 0, s>>>(d_bstep);
+    if (off32)
+        k_adj_e<IdxT, uint32_t><<<ge, bt, 0, s>>>(g, lEx, lEy, lEz, mEx, mEy, mEz, lHx, lHy, lHz, idx, d_tup, d_den[3],
+                                                  d_den[4], d_den[5], cpE, lpE, cpH, lpH, v.DB, v.dx, v.dy, v.dz, d_bstep);
+    else
+        k_adj_e<IdxT, uint64_t><<<ge, bt, 0, s>>>(g, lEx, lEy, lEz, mEx, mEy, mEz, lHx, lHy, lHz, idx, d_tup, d_den[3],
+                                                  d_den[4], d_den[5], cpE, lpE, cpH, lpH, v.DB, v.dx, v.dy, v.dz, d_bstep);
 }
 
 namespace {
