@@ -184,18 +184,50 @@ __device__ __forceinline__ void h_bulk_body(const Grid& g, const Box& b, int bx,
                                             const float* __restrict__ dhz, float DB, const Cpml& cp, float dx,
                                             float dy, float dz) {
     const int i = b.i0 + bx * kTX + (int)threadIdx.x;
-    const int j = b.j0 + by * kTY + (int)threadIdx.y;
+    const int j = __builtin_amdgcn_readfirstlane(b.j0 + by * kTY + (int)threadIdx.y);   // one row per wave
     if (i >= b.i0 + b.ni || j >= b.j0 + b.nj) return;
     const int k0 = b.k0 + bz * b.kc;
     const int k1 = min(k0 + b.kc, b.k0 + b.nk) - 1;
     const float dx_i = dhx[i - 1], dy_j = dhy[j - 1];
+    // Slabs: what does not change over the march (the face's arrays, the
+    // coefficients, the psi offset) before it, psi of a plane with the
+    // plane's fields: read in the branch that uses them they were a second
+    // latency per plane, behind a pointer load from the argument block.  The
+    // two x faces of a slot share one allocation, so a lane needs an offset.
     int qx = 0, qy = 0;
     const int fx = (C & kCx) ? slab_h(i, g.NX, cp.n[0], cp.n[1], qx) : -1;
     const int fy = (C & kCy) ? slab_h(j, g.NY, cp.n[2], cp.n[3], qy) : -1;
+    const bool sx = (C & kCx) && fx >= 0, sy = (C & kCy) && fy >= 0;
+    float cbx = 0.f, ccx = 0.f, cby = 0.f, ccy = 0.f;
+    OffT ox = 0, dox = 0, oy = 0, doy = 0;
+    if (sx) {
+        cbx = (fx ? cp.b[1] : cp.b[0])[qx - 1];
+        ccx = (fx ? cp.c[1] : cp.c[0])[qx - 1];
+        const OffT nt = (OffT)((fx ? cp.n[1] : cp.n[0]) - 1);
+        ox = ((fx ? (OffT)(cp.psi[1][0] - cp.psi[0][0]) : (OffT)0) + (OffT)(qx - 1) +
+              nt * ((OffT)(j - 1) + (OffT)g.NY * (OffT)(k0 - 1))) * 4u;
+        dox = nt * (OffT)g.NY * 4u;
+    }
+    if (sy) {
+        cby = (fy ? cp.b[3] : cp.b[2])[qy - 1];
+        ccy = (fy ? cp.c[3] : cp.c[2])[qy - 1];
+        const OffT nt = (OffT)((fy ? cp.n[3] : cp.n[2]) - 1);
+        oy = ((OffT)(i - 1) + (OffT)g.PX * ((OffT)(qy - 1) + nt * (OffT)(k0 - 1))) * 4u;
+        doy = (OffT)g.PX * nt * 4u;
+    }
+    float* const x0 = cp.psi[0][0];
+    float* const x1 = cp.psi[0][1];
+    float* const x0o = PP ? cp.pso[0][0] : x0;
+    float* const x1o = PP ? cp.pso[0][1] : x1;
+    float* const y0 = fy > 0 ? cp.psi[3][0] : cp.psi[2][0];
+    float* const y1 = fy > 0 ? cp.psi[3][1] : cp.psi[2][1];
+    float* const y0o = PP ? (fy > 0 ? cp.pso[3][0] : cp.pso[2][0]) : y0;
+    float* const y1o = PP ? (fy > 0 ? cp.pso[3][1] : cp.pso[2][1]) : y1;
     // byte offsets from the array bases (OffT: 32 bits where the arrays stay
     // under 4 GiB, so one VGPR addresses every array)
     const OffT PB = (OffT)g.PX * 4u, ZB = (OffT)g.plane * 4u;
     OffT o = (OffT)off(g, i, j, k0) * 4u;
+    const OffT ozc = ((OffT)(i - 1) + (OffT)g.PX * (OffT)(j - 1)) * 4u;
     float ey_k = ldo(Ey, o), ex_k = ldo(Ex, o);
     for (int k = k0; k <= k1; ++k) {
         const float ey_k1 = ldo(Ey, o + ZB);
@@ -206,47 +238,54 @@ __device__ __forceinline__ void h_bulk_body(const Grid& g, const Box& b, int bx,
         const float ey_xp = ldo(Ey, o + 4u);
         const float ex_yp = ldo(Ex, o + PB);
         const float dz_k = dhz[k - 1];
-        float hx = ldo_once(Hx, o) + DB * ((ez - ez_yp) * dy_j + (ey_k1 - ey_k) * dz_k);
-        float hy = ldo_once(Hy, o) + DB * ((ez_xp - ez) * dx_i + (ex_k - ex_k1) * dz_k);
-        float hz = ldo_once(Hz, o) + DB * ((ey_k - ey_xp) * dx_i + (ex_yp - ex_k) * dy_j);
-        if (C) {
-            if ((C & kCx) && fx >= 0) {                      // psi_Hyx, psi_Hzx
-                const int f = fx;
-                const int ntf = cp.n[f] - 1;
-                const long long po = (long long)(qx - 1) + (long long)ntf * ((long long)(j - 1) + (long long)g.NY * (k - 1));
-                const float cb = cp.b[f][qx - 1], cc = cp.c[f][qx - 1];
-                float p0 = cb * cp.psi[f][0][po] + cc * (ez_xp - ez) / dx;
-                (PP ? cp.pso[f][0] : cp.psi[f][0])[po] = p0;
-                hy = hy + DB * p0;
-                float p1 = cb * cp.psi[f][1][po] + cc * (ey_k - ey_xp) / dx;
-                (PP ? cp.pso[f][1] : cp.psi[f][1])[po] = p1;
-                hz = hz + DB * p1;
-            }
-            if ((C & kCy) && fy >= 0) {                      // psi_Hxy, psi_Hzy
-                const int f = 2 + fy;
-                const int ntf = cp.n[f] - 1;
-                const long long po = (long long)(i - 1) + (long long)g.PX * ((long long)(qy - 1) + (long long)ntf * (k - 1));
-                const float cb = cp.b[f][qy - 1], cc = cp.c[f][qy - 1];
-                float p0 = cb * cp.psi[f][0][po] + cc * (ez - ez_yp) / dy;
-                (PP ? cp.pso[f][0] : cp.psi[f][0])[po] = p0;
-                hx = hx + DB * p0;
-                float p1 = cb * cp.psi[f][1][po] + cc * (ex_yp - ex_k) / dy;
-                (PP ? cp.pso[f][1] : cp.psi[f][1])[po] = p1;
-                hz = hz + DB * p1;
-            }
-            int qz = 0;
-            const int fz = (C & kCz) ? slab_h(k, g.NZ, cp.n[4], cp.n[5], qz) : -1;
-            if ((C & kCz) && fz >= 0) {                      // psi_Hxz, psi_Hyz
-                const int f = 4 + fz;
-                const long long po = (long long)(i - 1) + (long long)g.PX * ((long long)(j - 1) + (long long)g.NY * (qz - 1));
-                const float cb = cp.b[f][qz - 1], cc = cp.c[f][qz - 1];
-                float p0 = cb * cp.psi[f][0][po] + cc * (ey_k1 - ey_k) / dz;
-                (PP ? cp.pso[f][0] : cp.psi[f][0])[po] = p0;
-                hx = hx + DB * p0;
-                float p1 = cb * cp.psi[f][1][po] + cc * (ex_k - ex_k1) / dz;
-                (PP ? cp.pso[f][1] : cp.psi[f][1])[po] = p1;
-                hy = hy + DB * p1;
-            }
+        const float hx0 = ldo_once(Hx, o), hy0 = ldo_once(Hy, o), hz0 = ldo_once(Hz, o);
+        float px0 = 0.f, px1 = 0.f, py0 = 0.f, py1 = 0.f, pz0 = 0.f, pz1 = 0.f, cbz = 0.f, ccz = 0.f;
+        if (sx) {
+            px0 = ldo(x0, ox);
+            px1 = ldo(x1, ox);
+        }
+        if (sy) {
+            py0 = ldo(y0, oy);
+            py1 = ldo(y1, oy);
+        }
+        int qz = 0;
+        const int fz = (C & kCz) ? slab_h(k, g.NZ, cp.n[4], cp.n[5], qz) : -1;
+        const bool sz = (C & kCz) && fz >= 0;
+        float* const z0 = fz > 0 ? cp.psi[5][0] : cp.psi[4][0];
+        float* const z1 = fz > 0 ? cp.psi[5][1] : cp.psi[4][1];
+        const OffT oz = ozc + (OffT)g.PX * (OffT)g.NY * (OffT)(qz > 0 ? qz - 1 : 0) * 4u;
+        if (sz) {
+            pz0 = ldo(z0, oz);
+            pz1 = ldo(z1, oz);
+            cbz = (fz ? cp.b[5] : cp.b[4])[qz - 1];
+            ccz = (fz ? cp.c[5] : cp.c[4])[qz - 1];
+        }
+        float hx = hx0 + DB * ((ez - ez_yp) * dy_j + (ey_k1 - ey_k) * dz_k);
+        float hy = hy0 + DB * ((ez_xp - ez) * dx_i + (ex_k - ex_k1) * dz_k);
+        float hz = hz0 + DB * ((ey_k - ey_xp) * dx_i + (ex_yp - ex_k) * dy_j);
+        if (sx) {                                            // psi_Hyx, psi_Hzx
+            const float p0 = cbx * px0 + ccx * (ez_xp - ez) / dx;
+            sto(p0, x0o, ox);
+            hy = hy + DB * p0;
+            const float p1 = cbx * px1 + ccx * (ey_k - ey_xp) / dx;
+            sto(p1, x1o, ox);
+            hz = hz + DB * p1;
+        }
+        if (sy) {                                            // psi_Hxy, psi_Hzy
+            const float p0 = cby * py0 + ccy * (ez - ez_yp) / dy;
+            sto(p0, y0o, oy);
+            hx = hx + DB * p0;
+            const float p1 = cby * py1 + ccy * (ex_yp - ex_k) / dy;
+            sto(p1, y1o, oy);
+            hz = hz + DB * p1;
+        }
+        if (sz) {                                            // psi_Hxz, psi_Hyz
+            const float p0 = cbz * pz0 + ccz * (ey_k1 - ey_k) / dz;
+            sto(p0, PP ? (fz ? cp.pso[5][0] : cp.pso[4][0]) : z0, oz);
+            hx = hx + DB * p0;
+            const float p1 = cbz * pz1 + ccz * (ex_k - ex_k1) / dz;
+            sto(p1, PP ? (fz ? cp.pso[5][1] : cp.pso[4][1]) : z1, oz);
+            hy = hy + DB * p1;
         }
         sto_once(hx, PP ? Hxo : Hx, o);
         sto_once(hy, PP ? Hyo : Hy, o);
@@ -254,6 +293,8 @@ __device__ __forceinline__ void h_bulk_body(const Grid& g, const Box& b, int bx,
         ey_k = ey_k1;
         ex_k = ex_k1;
         o += ZB;
+        ox += dox;
+        oy += doy;
     }
 }
 
@@ -272,17 +313,45 @@ __device__ __forceinline__ void e_bulk_body(const Grid& g, const Box& b, int bx,
                                             const float* __restrict__ dey, const float* __restrict__ dez,
                                             const Cpml& cp, float dx, float dy, float dz) {
     const int i = b.i0 + bx * kTX + (int)threadIdx.x;
-    const int j = b.j0 + by * kTY + (int)threadIdx.y;
+    const int j = __builtin_amdgcn_readfirstlane(b.j0 + by * kTY + (int)threadIdx.y);   // one row per wave
     if (i >= b.i0 + b.ni || j >= b.j0 + b.nj) return;
     const int k0 = b.k0 + bz * b.kc;
     const int k1 = min(k0 + b.kc, b.k0 + b.nk) - 1;
     const float dx_i = dex[i - 1], dy_j = dey[j - 1];
     const bool ix = i >= 2, jy = j >= 2;
+    // slabs as in h_bulk_body
     int qx = 0, tx = 0, qy = 0, ty = 0;
     const int fx = (C & kCx) ? slab_e(i, g.NX, cp.n[0], cp.n[1], qx, tx) : -1;
     const int fy = (C & kCy) ? slab_e(j, g.NY, cp.n[2], cp.n[3], qy, ty) : -1;
+    const bool sx = (C & kCx) && fx >= 0, sy = (C & kCy) && fy >= 0;
+    float cbx = 0.f, ccx = 0.f, cby = 0.f, ccy = 0.f;
+    OffT ox = 0, dox = 0, oy = 0, doy = 0;
+    if (sx) {
+        cbx = (fx ? cp.b[1] : cp.b[0])[qx - 1];
+        ccx = (fx ? cp.c[1] : cp.c[0])[qx - 1];
+        const OffT nt = (OffT)((fx ? cp.n[1] : cp.n[0]) - 1);
+        ox = ((fx ? (OffT)(cp.psi[1][0] - cp.psi[0][0]) : (OffT)0) + (OffT)tx +
+              nt * ((OffT)(j - 1) + (OffT)g.NY * (OffT)(k0 - 1))) * 4u;
+        dox = nt * (OffT)g.NY * 4u;
+    }
+    if (sy) {
+        cby = (fy ? cp.b[3] : cp.b[2])[qy - 1];
+        ccy = (fy ? cp.c[3] : cp.c[2])[qy - 1];
+        const OffT nt = (OffT)((fy ? cp.n[3] : cp.n[2]) - 1);
+        oy = ((OffT)(i - 1) + (OffT)g.PX * ((OffT)ty + nt * (OffT)(k0 - 1))) * 4u;
+        doy = (OffT)g.PX * nt * 4u;
+    }
+    float* const x0 = cp.psi[0][0];
+    float* const x1 = cp.psi[0][1];
+    float* const x0o = PP ? cp.pso[0][0] : x0;
+    float* const x1o = PP ? cp.pso[0][1] : x1;
+    float* const y0 = fy > 0 ? cp.psi[3][0] : cp.psi[2][0];
+    float* const y1 = fy > 0 ? cp.psi[3][1] : cp.psi[2][1];
+    float* const y0o = PP ? (fy > 0 ? cp.pso[3][0] : cp.pso[2][0]) : y0;
+    float* const y1o = PP ? (fy > 0 ? cp.pso[3][1] : cp.pso[2][1]) : y1;
     const OffT PB = (OffT)g.PX * 4u, ZB = (OffT)g.plane * 4u;
     OffT o = (OffT)off(g, i, j, k0) * 4u;   // byte offset, as in h_bulk_body
+    const OffT ozc = ((OffT)(i - 1) + (OffT)g.PX * (OffT)(j - 1)) * 4u;
     OffT oi = (OffT)off(g, i, j, k0) * (OffT)sizeof(IdxT);
     const OffT ZI = (OffT)g.plane * (OffT)sizeof(IdxT);
     float hx_km = 0.f, hy_km = 0.f;
@@ -307,60 +376,66 @@ __device__ __forceinline__ void e_bulk_body(const Grid& g, const Box& b, int bx,
         const float hy_xm = ldo(Hy, o - dxm);
         const float hx_ym = ldo(Hx, o - dym);
         const float ex0 = ldo_once(Ex, o), ey0 = ldo_once(Ey, o), ez0 = ldo_once(Ez, o);
+        float px0 = 0.f, px1 = 0.f, py0 = 0.f, py1 = 0.f, pz0 = 0.f, pz1 = 0.f, cbz = 0.f, ccz = 0.f;
+        if (sx) {
+            px0 = ldo(x0, ox);
+            px1 = ldo(x1, ox);
+        }
+        if (sy) {
+            py0 = ldo(y0, oy);
+            py1 = ldo(y1, oy);
+        }
+        int qz = 0, tz = 0;
+        const int fz = (C & kCz) ? slab_e(k, g.NZ, cp.n[4], cp.n[5], qz, tz) : -1;
+        const bool sz = (C & kCz) && fz >= 0;
+        float* const z0 = fz > 0 ? cp.psi[5][0] : cp.psi[4][0];
+        float* const z1 = fz > 0 ? cp.psi[5][1] : cp.psi[4][1];
+        const OffT oz = ozc + (OffT)g.PX * (OffT)g.NY * (OffT)tz * 4u;
+        if (sz) {
+            pz0 = ldo(z0, oz);
+            pz1 = ldo(z1, oz);
+            cbz = (fz ? cp.b[5] : cp.b[4])[qz - 1];
+            ccz = (fz ? cp.c[5] : cp.c[4])[qz - 1];
+        }
         const float gax = tup[t + 0], gbx = tup[t + 1], gay = tup[t + 2], gby = tup[t + 3], gaz = tup[t + 4],
                     gbz = tup[t + 5];
         float ex = gax * ex0 + gbx * ((hz - hz_ym) * dy_j + (hy_km - hy) * dz_k);
         float ey = gay * ey0 + gby * ((hz_xm - hz) * dx_i + (hx - hx_km) * dz_k);
         float ez = gaz * ez0 + gbz * ((hy - hy_xm) * dx_i + (hx_ym - hx) * dy_j);
-        if (C) {
-            if ((C & kCx) && fx >= 0) {                      // psi_Eyx, psi_Ezx
-                const int f = fx;
-                const int ntf = cp.n[f] - 1;
-                const long long po = (long long)tx + (long long)ntf * ((long long)(j - 1) + (long long)g.NY * (k - 1));
-                const float cb = cp.b[f][qx - 1], cc = cp.c[f][qx - 1];
-                if (k >= 2) {
-                    float p = cb * cp.psi[f][0][po] + cc * (hz_xm - hz) / dx;
-                    (PP ? cp.pso[f][0] : cp.psi[f][0])[po] = p;
-                    ey = ey + gby * p;
-                }
-                if (jy) {
-                    float p = cb * cp.psi[f][1][po] + cc * (hy - hy_xm) / dx;
-                    (PP ? cp.pso[f][1] : cp.psi[f][1])[po] = p;
-                    ez = ez + gbz * p;
-                }
+        if (sx) {                                            // psi_Eyx, psi_Ezx
+            if (k >= 2) {
+                const float p = cbx * px0 + ccx * (hz_xm - hz) / dx;
+                sto(p, x0o, ox);
+                ey = ey + gby * p;
             }
-            if ((C & kCy) && fy >= 0) {                      // psi_Exy, psi_Ezy
-                const int f = 2 + fy;
-                const int ntf = cp.n[f] - 1;
-                const long long po = (long long)(i - 1) + (long long)g.PX * ((long long)ty + (long long)ntf * (k - 1));
-                const float cb = cp.b[f][qy - 1], cc = cp.c[f][qy - 1];
-                if (k >= 2) {
-                    float p = cb * cp.psi[f][0][po] + cc * (hz - hz_ym) / dy;
-                    (PP ? cp.pso[f][0] : cp.psi[f][0])[po] = p;
-                    ex = ex + gbx * p;
-                }
-                if (ix) {
-                    float p = cb * cp.psi[f][1][po] + cc * (hx_ym - hx) / dy;
-                    (PP ? cp.pso[f][1] : cp.psi[f][1])[po] = p;
-                    ez = ez + gbz * p;
-                }
+            if (jy) {
+                const float p = cbx * px1 + ccx * (hy - hy_xm) / dx;
+                sto(p, x1o, ox);
+                ez = ez + gbz * p;
             }
-            int qz = 0, tz = 0;
-            const int fz = (C & kCz) ? slab_e(k, g.NZ, cp.n[4], cp.n[5], qz, tz) : -1;
-            if ((C & kCz) && fz >= 0) {                      // psi_Exz, psi_Eyz
-                const int f = 4 + fz;
-                const long long po = (long long)(i - 1) + (long long)g.PX * ((long long)(j - 1) + (long long)g.NY * tz);
-                const float cb = cp.b[f][qz - 1], cc = cp.c[f][qz - 1];
-                if (jy) {
-                    float p = cb * cp.psi[f][0][po] + cc * (hy_km - hy) / dz;
-                    (PP ? cp.pso[f][0] : cp.psi[f][0])[po] = p;
-                    ex = ex + gbx * p;
-                }
-                if (ix) {
-                    float p = cb * cp.psi[f][1][po] + cc * (hx - hx_km) / dz;
-                    (PP ? cp.pso[f][1] : cp.psi[f][1])[po] = p;
-                    ey = ey + gby * p;
-                }
+        }
+        if (sy) {                                            // psi_Exy, psi_Ezy
+            if (k >= 2) {
+                const float p = cby * py0 + ccy * (hz - hz_ym) / dy;
+                sto(p, y0o, oy);
+                ex = ex + gbx * p;
+            }
+            if (ix) {
+                const float p = cby * py1 + ccy * (hx_ym - hx) / dy;
+                sto(p, y1o, oy);
+                ez = ez + gbz * p;
+            }
+        }
+        if (sz) {                                            // psi_Exz, psi_Eyz
+            if (jy) {
+                const float p = cbz * pz0 + ccz * (hy_km - hy) / dz;
+                sto(p, PP ? (fz ? cp.pso[5][0] : cp.pso[4][0]) : z0, oz);
+                ex = ex + gbx * p;
+            }
+            if (ix) {
+                const float p = cbz * pz1 + ccz * (hx - hx_km) / dz;
+                sto(p, PP ? (fz ? cp.pso[5][1] : cp.pso[4][1]) : z1, oz);
+                ey = ey + gby * p;
             }
         }
         // components outside the reference's update ranges get their own
@@ -372,6 +447,8 @@ __device__ __forceinline__ void e_bulk_body(const Grid& g, const Box& b, int bx,
         hy_km = hy;
         o += ZB;
         oi += ZI;
+        ox += dox;
+        oy += doy;
     }
 }
 
