@@ -2755,16 +2755,19 @@ __global__ void __launch_bounds__(64 * kListWavesMany) k_ntff_list_batch(const N
     ntff_list_body<kListWavesMany>(a.L, a.bn, a.step, (int)blockIdx.x);
 }
 
-// Builds the contributor lists: one thread per (list row, bin offset) walks
-// the face cells in the reference's loop order and emits those that can reach
-// its bin, counting them per face pair first (FILL false), then writing them.
+// Builds the contributor lists: one wave per (list row, bin offset, face pair)
+// walks the face cells in the reference's loop order, 32 of a row on both sides
+// at a time, and emits those that can reach its bin, counting them first (FILL
+// false), then writing them at the rank a ballot gives them.
 // An FP64 linear model of the retarded time, widened by a margin that covers
 // the FP32 evaluation error (as in k_ntff_exact), gives the candidate cells;
 // the FP32 time of each candidate decides.  A cell whose exact offset x lies
 // within eps of a bin edge (eps: the FP32 rounding of n + x, doubled) is
 // listed for every bin it can reach.  On the device because a host loop over
-// the cells, angles and bins took longer than the run's far field itself
-// (100^3 with 37 angles: 117 ms on the host, 5.3 ms here).
+// the cells, angles and bins took longer than the run's far field itself, and
+// by waves because one thread per list leaves the longest lists and most of the
+// chip waiting.  Both passes, 100^3 with 37 angles: 117 ms on the host, 6.7 by
+// threads, 0.5 by waves; 200^3 with 3 angles 24.5 by threads, 0.7.
 struct NtffBuild {
     const float* ang;       // [n_angles][6]
     const int* win;         // per angle: lowest bin offset, offsets
@@ -2782,10 +2785,14 @@ struct NtffBuild {
 
 template <bool FILL>
 __global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    const int q = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    const int lane = (int)(threadIdx.x & 63);
     const int row = blockIdx.y;
+    const int m = (int)blockIdx.z / 3, a = (int)blockIdx.z % 3;   // the box's faces, then the images'; face pair
     const int kk = row % P.n_angles;
     if (q >= P.win[2 * kk + 1]) return;
+    const size_t at = (size_t)row * P.win_max + q;
+    if (P.pbc[a]) return;                                  // (the counts start at 0)
     const int Q = P.win[2 * kk] + q;
     const bool isW = row >= P.n_angles;
     const double shift = isW ? -1.0 : -0.5;
@@ -2793,76 +2800,96 @@ __global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
     const float s1 = an[2], c1 = an[3], s2 = an[4], c2 = an[5];
     const double g[3] = {(double)P.d[0] * s1 * c2, (double)P.d[1] * s1 * s2, (double)P.d[2] * c1};
     const double cdt = (double)P.c_dt;
-    const size_t at = (size_t)row * P.win_max + q;
     const int step = FILL ? P.dst[8 * at + 1] : 0;
-    for (int m = 0; m < 2; ++m)
-        for (int a = 0; a < 3; ++a) {                     // face pairs in the reference's order
-            int cnt = 0;
-            if (m < P.passes && !P.pbc[a]) {
-                uint2* out = FILL ? P.ent + P.dst[8 * at] + (long long)P.dst[8 * at + 2 + 3 * m + a] * step : nullptr;
-                const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
-                // sign bits of the two components of an image current
-                uint32_t sg = 0u;
-                if (m && (isW ? P.sgn_J[b] : P.sgn_M[b]) < 0.0f) sg |= 0x80000000u;
-                if (m && (isW ? P.sgn_J[c] : P.sgn_M[c]) < 0.0f) sg |= 0x40000000u;
-                // position along an axis, the image's on the ground plane's
-                auto pos_of = [&](int ax, int i) { return m && P.use_m[ax] ? P.off_m[ax] - i : i; };
-                const double sb = m && P.use_m[b] ? -1.0 : 1.0, sc = m && P.use_m[c] ? -1.0 : 1.0;
-                const double mu = -sb * g[b] / cdt, mv = -sc * g[c] / cdt;
-                double base[2];
-                for (int side = 0; side < 2; ++side) {
-                    const double S0 = (double)(pos_of(a, side ? P.hi[a] : P.lo[a]) - P.c[a]) * g[a] +
-                                      (double)(pos_of(b, 0) - P.c[b]) * g[b] + (double)(pos_of(c, 0) - P.c[c]) * g[c];
-                    base[side] = ((double)P.r_relay - S0) / cdt + shift;
-                }
-                const double marg = P.eps + 4e-3 + 4e-7 * fabs(base[0] + mu * P.lo[b] + mv * P.lo[c]);
-                const double lo_t = (double)Q - 1.0 - marg, hi_t = (double)Q + 1.0 + marg;
-                const double inv_mu = fabs(mu) < 1e-12 ? 0.0 : 1.0 / mu;
-                for (int v = P.lo[c]; v <= P.hi[c]; ++v) {
-                    int ulo[2], uhi[2];
-                    for (int side = 0; side < 2; ++side) {
-                        const double bv = base[side] + mv * v;
-                        if (inv_mu == 0.0) {
-                            const bool in = bv >= lo_t && bv <= hi_t;
-                            ulo[side] = in ? P.lo[b] : P.hi[b] + 1;
-                            uhi[side] = in ? P.hi[b] : P.lo[b] - 1;
-                        } else {
-                            const double u1 = (lo_t - bv) * inv_mu, u2 = (hi_t - bv) * inv_mu;
-                            ulo[side] = max(P.lo[b], (int)ceil(fmin(fmax(fmin(u1, u2), -1e9), 1e9)));
-                            uhi[side] = min(P.hi[b], (int)floor(fmax(fmin(fmax(u1, u2), 1e9), -1e9)));
-                        }
-                    }
-                    const bool e0 = ulo[0] <= uhi[0], e1 = ulo[1] <= uhi[1];
-                    if (!e0 && !e1) continue;
-                    const int ua = e0 ? (e1 ? min(ulo[0], ulo[1]) : ulo[0]) : ulo[1];
-                    const int ub = e0 ? (e1 ? max(uhi[0], uhi[1]) : uhi[0]) : uhi[1];
-                    for (int u = ua; u <= ub; ++u)
-                        for (int side = 0; side < 2; ++side) {
-                            if (u < ulo[side] || u > uhi[side]) continue;
-                            const int pos = side ? P.hi[a] : P.lo[a];
-                            int i, j, k;
-                            if (a == 0) { i = pos; j = u; k = v; }
-                            else if (a == 1) { i = u; j = pos; k = v; }
-                            else { i = u; j = v; k = pos; }
-                            i = pos_of(0, i);
-                            j = pos_of(1, j);
-                            k = pos_of(2, k);
-                            const float tfv = (P.r_relay - ((float)(i - P.c[0]) * P.d[0] * s1 * c2 +
-                                                            (float)(j - P.c[1]) * P.d[1] * s1 * s2 +
-                                                            (float)(k - P.c[2]) * P.d[2] * c1)) / P.c_dt;
-                            const double x = (double)tfv + shift;
-                            if (Q < (int)floor(x - P.eps) || Q > (int)floor(x + P.eps) + 1) continue;
-                            if (FILL) {
-                                const int face = 2 * a + side;
-                                const unsigned idx = (unsigned)face * P.stride + (unsigned)(u + P.fd0[face] * v);
-                                out[(long long)cnt * step] = make_uint2(idx | sg, __float_as_uint(tfv));
-                            }
-                            ++cnt;
-                        }
-                }
-            }
-            if (!FILL) P.count[6 * at + 3 * m + a] = cnt;
+    uint2* out = FILL ? P.ent + P.dst[8 * at] + (long long)P.dst[8 * at + 2 + 3 * m + a] * step : nullptr;
+    // axes by selects: an index would put the arguments in scratch
+    auto sel = [](int ax, const auto& v) { return ax == 0 ? v[0] : (ax == 1 ? v[1] : v[2]); };
+    const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+    // sign bits of the two components of an image current
+    uint32_t sg = 0u;
+    if (m && (isW ? sel(b, P.sgn_J) : sel(b, P.sgn_M)) < 0.0f) sg |= 0x80000000u;
+    if (m && (isW ? sel(c, P.sgn_J) : sel(c, P.sgn_M)) < 0.0f) sg |= 0x40000000u;
+    // position along an axis, the image's on the ground plane's
+    auto pos_of = [&](int ax, int i) { return m && sel(ax, P.use_m) ? sel(ax, P.off_m) - i : i; };
+    const double sb = m && sel(b, P.use_m) ? -1.0 : 1.0, sc = m && sel(c, P.use_m) ? -1.0 : 1.0;
+    const double mu = -sb * sel(b, g) / cdt, mv = -sc * sel(c, g) / cdt;
+    const int blo = sel(b, P.lo), bhi = sel(b, P.hi), clo = sel(c, P.lo), chi = sel(c, P.hi);
+    const int alo = sel(a, P.lo), ahi = sel(a, P.hi);
+    double base[2];
+    for (int side = 0; side < 2; ++side) {
+        const double S0 = (double)(pos_of(a, side ? ahi : alo) - sel(a, P.c)) * sel(a, g) +
+                          (double)(pos_of(b, 0) - sel(b, P.c)) * sel(b, g) + (double)(pos_of(c, 0) - sel(c, P.c)) * sel(c, g);
+        base[side] = ((double)P.r_relay - S0) / cdt + shift;
+    }
+    const double marg = P.eps + 4e-3 + 4e-7 * fabs(base[0] + mu * blo + mv * clo);
+    const double lo_t = (double)Q - 1.0 - marg, hi_t = (double)Q + 1.0 + marg;
+    const double inv_mu = fabs(mu) < 1e-12 ? 0.0 : 1.0 / mu;
+    // rows whose times over u meet [lo_t, hi_t], on either side
+    const double umin = fmin(mu * blo, mu * bhi), umax = fmax(mu * blo, mu * bhi);
+    int va = chi + 1, vb = clo - 1;
+    for (int side = 0; side < 2; ++side) {
+        int s0, s1v;
+        if (fabs(mv) < 1e-12) {
+            const bool in = base[side] + umax >= lo_t && base[side] + umin <= hi_t;
+            s0 = in ? clo : chi + 1;
+            s1v = in ? chi : clo - 1;
+        } else {
+            const double v1 = (lo_t - base[side] - umax) / mv, v2 = (hi_t - base[side] - umin) / mv;
+            s0 = max(clo, (int)ceil(fmin(fmax(fmin(v1, v2), -1e9), 1e9)));
+            s1v = min(chi, (int)floor(fmax(fmin(fmax(v1, v2), 1e9), -1e9)));
         }
+        if (s0 <= s1v) {
+            va = min(va, s0);
+            vb = max(vb, s1v);
+        }
+    }
+    int cnt = 0;
+    const int side = lane & 1;                             // lanes: cells u, low and high face of each
+    const int pos = side ? ahi : alo;
+    const int face = 2 * a + side;
+    const int fd = a == 0 ? P.fd0[0] : (a == 1 ? P.fd0[2] : P.fd0[4]);   // the same for both sides
+    for (int v = va; v <= vb; ++v) {
+        int ulo[2], uhi[2];
+        for (int h = 0; h < 2; ++h) {
+            const double bv = base[h] + mv * v;
+            if (inv_mu == 0.0) {
+                const bool in = bv >= lo_t && bv <= hi_t;
+                ulo[h] = in ? blo : bhi + 1;
+                uhi[h] = in ? bhi : blo - 1;
+            } else {
+                const double u1 = (lo_t - bv) * inv_mu, u2 = (hi_t - bv) * inv_mu;
+                ulo[h] = max(blo, (int)ceil(fmin(fmax(fmin(u1, u2), -1e9), 1e9)));
+                uhi[h] = min(bhi, (int)floor(fmax(fmin(fmax(u1, u2), 1e9), -1e9)));
+            }
+        }
+        const bool e0 = ulo[0] <= uhi[0], e1 = ulo[1] <= uhi[1];
+        if (!e0 && !e1) continue;
+        const int ua = e0 ? (e1 ? min(ulo[0], ulo[1]) : ulo[0]) : ulo[1];
+        const int ub = e0 ? (e1 ? max(uhi[0], uhi[1]) : uhi[0]) : uhi[1];
+        for (int u0 = ua; u0 <= ub; u0 += 32) {
+            const int u = u0 + (lane >> 1);
+            int i, j, k;
+            if (a == 0) { i = pos; j = u; k = v; }
+            else if (a == 1) { i = u; j = pos; k = v; }
+            else { i = u; j = v; k = pos; }
+            i = pos_of(0, i);
+            j = pos_of(1, j);
+            k = pos_of(2, k);
+            const float tfv = (P.r_relay - ((float)(i - P.c[0]) * P.d[0] * s1 * c2 + (float)(j - P.c[1]) * P.d[1] * s1 * s2 +
+                                            (float)(k - P.c[2]) * P.d[2] * c1)) / P.c_dt;
+            const double x = (double)tfv + shift;
+            const bool in = u >= (side ? ulo[1] : ulo[0]) && u <= (side ? uhi[1] : uhi[0]) &&
+                            Q >= (int)floor(x - P.eps) && Q <= (int)floor(x + P.eps) + 1;
+            const unsigned long long hits = __ballot(in);
+            if (FILL && in) {
+                const int p = cnt + __popcll(hits & ((1ull << lane) - 1ull));
+                const unsigned idx = (unsigned)face * P.stride + (unsigned)(u + fd * v);
+                out[(long long)p * step] = make_uint2(idx | sg, __float_as_uint(tfv));
+            }
+            cnt += __popcll(hits);
+        }
+    }
+    if (!FILL && lane == 0) P.count[6 * at + 3 * m + a] = cnt;
 }
 
 // NTFF retarded-time binning through an LDS histogram (f90:7643-7927 with

@@ -1696,7 +1696,8 @@ void aem_sim::build_ntff_lists(const std::vector<int>& win, unsigned stride) {
     B.count = dalloc<int>(cnt.size(), tmp);
     int* d_dst = dalloc<int>(dst.size(), tmp);
     B.dst = d_dst;
-    const dim3 grid(cdiv(win_max, 256), rows);
+    const dim3 grid(cdiv(win_max, 4), rows, 3 * B.passes);   // four waves per work-group
+    HIPCHK(hipMemsetAsync(B.count, 0, cnt.size() * sizeof(int), st));
     k_ntff_build<false><<<grid, 256, 0, st>>>(B);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(cnt.data(), B.count, cnt.size() * sizeof(int), hipMemcpyDeviceToHost, st));
