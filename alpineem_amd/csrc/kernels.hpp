@@ -488,17 +488,21 @@ struct BatchEntry {
     Box box;
 };
 
-// Entry of this work-group (binary search on `first`, uniform per group) and
-// its (x, y, z-chunk) block coordinates inside the entry's box.
-__device__ __forceinline__ BatchEntry entry_of(const BatchEntry* __restrict__ e, int n, int& bx, int& by, int& bz) {
-    const int g = (int)blockIdx.x;
+// Entry that work-group g belongs to (binary search on `first`, uniform per group).
+__device__ __forceinline__ BatchEntry entry_at(const BatchEntry* __restrict__ e, int n, int g) {
     int lo = 0, hi = n - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (e[mid].first <= g) lo = mid;
         else hi = mid - 1;
     }
-    const BatchEntry r = e[lo];
+    return e[lo];
+}
+
+// The same with the (x, y, z-chunk) block coordinates inside the entry's box.
+__device__ __forceinline__ BatchEntry entry_of(const BatchEntry* __restrict__ e, int n, int g, int& bx, int& by,
+                                               int& bz) {
+    const BatchEntry r = entry_at(e, n, g);
     const int nbx = (r.box.ni + kTX - 1) / kTX, nby = (r.box.nj + kTY - 1) / kTY;
     const int l = g - r.first;
     bx = l % nbx;
@@ -533,7 +537,7 @@ template <int C, typename OffT = uint64_t>
 __global__ void __launch_bounds__(kTX * kTY) k_h_bulk_batch(const HArgs* __restrict__ args,
                                                             const BatchEntry* __restrict__ ents, int n_ents) {
     int bx, by, bz;
-    const BatchEntry e = entry_of(ents, n_ents, bx, by, bz);
+    const BatchEntry e = entry_of(ents, n_ents, (int)blockIdx.x, bx, by, bz);
     const HArgs& a = args[e.member];
     h_bulk_body<C, false, OffT>(a.g, e.box, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hx, a.Hy, a.Hz, a.Ex, a.Ey, a.Ez, a.dhx, a.dhy,
                           a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
@@ -565,7 +569,7 @@ template <typename IdxT, int C, typename OffT = uint64_t>
 __global__ void __launch_bounds__(kTX * kTY) k_e_bulk_batch(const EArgs* __restrict__ args,
                                                             const BatchEntry* __restrict__ ents, int n_ents) {
     int bx, by, bz;
-    const BatchEntry e = entry_of(ents, n_ents, bx, by, bz);
+    const BatchEntry e = entry_of(ents, n_ents, (int)blockIdx.x, bx, by, bz);
     const EArgs& a = args[e.member];
     e_bulk_body<IdxT, C, false, OffT>(a.g, e.box, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Ex, a.Ey, a.Ez, a.Hx, a.Hy, a.Hz,
                                 static_cast<const IdxT*>(a.idx), a.tup, a.dex, a.dey, a.dez, a.cp, a.dx, a.dy, a.dz);
@@ -646,21 +650,11 @@ __device__ __forceinline__ float from_lane_above(float v, float last) {
 
 constexpr int kSpRows = 2;   // y rows marched together by one wave
 
-// Work-groups from nsp on update H of the y/z slab boxes (k_h_bulk, ping-pong):
-// they read the step-start state as the core does, so the launch is one where
-// there were two.
+// Tile l of box b; stup holds the coefficient tuples (uint8_t indices).
 template <typename IdxT, int C>
-__global__ void __launch_bounds__(64 * kSY) k_step_sp(SpArgs a, Box b, int nsp, HArgs h, BoxSet slabs) {
+__device__ __forceinline__ void sp_body(const SpArgs& a, const Box& b, int l, float* stup) {
     constexpr int R = kSpRows;
     constexpr bool kPacked = sizeof(IdxT) == 1;
-    __shared__ float stup[kPacked ? kSpTupMax * 6 : 1];
-    if ((int)blockIdx.x >= nsp) {
-        int bx, by, bz;
-        const Box sb = box_of(slabs, (int)blockIdx.x - nsp, bx, by, bz);
-        h_bulk_body<kCx | kCy | kCz, true, uint32_t>(h.g, sb, bx, by, bz, h.Hx, h.Hy, h.Hz, h.Hxo, h.Hyo, h.Hzo, h.Ex,
-                                                     h.Ey, h.Ez, h.dhx, h.dhy, h.dhz, h.DB, h.cp, h.dx, h.dy, h.dz);
-        return;
-    }
     if (kPacked) {   // before any wave leaves: every wave reaches the barrier
         const int tid = (int)(threadIdx.y * blockDim.x + threadIdx.x);
         for (int q = tid; q < a.n_tup * 6; q += (int)(blockDim.x * blockDim.y)) stup[q] = a.tup[q];
@@ -680,7 +674,6 @@ __global__ void __launch_bounds__(64 * kSY) k_step_sp(SpArgs a, Box b, int nsp, 
     // Tiles in launch order, x fastest.  (Dealing contiguous tile ranges to
     // each XCD, so that neighbours share an L2, cut this launch's reads from
     // 2.0x to 1.2x the algorithmic bytes, but took 1% longer here.)
-    const int l = (int)blockIdx.x;
     const int bx = l % nbx, by = (l / nbx) % nby, bz = l / (nbx * nby);
     const int lane = (int)threadIdx.x;
     const int i0 = b.i0 + bx * 64;
@@ -943,6 +936,47 @@ __global__ void __launch_bounds__(64 * kSY) k_step_sp(SpArgs a, Box b, int nsp, 
         on += ZB;
         prow += NY;
     }
+}
+
+// Work-groups from nsp on update H of the y/z slab boxes (k_h_bulk, ping-pong):
+// they read the step-start state as the core does, so the launch is one where
+// there were two.
+template <typename IdxT, int C>
+__global__ void __launch_bounds__(64 * kSY) k_step_sp(SpArgs a, Box b, int nsp, HArgs h, BoxSet slabs) {
+    __shared__ float stup[sizeof(IdxT) == 1 ? kSpTupMax * 6 : 1];
+    if ((int)blockIdx.x >= nsp) {
+        int bx, by, bz;
+        const Box sb = box_of(slabs, (int)blockIdx.x - nsp, bx, by, bz);
+        h_bulk_body<kCx | kCy | kCz, true, uint32_t>(h.g, sb, bx, by, bz, h.Hx, h.Hy, h.Hz, h.Hxo, h.Hyo, h.Hzo, h.Ex,
+                                                     h.Ey, h.Ez, h.dhx, h.dhy, h.dhz, h.DB, h.cp, h.dx, h.dy, h.dz);
+        return;
+    }
+    sp_body<IdxT, C>(a, b, (int)blockIdx.x, stup);
+}
+
+// The single pass of every member of a batch, and H of their slab boxes from
+// work-group nsp on.  In place, the core's fields are read twice and written
+// once in each phase; eight antennas of 80 to 160 cells a side took H 109 +
+// 76 and E 119 + 76 us (core + slabs) and the ports 11; now this launch takes
+// 269 and E of the slabs with the ports 75, the batched step 599 -> 567 us.
+// H of the slabs in a launch of its own: 212 + 68 us, the step 588.
+template <typename IdxT, int C>
+__global__ void __launch_bounds__(64 * kSY) k_step_sp_batch(const SpArgs* __restrict__ args,
+                                                            const BatchEntry* __restrict__ ents, int n_ents, int nsp,
+                                                            const HArgs* __restrict__ hargs,
+                                                            const BatchEntry* __restrict__ slabs, int n_slabs) {
+    __shared__ float stup[sizeof(IdxT) == 1 ? kSpTupMax * 6 : 1];
+    if ((int)blockIdx.x >= nsp) {
+        int bx, by, bz;
+        const BatchEntry e = entry_of(slabs, n_slabs, (int)blockIdx.x - nsp, bx, by, bz);
+        const HArgs& h = hargs[e.member];
+        h_bulk_body<kCx | kCy | kCz, true, uint32_t>(h.g, e.box, bx, by, bz, h.Hx, h.Hy, h.Hz, h.Hxo, h.Hyo, h.Hzo,
+                                                     h.Ex, h.Ey, h.Ez, h.dhx, h.dhy, h.dhz, h.DB, h.cp, h.dx, h.dy,
+                                                     h.dz);
+        return;
+    }
+    const BatchEntry e = entry_at(ents, n_ents, (int)blockIdx.x);
+    sp_body<IdxT, C>(args[e.member], e.box, (int)blockIdx.x - e.first, stup);
 }
 
 // ---------------------------------------------------------------------------
@@ -1524,6 +1558,24 @@ __global__ void __launch_bounds__(kTX * kTY) k_e_slabs(EArgs a, BoxSet bs, PortA
     e_bulk_body<IdxT, kCx | kCy | kCz, true, uint32_t>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo, a.Hx,
                                                        a.Hy, a.Hz, static_cast<const IdxT*>(a.idx), a.tup, a.dex, a.dey,
                                                        a.dez, a.cp, a.dx, a.dy, a.dz);
+}
+
+// The same over the members of a batch: the first `ports` work-groups take one
+// member's ports each.
+template <typename IdxT>
+__global__ void __launch_bounds__(kTX * kTY) k_e_slabs_batch(const EArgs* __restrict__ args,
+                                                             const BatchEntry* __restrict__ ents, int n_ents,
+                                                             const PortArgs* __restrict__ pargs, int ports) {
+    if ((int)blockIdx.x < ports) {
+        ports_body<true, true>(pargs[blockIdx.x], (int)(threadIdx.y * kTX + threadIdx.x), nullptr);
+        return;
+    }
+    int bx, by, bz;
+    const BatchEntry e = entry_of(ents, n_ents, (int)blockIdx.x - ports, bx, by, bz);
+    const EArgs& a = args[e.member];
+    e_bulk_body<IdxT, kCx | kCy | kCz, true, uint32_t>(a.g, e.box, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo,
+                                                       a.Hx, a.Hy, a.Hz, static_cast<const IdxT*>(a.idx), a.tup, a.dex,
+                                                       a.dey, a.dez, a.cp, a.dx, a.dy, a.dz);
 }
 
 // ---------------------------------------------------------------------------

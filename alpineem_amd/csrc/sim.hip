@@ -465,11 +465,13 @@ struct aem_sim {
     // sets, so a step reads one set and writes the other
     bool allow_sp = true;
     bool sp_ok = false;            // the deck admits it (set at creation)
-    bool batched = false;          // a batch steps this simulation: in-place kernels only
+    bool batched = false;          // a batch steps this simulation: its own steps are in place
     Box sp_box{};                  // core box of the single-pass kernel
     int par = 0;                   // which buffer set holds the fields now
     // k_adj_record reads E before its update, which the single pass has
     // already written; a design box records inside k_e_design, after it
+    SpArgs sp_args() const;        // the single pass of the next step
+    EArgs slab_e_args() const;     // and E of its slabs
     bool sp_active() const { return sp_ok && !batched && !(rec_on && !des_on); }
     void flip();
     void bind();
@@ -1019,7 +1021,6 @@ void aem_sim::bind() {
                     F[0], F[1], F[2], F[3], F[4], F[5], v.dx, v.dy, v.dz, d_step};
 }
 
-// After a single-pass step: the other buffer set now holds the fields.
 // The device state one step depends on, as (address, bytes): the six fields
 // and the CPML psi of the current buffer set, the port lines, the Drude
 // currents and E_old, the step counter.  (Thin sheets and SPICE ports, which
@@ -1070,6 +1071,21 @@ void aem_sim::restore(int q) {
     }
 }
 
+SpArgs aem_sim::sp_args() const {
+    const aem_plan_view& v = plan->v;
+    return SpArgs{g, F[0], F[1], F[2], F[3], F[4], F[5], F2[0], F2[1], F2[2], F2[3], F2[4], F2[5], d_idx, d_idx4, d_tup,
+                  n_tup, d_den[0], d_den[1], d_den[2], d_den[3], d_den[4], d_den[5], v.DB, cpH, cpE, v.dx, v.dy, v.dz};
+}
+
+EArgs aem_sim::slab_e_args() const {
+    EArgs es = ea;   // E of the slabs reads the new H
+    es.Hx = F2[3];
+    es.Hy = F2[4];
+    es.Hz = F2[5];
+    return es;
+}
+
+// After a single-pass step: the other buffer set now holds the fields.
 void aem_sim::flip() {
     for (int q = 0; q < 6; ++q) std::swap(F[q], F2[q]);
     for (int f = 0; f < 2; ++f)
@@ -1374,8 +1390,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     // launch when sp --, [1,2] the rest of H)
     if (mark) HIPCHK(hipEventRecord(mark[0], st));
     if (sp) {
-        const SpArgs sa{g, Ex, Ey, Ez, Hx, Hy, Hz, F2[0], F2[1], F2[2], F2[3], F2[4], F2[5], d_idx, d_idx4, d_tup,
-                        n_tup, d_den[0], d_den[1], d_den[2], d_den[3], d_den[4], d_den[5], v.DB, cpH, cpE, v.dx, v.dy, v.dz};
+        const SpArgs sa = sp_args();
         const Box& b = sp_box;
         const unsigned nsp = cdiv(b.ni, 64) * cdiv(b.nj, kSY * kSpRows) * cdiv(b.nk, b.kc);
         // (timed phases launch the slabs by themselves)
@@ -1392,10 +1407,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     }
     if (mark) HIPCHK(hipEventRecord(mark[1], st));
     if (sp) {
-        EArgs es = ea;   // E of the slabs reads the new H
-        es.Hx = F2[3];
-        es.Hy = F2[4];
-        es.Hz = F2[5];
+        const EArgs es = slab_e_args();
         // (single-pass decks always have 32-bit offsets)
         if (mark || !one_launch)
             for (size_t q = 1; q < bulk.size(); ++q)
@@ -2349,15 +2361,23 @@ struct aem_batch {
         unsigned blocks = 0;
     };
     std::vector<Group> hg, eg;
+    // two steps as single passes, from the members' buffer set into the other
+    // and back (arguments by direction); a last step alone runs in place
+    bool sp = false;
+    SpArgs* d_spargs[2] = {nullptr, nullptr};
+    HArgs* d_sphargs[2] = {nullptr, nullptr};
+    EArgs* d_speargs[2] = {nullptr, nullptr};
+    Group sp_core, sp_slabs;
+    int pass = 0;                  // 1 while the fields are in the members' other set
     bool off32 = true;             // every member's arrays under 4 GiB
     HArgs* d_hargs = nullptr;
     EArgs* d_eargs = nullptr;
-    PortArgs* d_pargs = nullptr;
+    PortArgs* d_pargs[2] = {nullptr, nullptr};   // by the buffer set that holds the fields
     int n_port = 0;
     // batched far fields: the face currents of every member binned by the
     // LDS histogram or by contributor lists, then each binning's own launch
-    // (by slot of the differences, see Beside)
-    NtffArgs* d_nargs[2] = {nullptr, nullptr};
+    // (by slot of the differences, see Beside; the currents also by buffer set)
+    NtffArgs* d_nargs[2][2] = {};
     NtffArgs* d_hist_args[2] = {nullptr, nullptr};
     NtffListArgs* d_list_args[2] = {nullptr, nullptr};
     Beside* beside = nullptr;      // set while a graph is captured
@@ -2403,6 +2423,9 @@ struct aem_batch {
         d_hargs = upload(ha);
         d_eargs = upload(ea);
         for (int q = 0; q < n; ++q) off32 = off32 && m[q]->off32;
+        sp = true;
+        for (aem_sim* s : m)
+            sp = sp && s->sp_ok && !(s->rec_on && !s->des_on) && s->plan->v.idx_bytes == 1;
         // bulk groups: one launch per kernel variant (H: by slab tests; E: by
         // slab tests and index width), entries in member order
         auto build = [&](bool e_phase, std::vector<Group>& out) {
@@ -2436,14 +2459,14 @@ struct aem_batch {
         };
         build(false, hg);
         build(true, eg);
-        std::vector<PortArgs> pa;
-        std::vector<NtffArgs> na[2], nh[2];
+        std::vector<PortArgs> pa[2];
+        std::vector<NtffArgs> na[2][2], nh[2];
         std::vector<NtffListArgs> nla[2];
         std::vector<int*> steps(n);
         for (int q = 0; q < n; ++q) {
             aem_sim* s = m[q];
             const aem_plan_view& v = s->plan->v;
-            if (v.n_ports > 0) pa.push_back(s->pa);
+            if (v.n_ports > 0) pa[0].push_back(s->pa);
             if (v.n_angles > 0 && s->ntff_mode != AEM_NTFF_OFF) {
                 const bool hist = s->ntff_mode == AEM_NTFF_HISTOGRAM;
                 const bool list = s->ntff_mode == AEM_NTFF_ORDERED && s->nl.blocks() > 0;
@@ -2453,7 +2476,7 @@ struct aem_batch {
                     xa[k].fstep = s->d_ffstep + k;
                 }
                 if (hist || list) {
-                    for (int k = 0; k < 2; ++k) na[k].push_back(xa[k]);
+                    for (int k = 0; k < 2; ++k) na[0][k].push_back(xa[k]);
                     ntff_mu = std::max(ntff_mu, s->ntff_mu);
                     ntff_mv = std::max(ntff_mv, s->ntff_mv);
                 }
@@ -2469,18 +2492,77 @@ struct aem_batch {
             }
             steps[q] = s->d_step;
         }
-        n_port = (int)pa.size();
-        n_ntff = (int)na[0].size();
+        n_port = (int)pa[0].size();
+        n_ntff = (int)na[0][0].size();
         n_hist = (int)nh[0].size();
         n_list = (int)nla[0].size();
-        d_pargs = upload(pa);
+        if (sp) create_sp(pa[1], na[0], na[1]);
         for (int k = 0; k < 2; ++k) {
-            d_nargs[k] = upload(na[k]);
+            d_pargs[k] = upload(pa[k]);
+            d_nargs[0][k] = upload(na[0][k]);
+            d_nargs[1][k] = upload(na[1][k]);
             d_hist_args[k] = upload(nh[k]);
             d_list_args[k] = upload(nla[k]);
         }
         d_steps = upload(steps);
         HIPCHK(hipStreamSynchronize(st));
+    }
+
+    // The single pass over all members: entries of the core boxes and of the
+    // slab boxes, arguments for either direction, and the port and current
+    // arguments of the members' other buffer set.
+    void create_sp(std::vector<PortArgs>& pa, const std::vector<NtffArgs> (&na0)[2], std::vector<NtffArgs> (&na1)[2]) {
+        const int n = (int)m.size();
+        std::vector<SpArgs> sa[2];
+        std::vector<HArgs> ha[2];
+        std::vector<EArgs> ea[2];
+        std::vector<BatchEntry> core, slabs;
+        long long cb = 0, sb = 0, columns = 0;
+        for (const aem_sim* s : m)
+            columns += (long long)cdiv(s->sp_box.ni, 64) * cdiv(s->sp_box.nj, kSY * kSpRows) * s->sp_box.nk;
+        const int most = columns / kSpPlanesLarge >= kSpLargeGroups ? kSpPlanesLarge : kSpPlanes;
+        for (int q = 0; q < n; ++q) {
+            aem_sim* s = m[q];
+            Box b = s->sp_box;
+            if (!s->planes_set) b.kc = (int)cdiv(b.nk, cdiv(b.nk, most));
+            core.push_back(BatchEntry{(int)cb, q, b});
+            cb += (long long)cdiv(b.ni, 64) * cdiv(b.nj, kSY * kSpRows) * cdiv(b.nk, b.kc);
+            for (const Launch& L : bulk_launches(s->plan->v, s->fuse_cpml, s->planes, false))
+                for (int k = 0; L.c != kCx && k < L.bs.n; ++k) {
+                    const Box& x = L.bs.b[k];
+                    slabs.push_back(BatchEntry{(int)sb, q, x});
+                    sb += (long long)cdiv(x.ni, kTX) * cdiv(x.nj, kTY) * cdiv(x.nk, x.kc);
+                }
+        }
+        if (cb + sb + n > 0x7fffffffLL) throw aem::Error(AEM_ERR_STATE, "batch too large for one bulk launch");
+        for (int k = 0; k < 2; ++k) {
+            for (aem_sim* s : m) {
+                sa[k].push_back(s->sp_args());
+                ha[k].push_back(s->ha);
+                ea[k].push_back(s->slab_e_args());
+                s->flip();
+                if (k == 0 && s->plan->v.n_ports > 0) pa.push_back(s->pa);
+            }
+            d_spargs[k] = upload(sa[k]);
+            d_sphargs[k] = upload(ha[k]);
+            d_speargs[k] = upload(ea[k]);
+        }
+        // the currents of member x read its fields from the other set
+        for (int k = 0; k < 2; ++k)
+            for (NtffArgs x : na0[k])
+                for (const aem_sim* s : m)
+                    if (x.Ex == s->F[0]) {
+                        x.Ex = s->F2[0], x.Ey = s->F2[1], x.Ez = s->F2[2];
+                        x.Hx = s->F2[3], x.Hy = s->F2[4], x.Hz = s->F2[5];
+                        na1[k].push_back(x);
+                        break;
+                    }
+        sp_core.ents = upload(core);
+        sp_core.n_ents = (int)core.size();
+        sp_core.blocks = (unsigned)cb;
+        sp_slabs.ents = upload(slabs);
+        sp_slabs.n_ents = (int)slabs.size();
+        sp_slabs.blocks = (unsigned)sb;
     }
 
     // batched bulk launches; 32-bit byte offsets when every member's arrays
@@ -2510,28 +2592,65 @@ struct aem_batch {
     }
 
     void enqueue(hipStream_t s) {
-        const dim3 bb(32, 8, 1);
-        const int n = (int)m.size();
         auto each = [&](unsigned part) {
             for (aem_sim* x : m) x->enqueue_parts(nullptr, s, part);
         };
         for (const Group& gr : hg)
             launch_h(gr, s);
         each(kPartHPre);
-        if (n_port) k_ports_h_batch<<<n_port, 256, 0, s>>>(d_pargs);
+        if (n_port) k_ports_h_batch<<<n_port, 256, 0, s>>>(d_pargs[0]);
         each(kPartHPost | kPartRecord);
         for (const Group& gr : eg) {
             if (gr.idx_bytes == 1) launch_e<uint8_t>(gr, s);
             else launch_e<uint16_t>(gr, s);
         }
         each(kPartEPre);
-        if (n_port) k_ports_e_batch<<<n_port, 256, 0, s>>>(d_pargs);
+        if (n_port) k_ports_e_batch<<<n_port, 256, 0, s>>>(d_pargs[0]);
         each(kPartEPost | kPartEOld);
+        enqueue_rest(s);
+    }
+
+    // One step as a single pass; two in a row bring the fields back to the
+    // members' own buffer set.
+    void enqueue_sp(hipStream_t s) {
+        const unsigned np = (unsigned)n_port;
+        k_step_sp_batch<uint8_t, kCx><<<sp_core.blocks + sp_slabs.blocks, dim3(64, kSY), 0, s>>>(
+            d_spargs[pass], sp_core.ents, sp_core.n_ents, (int)sp_core.blocks, d_sphargs[pass], sp_slabs.ents,
+            sp_slabs.n_ents);
+        for (aem_sim* x : m) x->flip();
+        if (sp_slabs.blocks + np > 0)
+            k_e_slabs_batch<uint8_t><<<sp_slabs.blocks + np, dim3(kTX, kTY, 1), 0, s>>>(
+                d_speargs[pass], sp_slabs.ents, sp_slabs.n_ents, d_pargs[pass ^ 1], n_port);
+        pass ^= 1;
+        // a design box updates its edges after the bulk, as in a member's own step
+        for (aem_sim* x : m) x->enqueue_parts(nullptr, s, kPartEPre);
+        enqueue_rest(s);
+    }
+
+    // Steps from here to n: singles in pairs, the last one in place.
+    int enqueue_next(hipStream_t s, int64_t left) {
+        if (!sp || left < 2) {
+            enqueue(s);
+            return 1;
+        }
+        enqueue_sp(s);
+        if (beside) beside->next();
+        enqueue_sp(s);
+        return 2;
+    }
+
+    // The step after its field updates.
+    void enqueue_rest(hipStream_t s) {
+        const dim3 bb(32, 8, 1);
+        const int n = (int)m.size();
+        auto each = [&](unsigned part) {
+            for (aem_sim* x : m) x->enqueue_parts(nullptr, s, part);
+        };
         each(kPartOutPre);
         if (n_ntff) {
             const int slot = beside ? beside->slot() : 0;
             if (beside) beside->before_currents(s);
-            k_ntff_currents_batch<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * n_ntff), bb, 0, s>>>(d_nargs[slot]);
+            k_ntff_currents_batch<<<dim3(cdiv(ntff_mu, 32), cdiv(ntff_mv, 8), 6 * n_ntff), bb, 0, s>>>(d_nargs[pass][slot]);
             const hipStream_t sb = beside ? beside->after_currents(s) : s;
             if (n_hist) k_ntff_hist_batch<<<dim3(max_angles, 6, n_hist), kHistThreads, 0, sb>>>(d_hist_args[slot]);
             if (n_list)
@@ -2592,7 +2711,7 @@ aem_status aem_batch_create(aem_sim* const* sims, int32_t n, aem_batch** out) {
     aem_status stt = aem::guard([&]() {
         for (aem_sim* s : b->m) {
             HIPCHK(hipStreamSynchronize(s->st));
-            // the batch steps its members with in-place kernels from here on
+            // the batch steps its members from here on
             s->batched = true;
             s->drop_graphs();
         }
@@ -2630,10 +2749,7 @@ aem_status aem_batch_run(aem_batch* b, int64_t n_steps, int32_t use_graph) {
                 ~Clear() { b->beside = nullptr; }
             } clear{b};
             HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-            for (int q = 0; q < kGraphSteps; ++q) {
-                b->enqueue(b->st);
-                bs.next();
-            }
+            for (int q = 0; q < kGraphSteps; bs.next()) q += b->enqueue_next(b->st, kGraphSteps - q);
             bs.join(b->st);
             HIPCHK(hipStreamEndCapture(b->st, &b->graph));
             HIPCHK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
@@ -2644,8 +2760,7 @@ aem_status aem_batch_run(aem_batch* b, int64_t n_steps, int32_t use_graph) {
                 HIPCHK(hipGraphLaunch(b->gexec, b->st));
                 q += kGraphSteps;
             } else {
-                b->enqueue(b->st);
-                ++q;
+                q += b->enqueue_next(b->st, n_steps - q);
             }
             if (q0 / kWatchSteps != q / kWatchSteps && q < n_steps)
                 for (aem_sim* s : b->m) s->enqueue_watch(b->st);
