@@ -9,7 +9,11 @@
 // Decks with nothing between the bulk H and bulk E updates of a core cell
 // (CPML, ports, materials; no sheets, TF/SF, PBC, Drude) run the bulk H and
 // E of the core box as one single-pass launch (k_step_sp) between two buffer
-// sets, the y/z CPML slabs as ping-pong bulk launches after it.
+// sets, H of the y/z CPML slabs in it or after it, then E of the slabs with the
+// ports beside it (k_e_slabs).  Other fused decks take core and slabs of a phase
+// in one launch up to a size (k_h_bulk_all, k_e_bulk_all); a periodic slab's
+// sheets, TF/SF, media and copies are one launch per phase (k_h_slab_fix,
+// k_e_slab_fix).
 // Every FP32 expression keeps the reference's left-to-right order and the
 // file is compiled with -ffp-contract=off, so the bulk, CPML, sheet, Drude
 // and port arithmetic is bit-identical to the serial reference.

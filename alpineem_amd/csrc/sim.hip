@@ -918,12 +918,12 @@ void aem_sim::create(const aem_sim_options* opt) {
         // registers, and the two x-slab tiles of each row took 5-12% longer at
         // 400^3, in sequence or on a second stream beside them)
         if (v.idx_bytes == 1) {   // word (cell of plane 1, q) = bytes of planes 4q+1 .. 4q+4
-            const size_t pl = (size_t)v.plane, nq = (size_t)(v.NZ + 3) / 4;
-            std::vector<uint32_t> w(pl * nq, 0u);
-            for (size_t k = 0; k < (size_t)v.NZ; ++k)
-                for (size_t c = 0; c < pl; ++c)
-                    w[(k >> 2) * pl + c] |= (uint32_t)v.tuple_idx8[k * pl + c] << (8 * (k & 3));
-            d_idx4 = up<uint32_t>(w.data(), w.size());
+            const long long nw = (long long)v.plane * ((v.NZ + 3) / 4);
+            d_idx4 = dalloc<uint32_t>((size_t)nw, owned);
+            // packed here from the uploaded bytes; by a host loop and a second
+            // upload the creation of a 400^3 antenna took 24 ms, now 5
+            k_pack_idx4<<<cdiv(nw, 256), 256, 0, st>>>(static_cast<const uint8_t*>(d_idx), d_idx4, (long long)v.plane,
+                                                       v.NZ);
         }
         for (int q = 0; q < 6; ++q) F2[q] = zeros<float>(nc + v.plane);
         {
@@ -2342,10 +2342,11 @@ aem_status aem_time_phases(aem_sim* s, int64_t n_steps, float* ms, int32_t n_ms)
 // parameter sweep).  The reference runs such populations as separate solver
 // processes (optimization_scripts/GA.py:11-65, main_ga.py:34-72).  Here one
 // graph-captured step advances every member: the bulk updates of all members
-// run as one launch per kernel variant, the ports, far-field currents and
-// histogram binning and the step counters as one launch each, and any other
-// part a member needs (sheets, TF/SF, Drude, separate CPML, PBC, plane sums,
-// ordered or atomic far-field binning) is enqueued for that member between
+// run as one launch per kernel variant (or, where every member admits the
+// single pass, as passes between the members' two buffer sets), the ports,
+// far-field currents, histogram and list binning and the step counters as one
+// launch each, and any other part a member needs (sheets, TF/SF, Drude, separate
+// CPML, PBC, plane sums, row-scan or atomic far-field binning) is enqueued for that member between
 // them in the reference's order.  Members keep their own device state, so
 // series, fields and finalisation are read per member afterwards.
 // ===========================================================================
