@@ -148,13 +148,8 @@ __device__ __forceinline__ Box box_of(const BoxSet& s, int g, int& bx, int& by, 
 }
 
 // Non-temporal access for the cell's own field values, which are read and
-// written exactly once per launch (the neighbour reads stay cached).
-template <class T>
-__device__ __forceinline__ T ld_once(const T* p) { return __builtin_nontemporal_load(p); }
-template <class T>
-__device__ __forceinline__ void st_once(T v, T* p) { __builtin_nontemporal_store(v, p); }
-
-// The same by byte offset from an array base.
+// written exactly once per launch (the neighbour reads stay cached), by byte
+// offset from an array base.
 template <class T, class OffT>
 __device__ __forceinline__ T ldo(const T* p, OffT ob) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + ob);
@@ -3152,8 +3147,6 @@ __global__ void k_phase_centre(Grid g, int ic, int jc, int kc, int T, const floa
     if (n < T) { P[3][n] = hx; P[4][n] = hy; P[5][n] = hz; }
 }
 
-__global__ void k_step_inc(int* step) { *step = *step + 1; }
-
 // Phase-centre samples (when do_pc) and the step counter in one launch.
 __global__ void k_step_end(Grid g, StepEnd e, const float* Ex, const float* Ey, const float* Ez, const float* Hx,
                            const float* Hy, const float* Hz, int* step) {
@@ -3839,9 +3832,6 @@ __device__ __forceinline__ bool e_upd(const Grid& g, int c, int i, int j, int k)
     if (c == 1) return i >= 2 && k >= 2;
     return i >= 2 && j >= 2;
 }
-__device__ __forceinline__ bool h_in(const Grid& g, int i, int j, int k) {
-    return i >= 1 && j >= 1 && k >= 1 && i <= g.NX - 1 && j <= g.NY - 1 && k <= g.NZ - 1;
-}
 
 // CPML psi cell of the E (slab_e) or H (slab_h) update normal to axis A at
 // (i,j,k): face f, local layer q and psi offset po (as in k_e_cpml_* /
@@ -3888,24 +3878,9 @@ __device__ __forceinline__ bool e_slot_ok(int A, int slot, int i, int j, int k) 
 __device__ __forceinline__ int e_slot_comp(int A, int slot) { return A == 0 ? 1 + slot : (A == 1 ? 2 * slot : slot); }
 __device__ __forceinline__ int h_slot_comp(int A, int slot) { return A == 0 ? 1 + slot : (A == 1 ? 2 * slot : slot); }
 
-// c * nu of an E / H psi cell, 0 where there is none.  The adjoint CPML
-// state holds nu = lambda_psi' + (gb or DB) lambda_field' of the step being
-// transposed; lambda_psi of the step before is b nu, folded into the next
-// update of nu.
-__device__ __forceinline__ float cnu_e(const Grid& g, const Cpml& p, const Cpml& lp, int A, int slot, int i, int j,
-                                       int k) {
-    int f, q;
-    long long po;
-    if (!e_psi(g, p, A, i, j, k, f, q, po) || !e_slot_ok(A, slot, i, j, k)) return 0.0f;
-    return p.c[f][q - 1] * lp.psi[f][slot][po];
-}
-__device__ __forceinline__ float cnu_h(const Grid& g, const Cpml& p, const Cpml& lp, int A, int slot, int i, int j,
-                                       int k) {
-    int f, q;
-    long long po;
-    if (!h_psi(g, p, A, i, j, k, f, q, po)) return 0.0f;
-    return p.c[f][q - 1] * lp.psi[f][slot][po];
-}
+// The adjoint CPML state holds nu = lambda_psi' + (gb or DB) lambda_field' of
+// the step being transposed; lambda_psi of the step before is b nu, folded into
+// the next update of nu.
 
 // c * nu of both slots of the E psi normal to axis A at the cell and at its
 // +1 neighbour along A (cn[slot][0: cell, 1: neighbour]); 0 where absent.

@@ -250,7 +250,8 @@ struct Launch {
 // 120^3 35 / 35 / 30 / 40, 160^3 78 / 63 / 58 / 56, 200^3 167 / 133 / 117 /
 // 108, 256^3 296 / 230 / 201 / 196; with more than kSpLargeGroups columns left
 // at twelve planes that is the better length (400^3 8 / 10 / 12 planes 625 / 617
-// / 607, 320^3 318 / 321 / 320, 200^3 104 / 112 / 121).
+// / 607, 320^3 318 / 321 / 320, 200^3 104 / 112 / 121).  (Slabs measured before
+// their data was found ahead of the march, which took 25-35% off them.)
 constexpr int kPlanes = 4;
 constexpr int kSpPlanes = 8, kSpPlanesLarge = 12;
 constexpr long long kBulkGroups = 4096, kSlabGroups = 2048, kSpGroups = 800, kSpLargeGroups = 8192;
@@ -261,7 +262,8 @@ constexpr long long kBulkGroups = 4096, kSlabGroups = 2048, kSpGroups = 800, kSp
 // since the combined kernel holds the registers of both.  Step, two launches /
 // one: single pass at 40^3 24 / 20 us, 100^3 51 / 49, 160^3 106 / 100, 256^3
 // 306 / 305, 320^3 472 / 477, 400^3 879 / 897; H and E phases at 40^3 25 / 18,
-// 160^3 124 / 118, 256^3 397 / 393, 400^3 1080 / 1092.
+// 160^3 124 / 118, 256^3 397 / 393, 400^3 1080 / 1092 (all before the slab
+// bodies got faster: 400^3 now 793 in two launches).
 constexpr long long kOneLaunchCells = 20000000;
 
 // Parts of a step, in the order the reference applies them.

@@ -15,8 +15,8 @@ from typing import Dict, Sequence, Tuple
 
 from .solver import Batch, Plan, Simulation
 
-# 0 is the library's own choice: about 10 planes per thread in balanced
-# chunks, fewer on small grids and thin boundary boxes.
+# 0 is the library's own choice: 4 planes per thread (8 or 12 in the single
+# pass) in balanced chunks, fewer on small grids and thin boundary boxes.
 CANDIDATES = (0, 2, 4, 6, 8, 10, 16)
 
 
