@@ -152,7 +152,7 @@ enum {
  * choose serial/OpenMP/OpenACC).  Zero-initialise, then set fields. */
 typedef struct aem_sim_options {
     int32_t ntff_binning;   /* AEM_NTFF_* */
-    int32_t planes;         /* z planes marched per thread in the bulk kernels; 0 = default (4) */
+    int32_t planes;         /* z planes marched per thread in the bulk kernels; 0 = by the size of the grid */
     int32_t no_cpml_fusion; /* 1: the separate CPML kernels after ports/TF/SF and one TF/SF launch per face pair */
     int32_t no_single_pass; /* 1: separate H and E bulk launches even where one single-pass launch qualifies */
     int32_t ntff_row_scan;  /* 1: ordered binning by the per-bin scan of staged face rows instead of the
@@ -429,8 +429,9 @@ int64_t aem_core_cells(const aem_sim* sim);
  * timed as phase 0 by aem_time_phases; phase 2 is then empty), 0 if as
  * separate H and E bulk launches, -1 for a null handle.  The single pass
  * needs a deck with the CPML folded into the bulk and no sheets, TF/SF, PBC
- * or Drude media, and is off for batch members and for material-gradient
- * records (aem_adjoint_record without a design box). */
+ * or Drude media, and is off in a batch member's own steps (a batch whose
+ * members all qualify steps by single passes of its own) and for
+ * material-gradient records (aem_adjoint_record without a design box). */
 int32_t aem_single_pass(const aem_sim* sim);
 
 #ifdef __cplusplus
