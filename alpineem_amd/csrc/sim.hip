@@ -29,11 +29,16 @@ using namespace aemk;
 
 namespace {
 
+// The error is read as well as reported: the runtime keeps it until then, and
+// the next check of a launch (hipGetLastError) would report it again, for a
+// call that succeeded.
 #define HIPCHK(x)                                                                                   \
     do {                                                                                            \
         hipError_t e_ = (x);                                                                        \
-        if (e_ != hipSuccess)                                                                       \
+        if (e_ != hipSuccess) {                                                                     \
+            (void)hipGetLastError();                                                                \
             throw aem::Error(AEM_ERR_DEVICE, std::string(#x) + ": " + hipGetErrorString(e_));        \
+        }                                                                                           \
     } while (0)
 
 template <class T>

@@ -1,0 +1,78 @@
+"""Simulations, batches and runs whose HIP calls fail (out of memory, a refused capture)
+leave the others, and themselves, as they were: the same fields in the buffers that the
+next step reads, late setup still allowed, the next batch and run in order.  On
+the CPU, against tests/hip_stub.cpp in place of the HIP runtime; the device
+code does nothing there, so a field changes only if a simulation looks at
+another buffer.  Each case runs in a process of its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+FIELDS = ("Ex", "Ey", "Ez", "Hx", "Hy", "Hz")
+
+PRELUDE = f"""
+import ctypes, sys
+stub = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
+sys.path.insert(0, {ROOT!r})
+import numpy as np
+from alpineem_amd import decks
+from alpineem_amd.solver import Batch, Plan, Simulation
+
+FIELDS = {FIELDS!r}
+fail = lambda name, nth: stub.stub_fail(name.encode(), ctypes.c_long(nth))
+
+def single_pass_sims(sizes, ntff="histogram", angles=2, steps=4000):
+    sims = [Simulation(Plan.from_text(decks.dipole(n=n, steps=steps, angles=angles, arm=6).text()), ntff=ntff)
+            for n in sizes]
+    assert all(s.single_pass for s in sims)
+    return sims
+
+def mark(sims):
+    # every member after an odd number of steps, its fields in its second buffer set
+    for q, s in enumerate(sims):
+        s.run(1, graph=False)
+        for r, f in enumerate(FIELDS):
+            s.set_field(f, np.full(s.plan.shape, 10.0 * q + r + 1.0, np.float32))
+
+def check(sims, what):
+    for q, s in enumerate(sims):
+        for r, f in enumerate(FIELDS):
+            x = s.field(f)
+            assert np.all(x == 10.0 * q + r + 1.0), (what, q, f, x.flat[0])
+
+def fails(call):
+    try:
+        call()
+    except RuntimeError as e:
+        assert "planted failure" in str(e), e
+        return True
+    return False
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stub") / "libhipstub.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-o", out, os.path.join(ROOT, "tests", "hip_stub.cpp")], check=True)
+    return out
+
+
+def run(stub, body):
+    r = subprocess.run([sys.executable, "-c", PRELUDE + body, stub], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+
+
+def test_a_failure_is_reported_once(stub):
+    """A simulation that could not be created does not fail another one's run."""
+    run(stub, """
+a = single_pass_sims((36,))[0]
+for n in (1, 5, 40):
+    fail("hipMalloc", n)
+    assert fails(lambda: single_pass_sims((38,)))
+    a.run(1, graph=False)
+    assert a.steps_done in (1, 2, 3)
+assert a.steps_done == 3
+""")
