@@ -2516,6 +2516,17 @@ struct aem_batch {
         HIPCHK(hipStreamSynchronize(st));
     }
 
+    // The members on their other buffer set while this lives, however it ends.
+    struct OtherSet {
+        const std::vector<aem_sim*>& m;
+        explicit OtherSet(const std::vector<aem_sim*>& sims) : m(sims) { flip(); }
+        ~OtherSet() { flip(); }
+        OtherSet(const OtherSet&) = delete;
+        void flip() const {
+            for (aem_sim* s : m) s->flip();
+        }
+    };
+
     // The single pass over all members: entries of the core boxes and of the
     // slab boxes, arguments for either direction, and the port and current
     // arguments of the members' other buffer set.
@@ -2543,14 +2554,20 @@ struct aem_batch {
                 }
         }
         if (cb + sb + n > 0x7fffffffLL) throw aem::Error(AEM_ERR_STATE, "batch too large for one bulk launch");
-        for (int k = 0; k < 2; ++k) {
-            for (aem_sim* s : m) {
+        auto args = [&](int k) {
+            for (const aem_sim* s : m) {
                 sa[k].push_back(s->sp_args());
                 ha[k].push_back(s->ha);
                 ea[k].push_back(s->slab_e_args());
-                s->flip();
-                if (k == 0 && s->plan->v.n_ports > 0) pa.push_back(s->pa);
+                if (k == 1 && s->plan->v.n_ports > 0) pa.push_back(s->pa);
             }
+        };
+        args(0);
+        {
+            OtherSet other{m};
+            args(1);
+        }
+        for (int k = 0; k < 2; ++k) {
             d_spargs[k] = upload(sa[k]);
             d_sphargs[k] = upload(ha[k]);
             d_speargs[k] = upload(ea[k]);
@@ -2717,13 +2734,12 @@ aem_status aem_batch_create(aem_sim* const* sims, int32_t n, aem_batch** out) {
     }
     b->m.assign(sims, sims + n);
     aem_status stt = aem::guard([&]() {
-        for (aem_sim* s : b->m) {
-            HIPCHK(hipStreamSynchronize(s->st));
-            // the batch steps its members from here on
+        for (aem_sim* s : b->m) HIPCHK(hipStreamSynchronize(s->st));
+        b->create();
+        for (aem_sim* s : b->m) {   // the batch steps its members from here on
             s->batched = true;
             s->drop_graphs();
         }
-        b->create();
     });
     if (stt != AEM_OK) {
         delete b;

@@ -31,11 +31,13 @@ def single_pass_sims(sizes, ntff="histogram", angles=2, steps=4000):
     return sims
 
 def mark(sims):
-    # every member after an odd number of steps, its fields in its second buffer set
+    # every member after an odd number of steps, its fields in its second
+    # buffer set, marked there only: set_field's copy to the other one fails
     for q, s in enumerate(sims):
         s.run(1, graph=False)
         for r, f in enumerate(FIELDS):
-            s.set_field(f, np.full(s.plan.shape, 10.0 * q + r + 1.0, np.float32))
+            fail("hipMemcpyAsync", 2)
+            assert fails(lambda: s.set_field(f, np.full(s.plan.shape, 10.0 * q + r + 1.0, np.float32)))
 
 def check(sims, what):
     for q, s in enumerate(sims):
@@ -75,4 +77,33 @@ for n in (1, 5, 40):
     a.run(1, graph=False)
     assert a.steps_done in (1, 2, 3)
 assert a.steps_done == 3
+""")
+
+
+@pytest.mark.parametrize("name", ["hipMalloc", "hipMemcpyAsync"])
+def test_failed_batch_creation_leaves_members(stub, name):
+    """Each allocation and upload of a batch's creation in turn fails."""
+    run(stub, f"""
+sims = single_pass_sims((36, 38))
+mark(sims)
+allocs = stub.stub_allocs()
+n = 0
+while True:
+    fail({name!r}, n + 1)
+    made = []
+    if not fails(lambda: made.append(Batch(sims))):
+        break
+    n += 1
+    check(sims, ({name!r}, n))
+    assert stub.stub_allocs() == allocs
+    # not a batch's member: its own step is a single pass, into the other buffer set
+    sims[0].run(1)
+    assert not np.any(sims[0].field("Ez") == 3.0), n
+    sims[0].run(1)
+    check(sims, ("after two steps of its own", n))
+assert n > 10, n
+fail("", 0)
+check(sims, "created")
+made[0].run(4)
+check(sims, "run")
 """)
