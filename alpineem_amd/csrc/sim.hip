@@ -88,7 +88,8 @@ struct Beside {
     hipEvent_t cur[2] = {nullptr, nullptr}, bin[2] = {nullptr, nullptr};
     int q = 0;                     // step within the graph
     bool used = false;             // a binning has been enqueued
-    Beside() {
+    Beside() = default;
+    void create() {
         HIPCHK(hipStreamCreateWithFlags(&s2, hipStreamNonBlocking));
         for (int k = 0; k < 2; ++k) {
             HIPCHK(hipEventCreateWithFlags(&cur[k], hipEventDisableTiming));
@@ -120,6 +121,38 @@ struct Beside {
     void next() { ++q; }
     void join(hipStream_t s) {
         if (used) HIPCHK(hipStreamWaitEvent(s, bin[(q - 1) & 1], 0));
+    }
+};
+
+// A graph of the steps that `body` enqueues on stream s.  Where the body or
+// the runtime fails, the capture is ended and what was captured dropped, so the
+// stream takes work again.
+struct Captured {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    Captured() = default;
+    Captured(const Captured&) = delete;
+    ~Captured() { drop(); }
+    void drop() {
+        if (exec) (void)hipGraphExecDestroy(exec);
+        if (graph) (void)hipGraphDestroy(graph);
+        exec = nullptr;
+        graph = nullptr;
+    }
+    template <class F>
+    void capture(hipStream_t s, F&& body) {
+        drop();
+        HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        try {
+            body();
+        } catch (...) {
+            (void)hipStreamEndCapture(s, &graph);
+            (void)hipGetLastError();   // of a capture left unjoined
+            drop();
+            throw;
+        }
+        HIPCHK(hipStreamEndCapture(s, &graph));
+        HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
     }
 };
 
@@ -516,10 +549,8 @@ struct aem_sim {
     template <class IdxT>
     void enqueue_backward_t(hipStream_t s, bool objective, double Fr, double Fi, const double* wV, const double* wI,
                             double* dga, double* dgb);
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec = nullptr;
+    Captured graph;
     int gpar = 0;                  // buffer set the graph starts from and ends on
-    void drop_graphs();
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     RunAhead ra;                   // bounds the steps a replay loop queues
     float last_ms = 0.f;
@@ -551,7 +582,7 @@ struct aem_sim {
         if (h_full) (void)hipHostFree(h_full);
         if (h_spI) (void)hipHostFree(h_spI);
         if (h_spV) (void)hipHostFree(h_spV);
-        drop_graphs();
+        graph.drop();
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         ra.destroy();
@@ -1325,13 +1356,6 @@ void aem_sim::enqueue_kmax_step(hipStream_t s) {
     both(kPartEOld | kPartOutPre | kPartNtff | kPartOutPost | kPartStep);
 }
 
-void aem_sim::drop_graphs() {
-    if (gexec) (void)hipGraphExecDestroy(gexec);
-    if (graph) (void)hipGraphDestroy(graph);
-    gexec = nullptr;
-    graph = nullptr;
-}
-
 // Enqueue the selected parts of one step on stream s, in the reference's
 // order.  A simulation run alone enqueues every part; a batch replaces the
 // bulk, port, far-field and step-counter parts by batched launches and
@@ -1894,30 +1918,33 @@ aem_status aem_run(aem_sim* s, int64_t n_steps, int32_t use_graph) {
     return aem::guard([&]() {
         if (n_steps == 0) return;
         // checkpoints and the full-field export act between steps
-        const bool whole = use_graph && s->ck_K == 0 && !s->full_on && (s->gexec || n_steps >= kGraphMin);
-        if (whole && !s->gexec) {
+        const bool whole = use_graph && s->ck_K == 0 && !s->full_on && (s->graph.exec || n_steps >= kGraphMin);
+        if (whole && !s->graph.exec) {
             s->gpar = s->par;
             Beside bs;
-            HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-            if (s->face_cells() >= kBesideCells) s->beside = &bs;
-            struct Clear {
+            bs.create();
+            struct Clear {   // (a capture that failed has run no step: the fields are where they were)
                 aem_sim* s;
-                ~Clear() { s->beside = nullptr; }
+                ~Clear() {
+                    s->beside = nullptr;
+                    if (s->par != s->gpar) s->flip();
+                }
             } clear{s};
-            for (int q = 0; q < kGraphSteps; ++q) {
-                s->enqueue_step();
-                bs.next();
-            }
-            bs.join(s->st);
-            HIPCHK(hipStreamEndCapture(s->st, &s->graph));
-            HIPCHK(hipGraphInstantiate(&s->gexec, s->graph, nullptr, nullptr, 0));
+            s->graph.capture(s->st, [&]() {
+                if (s->face_cells() >= kBesideCells) s->beside = &bs;
+                for (int q = 0; q < kGraphSteps; ++q) {
+                    s->enqueue_step();
+                    bs.next();
+                }
+                bs.join(s->st);
+            });
         }
         HIPCHK(hipEventRecord(s->ev0, s->st));
         for (int64_t q = 0, q0 = 0; q < n_steps; q0 = q) {
             if (s->ck_K > 0 && (s->steps_done + q) % s->ck_K == 0) s->snapshot((int)((s->steps_done + q) / s->ck_K));
             // (a single step first where the fields are in the other buffer set)
             if (whole && s->par == s->gpar && n_steps - q >= kGraphSteps) {
-                HIPCHK(hipGraphLaunch(s->gexec, s->st));
+                HIPCHK(hipGraphLaunch(s->graph.exec, s->st));
                 q += kGraphSteps;
             } else {
                 s->enqueue_step();
@@ -2392,16 +2419,14 @@ struct aem_batch {
     int n_ntff = 0, n_hist = 0, n_list = 0, max_angles = 0, max_list_blocks = 0, ntff_mu = 0, ntff_mv = 0;
     std::vector<int> ntff_alone;   // members whose far field bins outside the batch
     int** d_steps = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t gexec = nullptr;
+    Captured graph;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     RunAhead ra;
     float last_ms = 0.f;
 
     ~aem_batch() {
         if (st) (void)hipStreamSynchronize(st);
-        if (gexec) (void)hipGraphExecDestroy(gexec);
-        if (graph) (void)hipGraphDestroy(graph);
+        graph.drop();
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         ra.destroy();
@@ -2738,7 +2763,7 @@ aem_status aem_batch_create(aem_sim* const* sims, int32_t n, aem_batch** out) {
         b->create();
         for (aem_sim* s : b->m) {   // the batch steps its members from here on
             s->batched = true;
-            s->drop_graphs();
+            s->graph.drop();
         }
     });
     if (stt != AEM_OK) {
@@ -2762,26 +2787,31 @@ aem_status aem_batch_run(aem_batch* b, int64_t n_steps, int32_t use_graph) {
     return aem::guard([&]() {
         if (n_steps == 0) return;
         for (aem_sim* s : b->m) HIPCHK(hipStreamSynchronize(s->st));
-        const bool whole = use_graph && (b->gexec || n_steps >= kGraphMin);
-        if (whole && !b->gexec) {
+        const bool whole = use_graph && (b->graph.exec || n_steps >= kGraphMin);
+        if (whole && !b->graph.exec) {
             Beside bs;
+            bs.create();
             long long cells = 0;
             for (aem_sim* s : b->m) cells += s->face_cells();
-            if (cells >= kBesideCells) b->beside = &bs;
-            struct Clear {
+            struct Clear {   // (as in aem_run: a failure between the passes of a pair)
                 aem_batch* b;
-                ~Clear() { b->beside = nullptr; }
+                ~Clear() {
+                    b->beside = nullptr;
+                    if (b->pass)
+                        for (aem_sim* s : b->m) s->flip();
+                    b->pass = 0;
+                }
             } clear{b};
-            HIPCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-            for (int q = 0; q < kGraphSteps; bs.next()) q += b->enqueue_next(b->st, kGraphSteps - q);
-            bs.join(b->st);
-            HIPCHK(hipStreamEndCapture(b->st, &b->graph));
-            HIPCHK(hipGraphInstantiate(&b->gexec, b->graph, nullptr, nullptr, 0));
+            b->graph.capture(b->st, [&]() {
+                if (cells >= kBesideCells) b->beside = &bs;
+                for (int q = 0; q < kGraphSteps; bs.next()) q += b->enqueue_next(b->st, kGraphSteps - q);
+                bs.join(b->st);
+            });
         }
         HIPCHK(hipEventRecord(b->ev0, b->st));
         for (int64_t q = 0, q0 = 0; q < n_steps; q0 = q) {
             if (whole && n_steps - q >= kGraphSteps) {
-                HIPCHK(hipGraphLaunch(b->gexec, b->st));
+                HIPCHK(hipGraphLaunch(b->graph.exec, b->st));
                 q += kGraphSteps;
             } else {
                 q += b->enqueue_next(b->st, n_steps - q);
@@ -3033,7 +3063,7 @@ void cell_gradient(const aem::Plan& P, const AdjRec& r, const int lo[3], const i
     }
 }
 
-bool fresh(const aem_sim* s) { return s->steps_done == 0 && !s->gexec; }
+bool fresh(const aem_sim* s) { return s->steps_done == 0 && !s->graph.exec; }
 
 // A batch captured its members' kernel arguments (coefficient table, record
 // and objective state) when it was created; a member cannot gain a design
@@ -3448,21 +3478,18 @@ void backward_sweep(aem_sim* s, std::vector<double>& ha, std::vector<double>& hb
         if (v.idx_bytes == 1) s->enqueue_backward_t<uint8_t>(s->st, ff_src, F[0], F[1], d_wV, d_wI, dga, dgb);
         else s->enqueue_backward_t<uint16_t>(s->st, ff_src, F[0], F[1], d_wV, d_wI, dga, dgb);
     };
-    hipGraph_t gr = nullptr;
-    hipGraphExec_t gx = nullptr;
+    Captured gr;
     const int per = s->ck_K > 0 ? std::min(s->ck_K, T) : T;   // steps transposed without a break
-    if (per >= kGraphMin) {
-        HIPCHK(hipStreamBeginCapture(s->st, hipStreamCaptureModeThreadLocal));
-        for (int q = 0; q < kGraphSteps; ++q) one();
-        HIPCHK(hipStreamEndCapture(s->st, &gr));
-        HIPCHK(hipGraphInstantiate(&gx, gr, nullptr, nullptr, 0));
-    }
+    if (per >= kGraphMin)
+        gr.capture(s->st, [&]() {
+            for (int q = 0; q < kGraphSteps; ++q) one();
+        });
     int64_t launched = 0;
     auto back = [&](int n) {
         while (n > 0) {
             const int64_t l0 = launched;
-            if (gx && n >= kGraphSteps) {
-                HIPCHK(hipGraphLaunch(gx, s->st));
+            if (gr.exec && n >= kGraphSteps) {
+                HIPCHK(hipGraphLaunch(gr.exec, s->st));
                 n -= kGraphSteps;
                 launched += kGraphSteps;
             } else {
@@ -3505,8 +3532,7 @@ void backward_sweep(aem_sim* s, std::vector<double>& ha, std::vector<double>& hb
     float ms = 0.f;
     HIPCHK(hipEventElapsedTime(&ms, s->ev0, s->ev1));
     s->last_ms = ms / (float)T;
-    if (gx) (void)hipGraphExecDestroy(gx);
-    if (gr) (void)hipGraphDestroy(gr);
+    gr.drop();
     ha.resize(3 * ne);
     hb.resize(3 * ne);
     HIPCHK(hipMemcpy(ha.data(), dga, ha.size() * sizeof(double), hipMemcpyDeviceToHost));

@@ -107,3 +107,28 @@ check(sims, "created")
 made[0].run(4)
 check(sims, "run")
 """)
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_failed_capture_leaves_the_fields(stub, batch):
+    """Each call that makes the graph of a run in turn fails, the waits of the
+    second stream among them: nothing has run, and the same run then succeeds."""
+    run(stub, f"""
+sims = single_pass_sims((84, 36) if {batch} else (84,))
+mark(sims)
+target = Batch(sims) if {batch} else sims[0]
+graphs, done = stub.stub_graphs(), sims[0].steps_done
+calls = [("hipStreamCreateWithFlags", 1), ("hipStreamBeginCapture", 1), ("hipStreamWaitEvent", 31),
+         ("hipEventRecord", 32), ("hipStreamEndCapture", 1), ("hipGraphInstantiate", 1)]
+for name, count in calls:
+    for n in range(1, count + 1):
+        fail(name, n)
+        assert fails(lambda: target.run(64)), (name, n)
+        check(sims, (name, n))
+        assert sims[0].steps_done == done
+    assert stub.stub_graphs() - graphs in (0, 1), name   # an attempt's graph goes with the next one
+target.run(64)
+check(sims, "run")
+assert sims[0].steps_done == done + 64
+assert stub.stub_graphs() - graphs == 2
+""")
