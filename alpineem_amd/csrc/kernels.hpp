@@ -2287,6 +2287,13 @@ struct NtffExact {
 // candidate's staged bin.
 constexpr int kExactCells = 4096;   // staged cells per chunk (48 KB of LDS); rows of <= 2048 cells
 
+// Bins by which the FP32 retarded time can differ from its FP64 model, where
+// `size` bounds the distance and the terms it is formed from (r_relay plus the
+// largest |position x step| of each axis) in bins: at most nine roundings of
+// 2^-24 each.  The difference itself may be small where the terms are not, as
+// with a phase centre far outside the grid, so it does not bound them.
+__device__ __forceinline__ double time_margin(double size) { return 4e-3 + 6e-7 * size; }
+
 __global__ void __launch_bounds__(256) k_ntff_exact(NtffFaces f, NtffBins bn, NtffExact ex, const int* step) {
     __shared__ int sii[kExactCells];
     __shared__ float sw[kExactCells], sd[kExactCells];
@@ -2306,6 +2313,9 @@ __global__ void __launch_bounds__(256) k_ntff_exact(NtffFaces f, NtffBins bn, Nt
     const double cdt = (double)bn.c_dt;
     const double tn = (double)n + (isW ? 0.0 : 0.5) - 1.0;
     const double gg[3] = {(double)bn.dx * s1 * c2, (double)bn.dy * s1 * s2, (double)bn.dz * c1};
+    const double size = ((double)bn.r_relay + fabs(gg[0]) * max(abs(f.lo[0] - bn.ic), abs(f.hi[0] - bn.ic)) +
+                         fabs(gg[1]) * max(abs(f.lo[1] - bn.jc), abs(f.hi[1] - bn.jc)) +
+                         fabs(gg[2]) * max(abs(f.lo[2] - bn.kc), abs(f.hi[2] - bn.kc))) / cdt;
     for (int a = 0; a < 3; ++a) {             // face pairs in the reference's order
         if (a == comp || f.pbc[a]) continue;  // faces normal to a feed the other two components
         const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
@@ -2325,7 +2335,7 @@ __global__ void __launch_bounds__(256) k_ntff_exact(NtffFaces f, NtffBins bn, Nt
                               (double)icc * (c == 1 ? gg[1] : gg[2]);
             base[side] = tn + ((double)bn.r_relay - S0) / cdt;
         }
-        const double eps = 4e-3 + 4e-7 * fabs(base[0] + mu * f.lo[b] + mv * f.lo[c]);
+        const double eps = time_margin(size) + 4e-7 * fabs(base[0] + mu * f.lo[b] + mv * f.lo[c]);
         const double lo_t = (double)bin - 1.0 - eps, hi_t = (double)bin + 1.0 + eps;
         const double umin = fmin(mu * f.lo[b], mu * f.hi[b]), umax = fmax(mu * f.lo[b], mu * f.hi[b]);
         // rows (per side) whose t range over u meets [lo_t, hi_t]
@@ -2811,8 +2821,8 @@ __global__ void __launch_bounds__(64 * kListWavesMany) k_ntff_list_batch(const N
 // at a time, and emits those that can reach its bin, counting them first (FILL
 // false), then writing them at the rank a ballot gives them.
 // An FP64 linear model of the retarded time, widened by a margin that covers
-// the FP32 evaluation error (as in k_ntff_exact), gives the candidate cells;
-// the FP32 time of each candidate decides.  A cell whose exact offset x lies
+// the FP32 evaluation error (time_margin), gives the candidate cells; the FP32
+// time of each candidate decides, and k_ntff_expect checks that none is missed.  A cell whose exact offset x lies
 // within eps of a bin edge (eps: the FP32 rounding of n + x, doubled) is
 // listed for every bin it can reach.  On the device because a host loop over
 // the cells, angles and bins took longer than the run's far field itself, and
@@ -2834,6 +2844,14 @@ struct NtffBuild {
     uint2* ent;
 };
 
+// Retarded time of the cell (i, j, k), in the reference's FP32 order.
+__device__ __forceinline__ float build_time(const NtffBuild& P, const float* an, int i, int j, int k) {
+    const float s1 = an[2], c1 = an[3], s2 = an[4], c2 = an[5];
+    return (P.r_relay - ((float)(i - P.c[0]) * P.d[0] * s1 * c2 + (float)(j - P.c[1]) * P.d[1] * s1 * s2 +
+                         (float)(k - P.c[2]) * P.d[2] * c1)) / P.c_dt;
+}
+
+// grid (bin offsets / 4, list rows, face pairs)
 template <bool FILL>
 __global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
     const int q = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
@@ -2872,7 +2890,10 @@ __global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
                           (double)(pos_of(b, 0) - sel(b, P.c)) * sel(b, g) + (double)(pos_of(c, 0) - sel(c, P.c)) * sel(c, g);
         base[side] = ((double)P.r_relay - S0) / cdt + shift;
     }
-    const double marg = P.eps + 4e-3 + 4e-7 * fabs(base[0] + mu * blo + mv * clo);
+    double size = (double)P.r_relay;
+    for (int ax = 0; ax < 3; ++ax)
+        size += fabs(sel(ax, g)) * max(abs(pos_of(ax, sel(ax, P.lo)) - sel(ax, P.c)), abs(pos_of(ax, sel(ax, P.hi)) - sel(ax, P.c)));
+    const double marg = P.eps + time_margin(size / cdt);
     const double lo_t = (double)Q - 1.0 - marg, hi_t = (double)Q + 1.0 + marg;
     const double inv_mu = fabs(mu) < 1e-12 ? 0.0 : 1.0 / mu;
     // rows whose times over u meet [lo_t, hi_t], on either side
@@ -2926,8 +2947,7 @@ __global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
             i = pos_of(0, i);
             j = pos_of(1, j);
             k = pos_of(2, k);
-            const float tfv = (P.r_relay - ((float)(i - P.c[0]) * P.d[0] * s1 * c2 + (float)(j - P.c[1]) * P.d[1] * s1 * s2 +
-                                            (float)(k - P.c[2]) * P.d[2] * c1)) / P.c_dt;
+            const float tfv = build_time(P, an, i, j, k);
             const double x = (double)tfv + shift;
             const bool in = u >= (side ? ulo[1] : ulo[0]) && u <= (side ? uhi[1] : uhi[0]) &&
                             Q >= (int)floor(x - P.eps) && Q <= (int)floor(x + P.eps) + 1;
@@ -2941,6 +2961,35 @@ __global__ void __launch_bounds__(256) k_ntff_build(NtffBuild P) {
         }
     }
     if (!FILL && lane == 0) P.count[6 * at + 3 * m + a] = cnt;
+}
+
+// Entries that the lists of a row must hold per face pair, from the cells: each
+// is listed for every offset it can reach, whatever the window and the
+// candidates of k_ntff_build.  The builder compares its counts with these.
+// grid (any, list rows, face pairs)
+__global__ void __launch_bounds__(256) k_ntff_expect(NtffBuild P, int* expect) {
+    const int row = blockIdx.y;
+    const int m = (int)blockIdx.z / 3, a = (int)blockIdx.z % 3;
+    if (P.pbc[a]) return;
+    auto sel = [](int ax, const auto& v) { return ax == 0 ? v[0] : (ax == 1 ? v[1] : v[2]); };
+    const int b = a == 0 ? 1 : 0, c = a == 2 ? 1 : 2;
+    const int blo = sel(b, P.lo), clo = sel(c, P.lo), alo = sel(a, P.lo), ahi = sel(a, P.hi);
+    const long long nu = sel(b, P.hi) - blo + 1, cells = 2 * nu * (sel(c, P.hi) - clo + 1);
+    const float* an = P.ang + 6 * (row % P.n_angles);
+    const double shift = row >= P.n_angles ? -1.0 : -0.5;
+    int cnt = 0;
+    for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < cells; t += (long long)gridDim.x * blockDim.x) {
+        const int u = blo + (int)((t >> 1) % nu), v = clo + (int)((t >> 1) / nu), pos = t & 1 ? ahi : alo;
+        int i = a == 0 ? pos : u, j = a == 1 ? pos : (a == 0 ? u : v), k = a == 2 ? pos : v;
+        if (m && P.use_m[0]) i = P.off_m[0] - i;
+        if (m && P.use_m[1]) j = P.off_m[1] - j;
+        if (m && P.use_m[2]) k = P.off_m[2] - k;
+        const double x = (double)build_time(P, an, i, j, k) + shift;
+        cnt += (int)floor(x + P.eps) - (int)floor(x - P.eps) + 2;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) cnt += __shfl_xor(cnt, o);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&expect[6 * row + 3 * m + a], cnt);
 }
 
 // NTFF retarded-time binning through an LDS histogram (f90:7643-7927 with

@@ -1740,11 +1740,24 @@ void aem_sim::build_ntff_lists(const std::vector<int>& win, unsigned stride) {
     int* d_dst = dalloc<int>(dst.size(), tmp);
     B.dst = d_dst;
     const dim3 grid(cdiv(win_max, 4), rows, 3 * B.passes);   // four waves per work-group
+    std::vector<int> expect(6 * (size_t)rows, 0);
+    int* d_expect = dalloc<int>(expect.size(), tmp);
     HIPCHK(hipMemsetAsync(B.count, 0, cnt.size() * sizeof(int), st));
+    HIPCHK(hipMemsetAsync(d_expect, 0, expect.size() * sizeof(int), st));
     k_ntff_build<false><<<grid, 256, 0, st>>>(B);
+    k_ntff_expect<<<dim3(8, rows, 3 * B.passes), 256, 0, st>>>(B, d_expect);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(cnt.data(), B.count, cnt.size() * sizeof(int), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipMemcpyAsync(expect.data(), d_expect, expect.size() * sizeof(int), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
+    // every contribution is listed, within the window
+    for (int row = 0; row < rows; ++row)
+        for (int s = 0; s < 6; ++s) {
+            long long have = 0;
+            for (int q = 0; q < win_max; ++q) have += cnt[6 * ((size_t)row * win_max + q) + s];
+            if (have != expect[6 * (size_t)row + s])
+                throw aem::Error(AEM_ERR_STATE, "far-field list outside its bin window");
+        }
     // layout: a group per 64 bins of a row; a list much longer than its
     // group's others (a face in one bin) on its own, since the group's padding
     // and its chain of additions are those of its longest list
