@@ -1697,8 +1697,8 @@ void aem_sim::export_step() {
 // of the exact value, except that the FP32 rounding of t (at most one ulp of
 // the largest t, here doubled) can move it across a bin edge; the cell goes
 // into the list of every offset it can reach with either weight.  Larger than
-// kListBytes in total, the builder gives up and the row-scan kernel stays in
-// use.
+// kListBytes in total without any padding, the builder gives up and the row-scan
+// kernel stays in use.
 void aem_sim::build_ntff_lists(const std::vector<int>& win, unsigned stride) {
     constexpr size_t kListBytes = size_t(4) << 30;
     const aem_plan_view& v = plan->v;
@@ -1760,69 +1760,79 @@ void aem_sim::build_ntff_lists(const std::vector<int>& win, unsigned stride) {
         }
     // layout: a group per 64 bins of a row; a list much longer than its
     // group's others (a face in one bin) on its own, since the group's padding
-    // and its chain of additions are those of its longest list
+    // and its chain of additions are those of its longest list.  Where the
+    // padding would take the lists past kListBytes (many directions a few
+    // degrees off an axis double them), every list on its own, which adds none.
     constexpr int kLong = 1024;
     std::vector<ListDesc> groups, longs;
     size_t n_ent = 0;
-    for (int row = 0; row < rows; ++row) {
-        const int kk = row % v.n_angles;
-        const int wlo = win[2 * kk], wlen = win[2 * kk + 1];
-        for (int w0 = 0; w0 < wlen; w0 += 64) {
-            const int nbin = std::min(64, wlen - w0);
-            const size_t o0 = (size_t)row * win_max + w0;
-            int total[64], sorted[64];
-            for (int l = 0; l < nbin; ++l) {
-                total[l] = 0;
-                for (int s = 0; s < 6; ++s) total[l] += cnt[6 * (o0 + l) + s];
-                sorted[l] = total[l];
-            }
-            std::nth_element(sorted, sorted + nbin / 2, sorted + nbin);
-            const int lim = std::max(kLong, 4 * sorted[nbin / 2]);
-            ListDesc gd{};
-            gd.row = row;
-            gd.bin = wlo + w0;
-            int m[6] = {0, 0, 0, 0, 0, 0};
-            for (int l = 0; l < nbin; ++l) {
-                const int* c = &cnt[6 * (o0 + l)];
-                if (total[l] <= lim) {
-                    for (int s = 0; s < 6; ++s) m[s] = std::max(m[s], c[s]);
-                    continue;
+    auto layout = [&](bool grouped) {
+        groups.clear();
+        longs.clear();
+        n_ent = 0;
+        std::fill(dst.begin(), dst.end(), 0);
+        for (int row = 0; row < rows; ++row) {
+            const int kk = row % v.n_angles;
+            const int wlo = win[2 * kk], wlen = win[2 * kk + 1];
+            for (int w0 = 0; w0 < wlen; w0 += 64) {
+                const int nbin = std::min(64, wlen - w0);
+                const size_t o0 = (size_t)row * win_max + w0;
+                int total[64], sorted[64];
+                for (int l = 0; l < nbin; ++l) {
+                    total[l] = 0;
+                    for (int s = 0; s < 6; ++s) total[l] += cnt[6 * (o0 + l) + s];
+                    sorted[l] = total[l];
                 }
-                gd.skip |= 1ull << l;
-                ListDesc ld{};
-                ld.row = row;
-                ld.bin = wlo + w0 + l;
-                ld.first = (int)n_ent;
-                int* t = &dst[8 * (o0 + l)];
-                t[0] = (int)n_ent;
-                t[1] = 1;
-                for (int s = 0, p = 0; s < 6; ++s) {
-                    t[2 + s] = p;
-                    p += c[s];
-                    ld.seg[s] = p;
-                }
-                longs.push_back(ld);
-                n_ent += (size_t)total[l];
-                if (n_ent * sizeof(uint2) > kListBytes) return;
-            }
-            gd.first = (int)n_ent;
-            for (int s = 0, p = 0; s < 6; ++s) {
-                p += m[s];
-                gd.seg[s] = p;
-            }
-            if (gd.seg[5] == 0) continue;
-            n_ent += (size_t)64 * gd.seg[5];
-            if (n_ent * sizeof(uint2) > kListBytes) return;
-            for (int l = 0; l < nbin; ++l)
-                if (!((gd.skip >> l) & 1ull)) {
+                std::nth_element(sorted, sorted + nbin / 2, sorted + nbin);
+                const int lim = grouped ? std::max(kLong, 4 * sorted[nbin / 2]) : 0;
+                ListDesc gd{};
+                gd.row = row;
+                gd.bin = wlo + w0;
+                int m[6] = {0, 0, 0, 0, 0, 0};
+                for (int l = 0; l < nbin; ++l) {
+                    const int* c = &cnt[6 * (o0 + l)];
+                    if (total[l] <= lim) {
+                        for (int s = 0; s < 6; ++s) m[s] = std::max(m[s], c[s]);
+                        continue;
+                    }
+                    gd.skip |= 1ull << l;
+                    ListDesc ld{};
+                    ld.row = row;
+                    ld.bin = wlo + w0 + l;
+                    ld.first = (int)n_ent;
                     int* t = &dst[8 * (o0 + l)];
-                    t[0] = gd.first + l;
-                    t[1] = 64;
-                    for (int s = 0; s < 6; ++s) t[2 + s] = s ? gd.seg[s - 1] : 0;
+                    t[0] = (int)n_ent;
+                    t[1] = 1;
+                    for (int s = 0, p = 0; s < 6; ++s) {
+                        t[2 + s] = p;
+                        p += c[s];
+                        ld.seg[s] = p;
+                    }
+                    longs.push_back(ld);
+                    n_ent += (size_t)total[l];
+                    if (n_ent * sizeof(uint2) > kListBytes) return false;
                 }
-            groups.push_back(gd);
+                gd.first = (int)n_ent;
+                for (int s = 0, p = 0; s < 6; ++s) {
+                    p += m[s];
+                    gd.seg[s] = p;
+                }
+                if (gd.seg[5] == 0) continue;
+                n_ent += (size_t)64 * gd.seg[5];
+                if (n_ent * sizeof(uint2) > kListBytes) return false;
+                for (int l = 0; l < nbin; ++l)
+                    if (!((gd.skip >> l) & 1ull)) {
+                        int* t = &dst[8 * (o0 + l)];
+                        t[0] = gd.first + l;
+                        t[1] = 64;
+                        for (int s = 0; s < 6; ++s) t[2 + s] = s ? gd.seg[s - 1] : 0;
+                    }
+                groups.push_back(gd);
+            }
         }
-    }
+        return true;
+    };
+    if (!layout(true) && !layout(false)) return;
     if (groups.empty() && longs.empty()) return;
     // the longest chains of additions start first
     auto longer = [](const ListDesc& x, const ListDesc& y) { return x.seg[5] > y.seg[5]; };
