@@ -124,7 +124,6 @@ struct BoxSet {
     Box b[kMaxBoxes];
     int first[kMaxBoxes + 1];   // first work-group of each box; first[n] = total
     int n;
-    int core;                   // 1: box 0 is the core box (x-slab test only), the others slab boxes
 };
 
 // Box of work-group g and its (x, y, z-chunk) block coordinates.  The
@@ -518,18 +517,17 @@ __global__ void __launch_bounds__(kTX * kTY) k_h_bulk(HArgs a, BoxSet bs) {
                        a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
 }
 
-// The core box and the slab boxes in one launch: the same cells and
+// The core box (box 0) and the slab boxes in one launch: the same cells and
 // arithmetic, one launch and one tail less per phase.
-template <typename OffT>
 __global__ void __launch_bounds__(kTX * kTY) k_h_bulk_all(HArgs a, BoxSet bs) {
     int bx, by, bz;
     const Box b = box_of(bs, (int)blockIdx.x, bx, by, bz);
-    if ((int)blockIdx.x < bs.first[1] && bs.core)
-        h_bulk_body<kCx, false, OffT>(a.g, b, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hxo, a.Hyo, a.Hzo, a.Ex, a.Ey, a.Ez,
-                                      a.dhx, a.dhy, a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
+    if ((int)blockIdx.x < bs.first[1])
+        h_bulk_body<kCx, false, uint32_t>(a.g, b, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hxo, a.Hyo, a.Hzo, a.Ex, a.Ey, a.Ez,
+                                          a.dhx, a.dhy, a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
     else
-        h_bulk_body<kCx | kCy | kCz, false, OffT>(a.g, b, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hxo, a.Hyo, a.Hzo, a.Ex,
-                                                  a.Ey, a.Ez, a.dhx, a.dhy, a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
+        h_bulk_body<kCx | kCy | kCz, false, uint32_t>(a.g, b, bx, by, bz, a.Hx, a.Hy, a.Hz, a.Hxo, a.Hyo, a.Hzo, a.Ex,
+                                                      a.Ey, a.Ez, a.dhx, a.dhy, a.dhz, a.DB, a.cp, a.dx, a.dy, a.dz);
 }
 
 template <int C, typename OffT = uint64_t>
@@ -550,18 +548,18 @@ __global__ void __launch_bounds__(kTX * kTY) k_e_bulk(EArgs a, BoxSet bs) {
                              static_cast<const IdxT*>(a.idx), a.tup, a.dex, a.dey, a.dez, a.cp, a.dx, a.dy, a.dz);
 }
 
-template <typename IdxT, typename OffT>
+template <typename IdxT>
 __global__ void __launch_bounds__(kTX * kTY) k_e_bulk_all(EArgs a, BoxSet bs) {
     int bx, by, bz;
     const Box b = box_of(bs, (int)blockIdx.x, bx, by, bz);
     const IdxT* idx = static_cast<const IdxT*>(a.idx);
-    if ((int)blockIdx.x < bs.first[1] && bs.core)
-        e_bulk_body<IdxT, kCx, false, OffT>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo, a.Hx, a.Hy, a.Hz,
-                                            idx, a.tup, a.dex, a.dey, a.dez, a.cp, a.dx, a.dy, a.dz);
+    if ((int)blockIdx.x < bs.first[1])
+        e_bulk_body<IdxT, kCx, false, uint32_t>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo, a.Hx, a.Hy,
+                                                a.Hz, idx, a.tup, a.dex, a.dey, a.dez, a.cp, a.dx, a.dy, a.dz);
     else
-        e_bulk_body<IdxT, kCx | kCy | kCz, false, OffT>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo,
-                                                        a.Hx, a.Hy, a.Hz, idx, a.tup, a.dex, a.dey, a.dez, a.cp, a.dx,
-                                                        a.dy, a.dz);
+        e_bulk_body<IdxT, kCx | kCy | kCz, false, uint32_t>(a.g, b, bx, by, bz, a.Ex, a.Ey, a.Ez, a.Exo, a.Eyo, a.Ezo,
+                                                            a.Hx, a.Hy, a.Hz, idx, a.tup, a.dex, a.dey, a.dez, a.cp,
+                                                            a.dx, a.dy, a.dz);
 }
 
 template <typename IdxT, int C, typename OffT = uint64_t>
@@ -2494,7 +2492,6 @@ struct ListDesc {           // a group of 64 bins or one long list
     int bin;                // first bin offset
     int first;              // first entry
     int seg[6];             // ends of the face pairs x, y, z (then the images' x, y, z) in entries of a list
-    int pad;
     unsigned long long skip;   // group: lanes whose bin is a long list's
 };
 

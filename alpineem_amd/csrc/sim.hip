@@ -925,12 +925,13 @@ void aem_sim::create(const aem_sim_options* opt) {
     rdv[1] = make_rdiv(v.dy, v.kmax != 0);
     rdv[2] = make_rdiv(v.dz, v.kmax != 0);
     bulk = bulk_launches(v, fuse_cpml, planes, !planes_set);
-    if (bulk.size() == 2 && bulk[0].c == kCx && bulk[0].bs.n == 1 && bulk[0].cells() > 0 &&
+    // byte offsets of 32 bits where the arrays stay under 4 GiB
+    off32 = ((unsigned long long)v.ncell + (unsigned long long)v.plane) * 4ull < (1ull << 32);
+    if (off32 && bulk.size() == 2 && bulk[0].c == kCx && bulk[0].bs.n == 1 && bulk[0].cells() > 0 &&
         bulk[0].cells() + bulk[1].cells() <= kOneLaunchCells) {
         std::vector<Box> boxes{bulk[0].bs.b[0]};
         for (int q = 0; q < bulk[1].bs.n; ++q) boxes.push_back(bulk[1].bs.b[q]);
         all_boxes = make_launch(boxes, kCx | kCy | kCz);
-        all_boxes.bs.core = 1;
         one_launch = true;
     }
     for (int f = 0; f < 6; ++f)
@@ -940,11 +941,7 @@ void aem_sim::create(const aem_sim_options* opt) {
         }
     // the single-pass kernel takes the core launch's box (every x, y and z
     // outside the y/z slabs); the slab launch stays as it is
-    // k_step_sp addresses the fields by 32-bit byte offsets, as the bulk
-    // kernels do where they can
-    const bool small = ((unsigned long long)v.ncell + (unsigned long long)v.plane) * 4ull < (1ull << 32);
-    off32 = small;
-    sp_ok = allow_sp && fuse_cpml && small && single_pass_ok(v) && !bulk.empty() && bulk[0].c == kCx &&
+    sp_ok = allow_sp && fuse_cpml && off32 && single_pass_ok(v) && !bulk.empty() && bulk[0].c == kCx &&
             bulk[0].bs.n == 1;
     if (sp_ok) {
         sp_box = bulk[0].bs.b[0];
@@ -1430,8 +1427,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
                                                                                            with ? bulk[1].bs : BoxSet{});
     } else if (parts & kPartHBulk) {
         if (one_launch && !mark) {
-            if (off32) k_h_bulk_all<uint32_t><<<all_boxes.blocks(), bt, 0, s>>>(ha, all_boxes.bs);
-            else k_h_bulk_all<uint64_t><<<all_boxes.blocks(), bt, 0, s>>>(ha, all_boxes.bs);
+            k_h_bulk_all<<<all_boxes.blocks(), bt, 0, s>>>(ha, all_boxes.bs);
         } else {
             h_bulk(bulk[0]);
         }
@@ -1509,8 +1505,7 @@ void aem_sim::enqueue_step_t(hipEvent_t* mark, hipStream_t s, unsigned parts) {
     if (mark) HIPCHK(hipEventRecord(mark[2], st));
     if ((parts & kPartEBulk) && !sp) {
         if (one_launch && !mark) {
-            if (off32) k_e_bulk_all<IdxT, uint32_t><<<all_boxes.blocks(), bt, 0, s>>>(ea, all_boxes.bs);
-            else k_e_bulk_all<IdxT, uint64_t><<<all_boxes.blocks(), bt, 0, s>>>(ea, all_boxes.bs);
+            k_e_bulk_all<IdxT><<<all_boxes.blocks(), bt, 0, s>>>(ea, all_boxes.bs);
         } else {
             e_bulk(bulk[0]);
         }
