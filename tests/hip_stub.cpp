@@ -1,11 +1,12 @@
 // A host stand-in for the HIP runtime calls libaem.so makes: device memory is
-// host memory, kernels do nothing, and a chosen call of a chosen function
-// fails, as when memory runs out.  It lets the CPU tests take libaem's error
-// paths.  Loaded with RTLD_GLOBAL before libaem.so, whose references then bind
-// to these definitions.
+// host memory, kernels do nothing but are counted by name, and a chosen call of
+// a chosen function fails, as when memory runs out.  It lets the CPU tests take
+// libaem's error paths and see which kernels a deck's steps launch.  Loaded with
+// RTLD_GLOBAL before libaem.so, whose references then bind to these definitions.
 #include <cstddef>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <string>
 
 namespace {
@@ -14,6 +15,8 @@ std::string fail_name;
 long fail_left = 0;      // > 0: the fail_left-th call of fail_name from now fails
 int last_error = 0;
 long live_graphs = 0, live_allocs = 0;
+std::map<const void*, std::string> kernels;
+std::map<std::string, long> calls;   // kernel launches by mangled name, runtime calls by name
 
 struct Stream {
     bool capturing = false;
@@ -25,6 +28,7 @@ int error(int e) {
     return e;
 }
 int enter(const char* name) {
+    ++calls[name];
     if (fail_left > 0 && fail_name == name && --fail_left == 0) return error(kOutOfMemory);
     return 0;
 }
@@ -45,6 +49,15 @@ void stub_fail(const char* name, long nth) {
 long stub_pending() { return fail_left; }
 long stub_graphs() { return live_graphs; }
 long stub_allocs() { return live_allocs; }
+// calls of a runtime function, or launches of the kernels whose mangled name
+// holds `name` (with its length before it, as "9k_e_slabs")
+long stub_calls(const char* name) {
+    long n = 0;
+    for (const auto& c : calls)
+        if (c.first == name || (name[0] <= '9' && c.first.find(name) != std::string::npos)) n += c.second;
+    return n;
+}
+void stub_forget() { calls.clear(); }
 
 int hipMalloc(void** p, size_t n) {
     if (int e = enter("hipMalloc")) return e;
@@ -154,14 +167,17 @@ int hipGetSymbolAddress(void** p, const void*) {
     *p = buf;
     return 0;
 }
-int hipLaunchKernel(const void*, ...) { return 0; }
+int hipLaunchKernel(const void* f, ...) {
+    ++calls[kernels[f]];
+    return 0;
+}
 int __hipPushCallConfiguration(...) { return 0; }
 int __hipPopCallConfiguration(...) { return 0; }
 void** __hipRegisterFatBinary(const void*) {
     static void* h = nullptr;
     return &h;
 }
-void __hipRegisterFunction(...) {}
+void __hipRegisterFunction(void**, const void* f, char*, const char* name, ...) { kernels[f] = name; }
 void __hipRegisterVar(...) {}
 void __hipUnregisterFatBinary(void**) {}
 
