@@ -107,3 +107,15 @@ assert calls("k_step_sp_batch") == 0 and calls_of("k_e_bulk_batch") > 0
 body(t.test_gradient)
 assert calls_of("k_adj_e") > 0 and calls_of("k_adj_source_gather") > 0
 """)
+
+
+def test_run_ahead(stub):  # noqa: F811
+    """The host waits once per 32 steps, for the event of 32 steps before."""
+    run(stub, COUNT + """
+sim = single_pass_sims((36,))[0]
+sim.run(64)
+for steps in (640, 64):
+    stub.stub_forget()
+    sim.run(steps)
+    assert calls("hipEventSynchronize") == steps // 32 + 1, steps      # and for the end
+""")
