@@ -3293,6 +3293,11 @@ aem_status aem_adjoint_record(aem_sim* s, const int32_t* lo, const int32_t* hi) 
         aem::set_error("aem_adjoint_record: call before the first step");
         return AEM_ERR_STATE;
     }
+    // the design's kernels write its edges' record and gradient
+    if (s->des_on && !(std::equal(lo, lo + 3, s->rec_lo) && std::equal(hi, hi + 3, s->rec_hi))) {
+        aem::set_error("aem_adjoint_record: the simulation records its design box");
+        return AEM_ERR_STATE;
+    }
     if (const char* why = adjoint_unsupported(v)) {
         aem::set_error(std::string("aem_adjoint_record: the adjoint step does not include ") + why);
         return AEM_ERR_UNSUPPORTED;

@@ -132,3 +132,24 @@ check(sims, "run")
 assert sims[0].steps_done == done + 64
 assert stub.stub_graphs() - graphs == 2
 """)
+
+
+def test_a_design_box_is_the_record_box(stub):
+    """The design's kernels write record and gradient of its own edges, so
+    another record box is refused: its buffers would have another size."""
+    run(stub, """
+dk, lo, hi = decks.adjoint_deck(n=44, steps=8, box=(5, 6, 4))
+plan = Plan.from_text(dk.text())
+sim = Simulation(plan, ntff="off")
+sim.record_design(lo, [h - 1 for h in hi])       # another box before there is a design: as before
+sim = Simulation(plan, ntff="off")
+sim.design_box(lo, hi)
+for a, b in ((lo, [h - 1 for h in hi]), ([l - 1 for l in lo], hi)):
+    try:
+        sim.record_design(a, b)
+        assert False, (a, b)
+    except RuntimeError as e:
+        assert "design box" in str(e), e
+sim.record_design(lo, hi)
+sim.run()
+""")
