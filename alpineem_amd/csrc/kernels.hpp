@@ -3000,12 +3000,17 @@ __global__ void __launch_bounds__(256) k_ntff_expect(NtffBuild P, int* expect) {
 // k_ntff_bins; only the FP64 summation order differs from the serial reference
 // (agreement at FP32 rounding level).
 //
-// Bound by the retarded time's arithmetic and the LDS additions.  So both
+// Where a direction spreads the cells over many bins, a work-group's LDS unit and
+// vector units are both busy two thirds of its time.  So both
 // currents share one bin and weight, the three products of the time come from
 // tables per row and column, indices are 32-bit, and 16 waves with four cells
 // per thread in flight cover the loads.  150^3 with 73 angles: 134 us; one
 // histogram per accumulator with 4 waves had taken 263, 16 waves alone 213,
 // all but the lane orientation and the DPP sums 201.
+// What bounds the launch is its slowest directions: one alone takes 33 us
+// oblique, 50 along an axis, 71 at 5 and 113 at 2.5 degrees off one, where runs
+// of fewer than 16 lanes share a bin and their LDS additions take turns.  Over
+// the launch a compute unit is busy 29% of the time.
 constexpr int kHistMax = 4096;   // bins of one window held in LDS (64 KB for two)
 constexpr int kHistThreads = 1024;
 constexpr int kHistCells = 4;    // cells per thread in flight

@@ -3,8 +3,7 @@
 // aem_sim_create uploads a plan (the reference's "!$acc data" region,
 // fdtd_solver.f90:4380-4430); aem_run enqueues the leapfrog step
 // (fdtd_solver.f90:4440-8299) on the sim's stream, optionally replaying a
-// captured hipGraph per step (one per buffer set when the single-pass step
-// alternates two sets of fields); aem_finalize runs the post-loop products
+// captured hipGraph of sixteen steps; aem_finalize runs the post-loop products
 // (fdtd_solver.f90:8340-8534) on the device.
 #include <hip/hip_runtime.h>
 
@@ -80,10 +79,14 @@ constexpr int kRunAheadChunk = 2 * kGraphSteps;
 // q wait for the binning of step q - 2, and the graph ends with the last
 // binning.  The two waits between the streams cost about 11 us per step, so a
 // far-field box of less than kBesideCells face cells keeps one stream.
-// Measured per step, beside / in turn: 40^3 with 3 angles (2,000 face cells)
-// 64 / 57 us, 64^3 (10,600) 70 / 68, 76^3 (17,500) 80 / 82, 100^3 91 / 100;
-// LDS histogram at 64^3 70 / 74, 76^3 82 / 100, 100^3 107 / 151; 200^3 with 3
-// angles 295 / 387.
+// Measured per step, beside / in turn, dipoles with 3 angles: ordered lists at
+// 40^3 (1,700 face cells) 32 / 32 us, 56^3 (6,500) 34 / 34, 64^3 (10,100) 37 /
+// 38, 72^3 (14,400) 44 / 47, 76^3 (16,900) 47 / 51, 100^3 (35,600) 58 / 75; LDS
+// histogram at 64^3 36 / 30, 72^3 43 / 40, 76^3 45 / 43, 84^3 (22,300) 47 / 47,
+// 100^3 57 / 62; TF/SF spheres, lists, at 64^3 46 / 42, 72^3 54 / 56, 76^3 57 / 59.
+// So the line lies between the lists' crossing (about 10,000) and the
+// histogram's (22,000).  Batches gain at every size measured (two members with
+// 4,400 cells 57 / 66, four with 13,200 74 / 95).
 constexpr long long kBesideCells = 16000;
 struct Beside {
     hipStream_t s2 = nullptr;
@@ -283,27 +286,29 @@ struct Launch {
 // waits for its own loads, so where the launch has fewer work-groups than
 // kBulkGroups (kSlabGroups, kSpGroups) the march is cut: more and shorter
 // columns, although each reads its first plane's neighbour again.  Measured
-// (us per launch, planes 1 / 2 / 4 / 8): bulk H core at 40^3 7.1 / 8.6 / 11.3 /
-// 14.0, 80^3 9.9 / 10.7 / 13.4, 150^3 31.5 / 30.3 / 33.5, 200^3 80 / 74 / 74,
-// 256^3 142 / 133 / 130; y/z slabs (H and E) at 120^3 37 / 36 / 43, 150^3 49 /
-// 48 / 51, 200^3 84 / 81 / 84; single pass at 40^3 11.5 / 13.6 / 18.9 / 29.2,
-// 120^3 35 / 35 / 30 / 40, 160^3 78 / 63 / 58 / 56, 200^3 167 / 133 / 117 /
-// 108, 256^3 296 / 230 / 201 / 196; with more than kSpLargeGroups columns left
-// at twelve planes that is the better length (400^3 8 / 10 / 12 planes 625 / 617
-// / 607, 320^3 318 / 321 / 320, 200^3 104 / 112 / 121).  (Slabs measured before
-// their data was found ahead of the march, which took 25-35% off them.)
+// (us per launch by events, planes 1 / 2 / 4 / 8): bulk H core at 40^3 7.0 /
+// 7.6 / 8.7 / 9.8, 80^3 9.5 / 9.9 / 10.1 / 12.5, 150^3 25 / 24 / 25 / 27, 200^3
+// 58 / 58 / 59 / 60, 256^3 98 / 98 / 101 / 102, 400^3 381 / 393 / 388 / 401 (E
+// 425 / 431 / 406 / 416); y/z slabs of H at 120^3 16 / 16 / 18 / 20, 200^3 30 / 30 /
+// 30 / 30, 256^3 37 / 37 / 37 / 38, 400^3 78 / 76 / 74 / 74; single pass at 40^3
+// 11 / 13 / 17 / 26, 120^3 35 / 34 / 30 / 36, 160^3 73 / 62 / 58 / 56, 200^3 160 /
+// 126 / 112 / 106, 256^3 278 / 216 / 191 / 189, 400^3 1002 / 811 / 696 / 666.  With
+// more than kSpLargeGroups columns left at twelve planes the single pass takes
+// those: within 1% of eight at 400^3 (667), worse below (320^3 345 / 336, 200^3
+// 115 / 106).
 constexpr int kPlanes = 4;
 constexpr int kSpPlanes = 8, kSpPlanesLarge = 12;
 constexpr long long kBulkGroups = 4096, kSlabGroups = 2048, kSpGroups = 800, kSpLargeGroups = 8192;
 
 // Grids up to kOneLaunchCells update the core box and the slab boxes of a
 // phase in one launch (the single pass with the slabs' H), which saves a launch
-// and lets the slabs fill the core's last work-groups; larger ones keep two,
-// since the combined kernel holds the registers of both.  Step, two launches /
-// one: single pass at 40^3 24 / 20 us, 100^3 51 / 49, 160^3 106 / 100, 256^3
-// 306 / 305, 320^3 472 / 477, 400^3 879 / 897; H and E phases at 40^3 25 / 18,
-// 160^3 124 / 118, 256^3 397 / 393, 400^3 1080 / 1092 (all before the slab
-// bodies got faster: 400^3 now 793 in two launches).
+// and lets the slabs fill the core's last work-groups.  Step, two launches /
+// one: single pass at 40^3 15.6 / 11.6 us, 100^3 41.7 / 35.4, 160^3 85 / 75, 256^3
+// 251 / 239, 320^3 419 / 402, 400^3 796 / 782; H and E phases at 40^3 20.6 / 15.2,
+// 100^3 46.7 / 39.0, 160^3 91 / 86, 256^3 274 / 264, 320^3 496 / 486, 400^3 939 /
+// 945.  The line was drawn when the slab bodies took more registers and larger
+// grids lost 1-2% in one launch; with today's it could lie higher for the single
+// pass.
 constexpr long long kOneLaunchCells = 20000000;
 
 // Parts of a step, in the order the reference applies them.

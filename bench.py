@@ -6,8 +6,9 @@ z-directed 50 ohm lumped port at the centre driven by a Gaussian of spread
 40 dt and t_spread 160 dt.  A "step" is one full leapfrog step (H phase,
 E phase, CPML, port, per-step outputs).  Inputs are resident in HBM before
 the timed region; W warm-up steps are run first, then exactly K steps are
-timed (wall clock around a device-synchronised replay of K captured step
-graphs).  value = 400^3 x K / seconds, in Gcell-updates/s.
+timed (wall clock around a device-synchronised run of K steps, in captured
+graphs of sixteen where K is at least 48).  value = 400^3 x K / seconds, in
+Gcell-updates/s.
 
 The JSON line also carries
   roofline      the dominant kernel's algorithmic HBM bytes per launch over its
