@@ -119,3 +119,12 @@ for steps in (640, 64):
     sim.run(steps)
     assert calls("hipEventSynchronize") == steps // 32 + 1, steps      # and for the end
 """)
+
+
+def test_slab_incidence(stub):  # noqa: F811
+    run(stub, COUNT + """
+from tests import test_gpu_slab_incidence as t
+for ax, inc in ((0, (90.0, 180.0)), (1, (90.0, 270.0)), (2, (180.0, 0.0))):
+    body(t.test_incidence_equals_separate_launches, ax, inc, 90.0)
+    assert calls("k_h_slab_fix") > 0 and calls("k_plane_sums") == 110 + calls("k_h_slab_fix"), ax
+""")
