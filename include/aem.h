@@ -295,7 +295,7 @@ aem_status aem_ffdft_get(aem_sim* sim, double* out, int64_t n);
 /* Record the design box of cells [lo, hi] (1-based, inclusive, in the
  * interior outside the CPML slabs) during the run: every step stores E and
  * the update's curl term on the box's edges (time_steps * 6 * edges floats).
- * Call before the first step. */
+ * Call before the first step; after aem_design_box only with its box. */
 aem_status aem_adjoint_record(aem_sim* sim, const int32_t* lo, const int32_t* hi);
 
 /* After the full run: gradient of J = |F|^2 with respect to the relative
