@@ -67,10 +67,8 @@ constexpr int kGraphMin = 48;
 // after every kRunAheadChunk steps the host records an event and waits
 // for the one it recorded a chunk earlier.  The device always has a chunk
 // of work queued, while the runtime is never handed a whole run at once (a
-// 3000-step, 64-member population is about 10^6 kernel dispatches).  Two graphs
-// a chunk; four give the same times (40^3 dipole, 75 x 30 x 30 periodic slab,
-// eight antennas: within 0.2%).
-constexpr int kRunAheadChunk = 2 * kGraphSteps;
+// 3000-step, 64-member population is about 10^6 kernel dispatches).
+constexpr int kRunAheadChunk = 64;
 
 // Beside the next step: the far-field binning of a step reads that step's
 // current differences only, so inside a captured graph it runs on a second

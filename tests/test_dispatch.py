@@ -109,18 +109,6 @@ assert calls_of("k_adj_e") > 0 and calls_of("k_adj_source_gather") > 0
 """)
 
 
-def test_run_ahead(stub):  # noqa: F811
-    """The host waits once per 32 steps, for the event of 32 steps before."""
-    run(stub, COUNT + """
-sim = single_pass_sims((36,))[0]
-sim.run(64)
-for steps in (640, 64):
-    stub.stub_forget()
-    sim.run(steps)
-    assert calls("hipEventSynchronize") == steps // 32 + 1, steps      # and for the end
-""")
-
-
 def test_slab_incidence(stub):  # noqa: F811
     run(stub, COUNT + """
 from tests import test_gpu_slab_incidence as t
