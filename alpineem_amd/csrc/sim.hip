@@ -67,8 +67,10 @@ constexpr int kGraphMin = 48;
 // after every kRunAheadChunk steps the host records an event and waits
 // for the one it recorded a chunk earlier.  The device always has a chunk
 // of work queued, while the runtime is never handed a whole run at once (a
-// 3000-step, 64-member population is about 10^6 kernel dispatches).
-constexpr int kRunAheadChunk = 64;
+// 3000-step, 64-member population is about 10^6 kernel dispatches).  A chunk is
+// four graphs, so a run in graphs has at most eight launches queued; chunks of
+// two cost 0.2% where a step takes 15-35 us (40^3 dipole, 120 x 30 x 30 Drude slab).
+constexpr int kRunAheadChunk = 4 * kGraphSteps;
 
 // Beside the next step: the far-field binning of a step reads that step's
 // current differences only, so inside a captured graph it runs on a second

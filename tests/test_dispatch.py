@@ -116,3 +116,15 @@ for ax, inc in ((0, (90.0, 180.0)), (1, (90.0, 270.0)), (2, (180.0, 0.0))):
     body(t.test_incidence_equals_separate_launches, ax, inc, 90.0)
     assert calls("k_h_slab_fix") > 0 and calls("k_plane_sums") == 110 + calls("k_h_slab_fix"), ax
 """)
+
+
+def test_run_ahead(stub):  # noqa: F811
+    """The host waits once per 64 steps, for the event of 64 steps before."""
+    run(stub, COUNT + """
+sim = single_pass_sims((36,))[0]
+sim.run(128)
+for steps in (640, 64):
+    stub.stub_forget()
+    sim.run(steps)
+    assert calls("hipEventSynchronize") == steps // 64 + 1, steps      # and for the end
+""")
